@@ -11,14 +11,15 @@
 // the TTGT route (cudense.jl:170-236): tiles are gathered straight from the
 // tensors into LDS, in whichever direction (m/n or k) is contiguous in HBM.
 //
-// Tile: 128x128 per 256-thread workgroup, 2x2 waves of 64x64, each wave a
-// 4x4 grid of 16x16 MFMA blocks (FP64 launches with fewer tiles than
-// workgroup slots: 64x64, 2x2 waves of 32x32).
-//   FP64   : v_mfma_f64_16x16x4_f64, FP64 accumulate          (BK = 16)
-//   FP32   : v_mfma_f32_16x16x4_f32, FP32 accumulate          (BK = 16)
-//   BF16x3 : a = ah + al, b = bh + bl (bf16, round-to-nearest-even);
-//            ah*bh + ah*bl + al*bh on v_mfma_f32_16x16x32_bf16,
-//            FP32 accumulate (Henry, Tang & Heinecke, ARITH 2019) (BK = 32)
+// 256-thread workgroups, 2x2 waves:
+//   native : gett_native_kernel, 32 x 32 to 128 x 128 tiles,
+//            v_mfma_f64_16x16x4_f64 (FP64 storage, FP64 accumulate) or
+//            v_mfma_f32_16x16x4_f32 (FP32 storage, FP32 accumulate)
+//   FP32 on FP64 storage, BF16x3 : gett_kernel, 128 x 128 tiles,
+//            v_mfma_f32_16x16x4_f32; BF16x3 splits a = ah + al, b = bh + bl
+//            (bf16, round-to-nearest-even) and sums ah*bh + ah*bl + al*bh on
+//            v_mfma_f32_16x16x32_bf16, FP32 accumulate (Henry, Tang &
+//            Heinecke, ARITH 2019)
 // Workgroup ids are remapped so that each XCD (ids congruent mod 8) works on
 // a contiguous group of tiles sharing A/B panels in its own L2.
 #include <hip/hip_runtime.h>
@@ -47,12 +48,10 @@ __device__ __forceinline__ uint16_t f2bf_rne(float x) {
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
-template <typename T, int MODE, int TS = 128>
+template <int MODE>
 struct GettTraits {
   static constexpr bool BF = (MODE == ITG_MODE_BF16X3);
-  static constexpr bool F64 = (MODE == ITG_MODE_NATIVE) && std::is_same<T, double>::value;
-  using CT = typename std::conditional<F64, double, float>::type;
-  static constexpr int BM = TS, BN = TS;   // 128, or 64 for FP64 launches with few tiles
+  static constexpr int BM = 128, BN = 128;
   static constexpr int BKT = BF ? 32 : 16;
   static constexpr int NPT = BM * BKT / 256;   // elements per thread per operand
 };
@@ -73,10 +72,106 @@ __device__ __forceinline__ void tile_coords(int64_t tilesM, int64_t tilesN, int6
   tn = in / gsize;
 }
 
-template <typename T, int MODE, bool AK, bool BKF, int TS = 128>
+// Epilogue of gett_kernel's 128 x 128 tile (2 x 2 waves of 4 x 4 blocks):
+// lane holds D[4*lg + r][lr] of each 16x16 block
+template <typename T>
+__device__ __forceinline__ void gett_epilogue(const GettArgs& g, f4_t (&acc)[4][4], int64_t m0,
+                                              int64_t n0, int wm, int wn, int lr, int lg) {
+  constexpr int BM = 128, BN = 128, WH = 64, WT = 4;
+  using CT = float;
+  if (g.partial) {
+    CT* P = (CT*)g.partial + (int64_t)blockIdx.z * g.M * g.N;
+#pragma unroll
+    for (int i = 0; i < WT; ++i)
+#pragma unroll
+      for (int j = 0; j < WT; ++j) {
+        int64_t n = n0 + wn * WH + j * 16 + lr;
+        if (n >= g.N) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          int64_t m = m0 + wm * WH + i * 16 + 4 * lg + r;
+          if (m < g.M) P[m * g.N + n] = acc[i][j][r];
+        }
+      }
+    return;
+  }
+  T* C = (T*)g.C;
+  if (g.sCm == 1 && g.sCn >= 0 && m0 + BM <= g.M && n0 + BN <= g.N) {
+    // interior tile of a column-major C: one column pointer per j and
+    // compile-time row offsets, no per-element bounds or offset arithmetic
+    // (a short epilogue: this code runs once per tile, from a cold
+    // instruction cache on small launches)
+    T* cb = C + (n0 + wn * WH + lr) * g.sCn + m0 + wm * WH + 4 * lg;
+    const double al = g.alpha, be = g.beta;
+    if (be != 0.0) {
+#pragma unroll
+      for (int j = 0; j < WT; ++j) {
+        T* cj = cb + (int64_t)(j * 16) * g.sCn;
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int mo = i * 16 + r;
+            cj[mo] = (T)(al * (double)acc[i][j][r] + be * (double)cj[mo]);
+          }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < WT; ++j) {
+        T* cj = cb + (int64_t)(j * 16) * g.sCn;
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) cj[i * 16 + r] =
+              (T)(al * (double)acc[i][j][r]);
+      }
+    }
+    return;
+  }
+  if (g.sCn == 1 && g.sCm >= 0 && m0 + BM <= g.M && n0 + BN <= g.N) {
+    // the same for a row-major C (itg_gemm's C^T): one row pointer per
+    // (i, r), compile-time column offsets
+    T* cb = C + (m0 + wm * WH + 4 * lg) * g.sCm + n0 + wn * WH + lr;
+    const double al = g.alpha, be = g.beta;
+#pragma unroll
+    for (int i = 0; i < WT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        T* ci = cb + (int64_t)(i * 16 + r) * g.sCm;
+        if (be != 0.0) {
+#pragma unroll
+          for (int j = 0; j < WT; ++j)
+            ci[j * 16] = (T)(al * (double)acc[i][j][r] + be * (double)ci[j * 16]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < WT; ++j) ci[j * 16] = (T)(al * (double)acc[i][j][r]);
+        }
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < WT; ++i)
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      int64_t n = n0 + wn * WH + j * 16 + lr;
+      if (n >= g.N) continue;
+      int64_t on = goff(g.tCn, g.sCn, n);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        int64_t m = m0 + wm * WH + i * 16 + 4 * lg + r;
+        if (m >= g.M) continue;
+        int64_t o = on + goff(g.tCm, g.sCm, m);
+        double v = g.alpha * (double)acc[i][j][r];
+        if (g.beta != 0.0) v += g.beta * (double)C[o];
+        C[o] = (T)v;
+      }
+    }
+}
+
+template <typename T, int MODE, bool AK, bool BKF>
 __global__ __launch_bounds__(256, 2) void gett_kernel(GettArgs g) {
-  using TR = GettTraits<T, MODE, TS>;
-  using CT = typename TR::CT;
+  using TR = GettTraits<MODE>;
+  using CT = float;
   constexpr int BM = TR::BM, BN = TR::BN, BKT = TR::BKT, NPT = TR::NPT;
   // four waves in 2 x 2, each a WH x WH sub-tile of WT x WT 16 x 16 blocks
   constexpr int WH = BM / 2, WT = BM / 32;
@@ -199,12 +294,11 @@ __global__ __launch_bounds__(256, 2) void gett_kernel(GettArgs g) {
     }
   };
 
-  typedef typename std::conditional<TR::F64, d4_t, f4_t>::type acc_t;
-  acc_t acc[WT][WT];
+  f4_t acc[WT][WT];
 #pragma unroll
   for (int i = 0; i < WT; ++i)
 #pragma unroll
-    for (int j = 0; j < WT; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int j = 0; j < WT; ++j) acc[i][j] = f4_t{0, 0, 0, 0};
 
   const int lr = lane & 15, lg = lane >> 4;
   if (kbeg < kend) load(kbeg);
@@ -247,105 +341,284 @@ __global__ __launch_bounds__(256, 2) void gett_kernel(GettArgs g) {
         for (int i = 0; i < WT; ++i)
 #pragma unroll
           for (int j = 0; j < WT; ++j) {
-            if constexpr (TR::F64)
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-            else if constexpr (!BF)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
           }
       }
     }
   }
 
-  // epilogue: lane holds D[row][lr] of each 16x16 block, with row = 4*lg + r
-  // for the FP32-accumulating MFMAs (4-row groups) and row = 4*r + lg for
-  // v_mfma_f64_16x16x4_f64 (1-row groups)
-  if (g.partial) {
-    CT* P = (CT*)g.partial + (int64_t)blockIdx.z * g.M * g.N;
+  gett_epilogue<T>(g, acc, m0, n0, wm, wn, lr, lg);
+}
+
+// ---------------------------------------------------------- native kernel
+// FP64 storage with FP64 MFMA and FP32 storage with FP32 MFMA. TS x TS
+// tile per 256-thread workgroup (2 x 2 waves of TS/2 x TS/2, 16x16x4
+// blocks), K staged 16 deep through two LDS buffers with one barrier per
+// stage.
+//
+// Bound: the matrix pipe, if the loader and the fragment reads stay out of
+// its way. A wave issues (TS/32)^2 products per 4 k, 64 (FP64) or 32 (FP32)
+// cycles each.
+//  - Of an element's offset only the part that changes is recomputed: an
+//    operand read along its free index (KF false) takes k from the wave's
+//    number, so k's offset (stride or table) is wave-uniform and lives in
+//    scalar registers, and the per-lane pointer is fixed for the whole
+//    launch; an operand read along k keeps one pointer per row and adds the
+//    lane's k offset, which (if it comes from a table) is fetched one stage
+//    before the loads that use it. Rows past M or N read the last row
+//    instead of being masked (their results are never stored); only the
+//    last, partial stage masks k.
+//  - Block (i, j) of a wave holds rows WT q + i and columns WT q + j,
+//    q < 16, of its sub-tile, so a lane's WT fragments are consecutive in
+//    LDS (one 16-byte read for four FP32 or two FP64) and its WT outputs of
+//    a row are one vector store.
+//
+// LDS: [k][m] rows of TS elements, element (k, m) at m ^ sw(k), sw a
+// multiple of 4 so that the vectors stay whole; a store of 16 k x 4 m (or
+// 8 x 8) by a wave that loads along k then covers every bank evenly.
+template <typename T>
+__device__ __forceinline__ int native_sw(int k) {
+  return std::is_same<T, double>::value ? ((k & 1) << 4) | (((k >> 1) & 3) << 2)
+                                        : ((k & 3) << 4) | (((k >> 2) & 3) << 2);
+}
+
+// one operand's loader: X(row, k), rows [r0, r0 + TS), TS * BK / 256
+// elements per thread and stage
+template <typename T, int TS, int BK, bool KF, bool TAB>
+struct NativeLoader {
+  static constexpr int NPT = TS * BK / 256;
+  static constexpr bool UNI = !KF && TS >= 64;   // k uniform over a wave
+  static constexpr int STEP = KF ? 256 / BK : 256 / TS;
+  static constexpr int MASK = TS < 64 ? TS - 1 : 63;   // swizzle within the row
+  static constexpr int NKO = KF ? 1 : NPT;   // k values of a thread in a stage
+  const T* p[KF ? NPT : 1];
+  const int64_t* tk;         // k offsets from the chunk's first k: table or null
+  int64_t sk;                // their stride, if not
+  int64_t kn[TAB ? NKO : 1]; // offsets of the next stage's k (!TAB: of its first)
+  int kf;                    // KF: k of this thread in a stage; else its first k
+  int klen;
+  T r[NPT];
+
+  __device__ __forceinline__ void init(const T* X, int64_t r0, int64_t rows, const int64_t* tr,
+                                       int64_t sr, const int64_t* tkk, int64_t skk, int64_t kbeg,
+                                       int len) {
+    const int t = threadIdx.x;
+    const bool tab = TAB && skk < 0;
+    tk = tab ? tkk + kbeg : nullptr;
+    sk = skk;
+    klen = len;
+    if (!tab) X += kbeg * skk;
+    if constexpr (KF) {
+      kf = t % BK;
 #pragma unroll
-    for (int i = 0; i < WT; ++i)
+      for (int i = 0; i < NPT; ++i) {
+        int64_t row = r0 + t / BK + STEP * i;
+        row = row < rows ? row : rows - 1;
+        p[i] = X + goff(tr, sr, row);
+      }
+    } else {
+      kf = UNI ? __builtin_amdgcn_readfirstlane(t / TS) : t / TS;
+      int64_t row = r0 + t % TS;
+      row = row < rows ? row : rows - 1;
+      p[0] = X + goff(tr, sr, row);
+    }
+    if constexpr (TAB) offsets(0);
+    else kn[0] = kf * sk;
+  }
+  // kn of the stage at k0, held inside the range (a table ends there)
+  __device__ __forceinline__ void offsets(int k0) {
 #pragma unroll
-      for (int j = 0; j < WT; ++j) {
-        int64_t n = n0 + wn * WH + j * 16 + lr;
-        if (n >= g.N) continue;
+    for (int i = 0; i < NKO; ++i) {
+      int k = k0 + kf + STEP * i;
+      k = k < klen ? k : klen - 1;
+      kn[i] = tk ? tk[k] : k * sk;
+    }
+  }
+  // the stage at k0; stages are loaded in order
+  __device__ __forceinline__ void load(int k0) {
+    if (TAB || k0 + BK <= klen) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          int64_t m = m0 + wm * WH + i * 16 + (TR::F64 ? 4 * r + lg : 4 * lg + r);
-          if (m < g.M) P[n * g.M + m] = acc[i][j][r];
+      for (int i = 0; i < NPT; ++i)
+        r[i] = p[KF ? i : 0][KF ? kn[0] : TAB ? kn[TAB ? i % NKO : 0] : kn[0] + (STEP * i) * sk];
+    } else {
+#pragma unroll
+      for (int i = 0; i < NPT; ++i) {
+        const int k = k0 + kf + (KF ? 0 : STEP * i);
+        r[i] = k < klen ? p[KF ? i : 0][k * sk] : (T)0;
+      }
+    }
+    if constexpr (TAB) {
+      if (k0 + BK > klen) {
+#pragma unroll
+        for (int i = 0; i < NPT; ++i)
+          if (k0 + kf + (KF ? 0 : STEP * i) >= klen) r[i] = (T)0;
+      }
+      offsets(k0 + BK);
+    } else {
+      kn[0] += BK * sk;
+    }
+  }
+  __device__ __forceinline__ void store(T* s) const {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+      const int m = KF ? t / BK + STEP * i : t % TS;
+      const int k = KF ? kf : kf + STEP * i;
+      s[k * TS + (m ^ (native_sw<T>(k) & MASK))] = r[i];
+    }
+  }
+};
+
+// WT consecutive elements, read from LDS in 16-byte pieces (aligned) or
+// written to memory (element-aligned)
+template <typename T, int WT>
+struct NativeVec {
+  typedef T vec __attribute__((ext_vector_type(WT)));
+  typedef T uvec __attribute__((ext_vector_type(WT), aligned(sizeof(T))));
+};
+
+template <typename T, int TS, bool AK, bool BKF, bool TAB>
+__global__ __launch_bounds__(256, TS == 128 ? 2 : 4) void gett_native_kernel(GettArgs g) {
+  constexpr bool F64 = std::is_same<T, double>::value;
+  constexpr int BK = 16, WH = TS / 2, WT = TS / 32, NK = BK / 4;
+  constexpr int MASK = TS < 64 ? TS - 1 : 63;
+  __shared__ __attribute__((aligned(16))) T smem[2][2][BK * TS];   // [buffer][operand]
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = wave & 1, wn = wave >> 1;
+  int64_t tm, tn;
+  tile_coords(g.tilesM, g.tilesN, tm, tn);
+  if (g.band && tm > tn + 1) return;   // whole workgroup, before any barrier
+  const int64_t m0 = tm * TS, n0 = tn * TS;
+  const int64_t kbeg = (int64_t)blockIdx.z * g.kchunk;
+  const int klen = (int)(kbeg + g.kchunk < g.K ? g.kchunk : g.K - kbeg);
+
+  NativeLoader<T, TS, BK, AK, TAB> la;
+  NativeLoader<T, TS, BK, BKF, TAB> lb;
+  la.init((const T*)g.A, m0, g.M, g.tAm, g.sAm, g.tAk, g.sAk, kbeg, klen);
+  lb.init((const T*)g.B, n0, g.N, g.tBn, g.sBn, g.tBk, g.sBk, kbeg, klen);
+
+  typedef typename std::conditional<F64, d4_t, f4_t>::type acc_t;
+  acc_t acc[WT][WT];
+#pragma unroll
+  for (int i = 0; i < WT; ++i)
+#pragma unroll
+    for (int j = 0; j < WT; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+
+  const int lr = lane & 15, lg = lane >> 4;
+  const int ma = wm * WH + WT * lr, nb = wn * WH + WT * lr;
+  la.load(0);
+  lb.load(0);
+  la.store(smem[0][0]);
+  lb.store(smem[0][1]);
+  if (BK < klen) {
+    la.load(BK);
+    lb.load(BK);
+  }
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < klen; k0 += BK) {
+    const T* As = smem[buf][0];
+    const T* Bs = smem[buf][1];
+    typedef typename NativeVec<T, WT>::vec vec;
+    vec a[2], b[2];
+    auto frag = [&](int kk) {
+      const int k = kk * 4 + lg, sw = native_sw<T>(k) & MASK;
+      a[kk & 1] = *(const vec*)(As + k * TS + (ma ^ sw));
+      b[kk & 1] = *(const vec*)(Bs + k * TS + (nb ^ sw));
+    };
+    frag(0);
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      if (kk + 1 < NK) frag(kk + 1);
+      if (kk == 1) {
+        // the first products are in the matrix pipe: store the next stage
+        // (the other buffer was last read before the barrier that ended
+        // the previous stage) and start the loads of the one after
+        __builtin_amdgcn_sched_barrier(0);
+        if (k0 + BK < klen) {
+          la.store(smem[buf ^ 1][0]);
+          lb.store(smem[buf ^ 1][1]);
+          if (k0 + 2 * BK < klen) {
+            la.load(k0 + 2 * BK);
+            lb.load(k0 + 2 * BK);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int j = 0; j < WT; ++j) {
+          if constexpr (F64)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[kk & 1][i], b[kk & 1][j],
+                                                             acc[i][j], 0, 0, 0);
+          else
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kk & 1][i], b[kk & 1][j],
+                                                             acc[i][j], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    buf ^= 1;
+  }
+
+  // lane holds D[q][lr] of each block, q = 4 lg + r (FP32) or 4 r + lg
+  // (FP64): rows m0 + wm WH + WT q + i, columns n .. n + WT - 1
+  const int64_t n = n0 + wn * WH + WT * lr;
+  const int64_t mb = m0 + wm * WH;
+  if (n >= g.N) return;
+  const int nw = g.N - n < WT ? (int)(g.N - n) : WT;   // live columns of this lane
+  typedef typename NativeVec<T, WT>::uvec uvec;
+  if (g.partial || (g.sCn == 1 && g.sCm >= 0)) {
+    T* P = g.partial ? (T*)g.partial + (int64_t)blockIdx.z * g.M * g.N : (T*)g.C;
+    const int64_t ld = g.partial ? g.N : g.sCm;
+    const double al = g.partial ? 1.0 : g.alpha, be = g.partial ? 0.0 : g.beta;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < WT; ++i) {
+        const int64_t m = mb + WT * (F64 ? 4 * r + lg : 4 * lg + r) + i;
+        if (m >= g.M) continue;
+        T* c = P + m * ld + n;
+        if (nw == WT) {
+          uvec v;
+          if (be != 0.0) {
+            const uvec o = *(const uvec*)c;
+#pragma unroll
+            for (int j = 0; j < WT; ++j) v[j] = (T)(al * (double)acc[i][j][r] + be * (double)o[j]);
+          } else {
+#pragma unroll
+            for (int j = 0; j < WT; ++j) v[j] = (T)(al * (double)acc[i][j][r]);
+          }
+          *(uvec*)c = v;
+        } else {
+#pragma unroll
+          for (int j = 0; j < WT; ++j)
+            if (j < nw) {
+              double v = al * (double)acc[i][j][r];
+              if (be != 0.0) v += be * (double)c[j];
+              c[j] = (T)v;
+            }
         }
       }
     return;
   }
   T* C = (T*)g.C;
-  if (g.sCm == 1 && g.sCn >= 0 && m0 + BM <= g.M && n0 + BN <= g.N) {
-    // interior tile of a column-major C: one column pointer per j and
-    // compile-time row offsets, no per-element bounds or offset arithmetic
-    // (a short epilogue: this code runs once per tile, from a cold
-    // instruction cache on small launches)
-    T* cb = C + (n0 + wn * WH + lr) * g.sCn + m0 + wm * WH + (TR::F64 ? lg : 4 * lg);
-    const double al = g.alpha, be = g.beta;
-    if (be != 0.0) {
 #pragma unroll
-      for (int j = 0; j < WT; ++j) {
-        T* cj = cb + (int64_t)(j * 16) * g.sCn;
+  for (int j = 0; j < WT; ++j) {
+    if (j >= nw) continue;
+    const int64_t on = goff(g.tCn, g.sCn, n + j);
 #pragma unroll
-        for (int i = 0; i < WT; ++i)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int mo = i * 16 + (TR::F64 ? 4 * r : r);
-            cj[mo] = (T)(al * (double)acc[i][j][r] + be * (double)cj[mo]);
-          }
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < WT; ++j) {
-        T* cj = cb + (int64_t)(j * 16) * g.sCn;
-#pragma unroll
-        for (int i = 0; i < WT; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) cj[i * 16 + (TR::F64 ? 4 * r : r)] =
-              (T)(al * (double)acc[i][j][r]);
-      }
-    }
-    return;
-  }
-  if (g.sCn == 1 && g.sCm >= 0 && m0 + BM <= g.M && n0 + BN <= g.N) {
-    // the same for a row-major C (itg_gemm's C^T): one row pointer per
-    // (i, r), compile-time column offsets
-    T* cb = C + (m0 + wm * WH + (TR::F64 ? lg : 4 * lg)) * g.sCm + n0 + wn * WH + lr;
-    const double al = g.alpha, be = g.beta;
-#pragma unroll
-    for (int i = 0; i < WT; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        T* ci = cb + (int64_t)(i * 16 + (TR::F64 ? 4 * r : r)) * g.sCm;
-        if (be != 0.0) {
-#pragma unroll
-          for (int j = 0; j < WT; ++j)
-            ci[j * 16] = (T)(al * (double)acc[i][j][r] + be * (double)ci[j * 16]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < WT; ++j) ci[j * 16] = (T)(al * (double)acc[i][j][r]);
-        }
-      }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < WT; ++i)
-#pragma unroll
-    for (int j = 0; j < WT; ++j) {
-      int64_t n = n0 + wn * WH + j * 16 + lr;
-      if (n >= g.N) continue;
-      int64_t on = goff(g.tCn, g.sCn, n);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        int64_t m = m0 + wm * WH + i * 16 + (TR::F64 ? 4 * r + lg : 4 * lg + r);
+      for (int i = 0; i < WT; ++i) {
+        const int64_t m = mb + WT * (F64 ? 4 * r + lg : 4 * lg + r) + i;
         if (m >= g.M) continue;
-        int64_t o = on + goff(g.tCm, g.sCm, m);
+        const int64_t o = on + goff(g.tCm, g.sCm, m);
         double v = g.alpha * (double)acc[i][j][r];
         if (g.beta != 0.0) v += g.beta * (double)C[o];
         C[o] = (T)v;
       }
-    }
+  }
 }
 
 // split-K reduction + epilogue
@@ -358,7 +631,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GettArgs g, int nspl
        e += (int64_t)gridDim.x * blockDim.x) {
     double s = 0.0;
     for (int z = 0; z < nsplit; ++z) s += (double)P[z * MN + e];
-    int64_t m = e % g.M, n = e / g.M;
+    int64_t n = e % g.N, m = e / g.N;
     int64_t o = goff(g.tCm, g.sCm, m) + goff(g.tCn, g.sCn, n);
     double v = g.alpha * s;
     if (g.beta != 0.0) v += g.beta * (double)C[o];
@@ -726,22 +999,14 @@ static int build_plan(itg_ctx* ctx, const std::string& key, int rA, const int64_
   return ITG_OK;
 }
 
-template <typename T, int MODE, int TS = 128>
+template <typename T, int MODE>
 static int launch_gett_t(itg_ctx* ctx, GettArgs& g, bool ak, bool bk) {
-  using TR = GettTraits<T, MODE, TS>;
-  using CT = typename TR::CT;
+  using TR = GettTraits<MODE>;
+  using CT = float;
   g.tilesM = (g.M + TR::BM - 1) / TR::BM;
   g.tilesN = (g.N + TR::BN - 1) / TR::BN;
   int64_t tiles = g.tilesM * g.tilesN;
   if (tiles > 0x7fffffff) return itg_fail(ctx, ITG_EUNSUPPORTED, "contraction too large");
-  if constexpr (TR::F64 && TS == 128) {
-    // FP64 with fewer 128 x 128 tiles than workgroup slots, or a short K:
-    // 64 x 64 tiles give each wave a quarter of the MFMA chain per k step
-    // and four times the workgroups, more of them resident per CU (the
-    // K = 64 trailing updates of the eigensolver)
-    if (tiles < 2 * (int64_t)std::max(ctx->num_cu, 1) || g.K <= 128)
-      return launch_gett_t<T, MODE, 64>(ctx, g, ak, bk);
-  }
   // split K when the output has too few tiles to fill the chip
   int nsplit = 1;
   int64_t target = 2 * (int64_t)std::max(ctx->num_cu, 1);
@@ -774,15 +1039,124 @@ static int launch_gett_t(itg_ctx* ctx, GettArgs& g, bool ak, bool bk) {
   }
   dim3 grid((unsigned)tiles, 1, (unsigned)nsplit);
   int tk = itg_tstart(ctx, ITG_K_GETT);
-  if (ak && bk) gett_kernel<T, MODE, true, true, TS><<<grid, 256, 0, ctx->stream>>>(g);
-  else if (ak) gett_kernel<T, MODE, true, false, TS><<<grid, 256, 0, ctx->stream>>>(g);
-  else if (bk) gett_kernel<T, MODE, false, true, TS><<<grid, 256, 0, ctx->stream>>>(g);
-  else gett_kernel<T, MODE, false, false, TS><<<grid, 256, 0, ctx->stream>>>(g);
+  if (ak && bk) gett_kernel<T, MODE, true, true><<<grid, 256, 0, ctx->stream>>>(g);
+  else if (ak) gett_kernel<T, MODE, true, false><<<grid, 256, 0, ctx->stream>>>(g);
+  else if (bk) gett_kernel<T, MODE, false, true><<<grid, 256, 0, ctx->stream>>>(g);
+  else gett_kernel<T, MODE, false, false><<<grid, 256, 0, ctx->stream>>>(g);
   ITG_LAUNCH_CHECK(ctx);
   itg_tstop(ctx, tk, ITG_K_GETT, 2.0 * g.M * g.N * g.K,
             (double)sizeof(T) * (g.M * g.K + g.K * g.N + g.M * g.N * (g.beta != 0.0 ? 2 : 1)));
   if (nsplit > 1) {
     splitk_reduce_kernel<T, CT><<<itg_blocks(g.M * g.N, 256, 4096), 256, 0, ctx->stream>>>(g, nsplit);
+    ITG_LAUNCH_CHECK(ctx);
+  }
+  return ITG_OK;
+}
+
+template <typename T, int TS, bool TAB>
+static void native_kernel(itg_ctx* ctx, const GettArgs& g, dim3 grid, bool ak, bool bk) {
+  hipStream_t st = ctx->stream;
+  if (ak && bk) gett_native_kernel<T, TS, true, true, TAB><<<grid, 256, 0, st>>>(g);
+  else if (ak) gett_native_kernel<T, TS, true, false, TAB><<<grid, 256, 0, st>>>(g);
+  else if (bk) gett_native_kernel<T, TS, false, true, TAB><<<grid, 256, 0, st>>>(g);
+  else gett_native_kernel<T, TS, false, false, TAB><<<grid, 256, 0, st>>>(g);
+}
+
+template <typename T, int TS>
+static void native_kernel(itg_ctx* ctx, const GettArgs& g, dim3 grid, bool ak, bool bk) {
+  if (g.sAk < 0 || g.sBk < 0) native_kernel<T, TS, true>(ctx, g, grid, ak, bk);
+  else native_kernel<T, TS, false>(ctx, g, grid, ak, bk);
+}
+
+// Tile and K split of the native kernel by estimated time. A CU with nw
+// workgroups takes lat + (nw - 1) mf per 16-deep stage: lat is the stage
+// of a workgroup alone on its CU (barrier, LDS and load latency exposed), mf
+// what each further one adds; a split adds a launch and its partials'
+// traffic. Measured on MI355X (us; one workgroup per CU and many):
+//            FP64 lat  mf      FP32 lat  mf
+//   32 x 32       0.44 0.23         0.30 0.146
+//   64 x 64       0.97 0.55         0.50 0.31
+// 128 x 128          -    -         1.29 1.0
+// FP64 at 128 x 128 gains nothing over 64 x 64 (59 against 61 TFLOP/s at
+// 4096^3: 64 cycles per product hide the smaller tile's reads) and rounds
+// worse, so it is not built. The estimates are within 15% of the measured
+// times over 18 shapes, 80 x 20 x 100 to 4096^3, and pick the fastest tile
+// and split or one within 10% of it.
+struct NativeChoice {
+  int ts, nsplit;
+};
+static NativeChoice choose_native(const itg_ctx* ctx, const GettArgs& g, bool f64) {
+  struct Tile {
+    int ts;
+    double lat, mf;
+  };
+  static const Tile t64[] = {{32, 0.44, 0.23}, {64, 0.97, 0.55}};
+  static const Tile t32[] = {{32, 0.30, 0.146}, {64, 0.50, 0.31}, {128, 1.29, 1.0}};
+  const Tile* tiles = f64 ? t64 : t32;
+  const int nt = f64 ? 2 : 3;
+  const double cus = std::max(ctx->num_cu, 1);
+  const double es = f64 ? 8.0 : 4.0;
+  const double mn = (double)g.M * (double)g.N;
+  NativeChoice best = {64, 1};
+  double tbest = -1.0;
+  for (int i = 0; i < nt; ++i) {
+    const int ts = tiles[i].ts;
+    // a band of one tile above the diagonal has to hold 64 of them
+    if (g.band && ts < 64) continue;
+    const double nm = (double)((g.M + ts - 1) / ts), nn = (double)((g.N + ts - 1) / ts);
+    const double wg = g.band ? 0.5 * nm * (nn + 3.0) : nm * nn;
+    for (int sp = 1; sp <= 64; sp *= 2) {
+      if (sp > 1 && (g.band || g.K < 32 * (int64_t)sp)) break;
+      // no more partials than a no-alloc call's scratch holds
+      if (sp > 1 && ctx->fixed_ws && mn * es * sp > (double)ctx->fixed_ws_bytes) break;
+      const double nw = std::ceil(wg * sp / cus);
+      const double stages = std::ceil(std::ceil((double)g.K / sp) / 16.0);
+      double t = stages * (tiles[i].lat + (nw - 1.0) * tiles[i].mf);
+      if (sp > 1) t += 2.5 + (sp + 1.0) * mn * es / 3.0e6;
+      if (tbest < 0.0 || t < tbest) {
+        tbest = t;
+        best = {ts, sp};
+      }
+    }
+  }
+  return best;
+}
+
+template <typename T>
+static int launch_native(itg_ctx* ctx, GettArgs& g, bool ak, bool bk) {
+  constexpr bool F64 = std::is_same<T, double>::value;
+  NativeChoice c = choose_native(ctx, g, F64);
+  g.tilesM = (g.M + c.ts - 1) / c.ts;
+  g.tilesN = (g.N + c.ts - 1) / c.ts;
+  const int64_t tiles = g.tilesM * g.tilesN;
+  if (tiles > 0x7fffffff) return itg_fail(ctx, ITG_EUNSUPPORTED, "contraction too large");
+  // a workgroup counts its k in 32 bits
+  constexpr int64_t kMaxChunk = (int64_t)1 << 30;
+  int64_t nsplit = std::max<int64_t>(c.nsplit, (g.K + kMaxChunk - 1) / kMaxChunk);
+  g.partial = nullptr;
+  g.kchunk = g.K;
+  if (nsplit > 1) {
+    const int64_t chunk = ((g.K + nsplit - 1) / nsplit + 15) / 16 * 16;
+    nsplit = (g.K + chunk - 1) / chunk;
+    g.kchunk = chunk;
+    void* ws = ctx->fixed_ws;
+    if (!ws) {
+      int rc = itg_workspace(ctx, (size_t)nsplit * g.M * g.N * sizeof(T), &ws);
+      if (rc) return rc;
+    }
+    g.partial = ws;
+  }
+  dim3 grid((unsigned)tiles, 1, (unsigned)nsplit);
+  const int tk = itg_tstart(ctx, ITG_K_GETT);
+  if (c.ts == 32) native_kernel<T, 32>(ctx, g, grid, ak, bk);
+  else if (F64 || c.ts == 64) native_kernel<T, 64>(ctx, g, grid, ak, bk);
+  else native_kernel<float, 128>(ctx, g, grid, ak, bk);
+  ITG_LAUNCH_CHECK(ctx);
+  itg_tstop(ctx, tk, ITG_K_GETT, 2.0 * g.M * g.N * g.K,
+            (double)sizeof(T) * (g.M * g.K + g.K * g.N + g.M * g.N * (g.beta != 0.0 ? 2 : 1)));
+  if (nsplit > 1) {
+    splitk_reduce_kernel<T, T><<<itg_blocks(g.M * g.N, 256, 4096), 256, 0, ctx->stream>>>(
+        g, (int)nsplit);
     ITG_LAUNCH_CHECK(ctx);
   }
   return ITG_OK;
@@ -803,12 +1177,12 @@ static int launch_gett(itg_ctx* ctx, int dtype, int mode, GettArgs& g, bool ak, 
     return ITG_OK;
   }
   if (dtype == ITG_F64) {
-    if (mode == ITG_MODE_NATIVE) return launch_gett_t<double, ITG_MODE_NATIVE>(ctx, g, ak, bk);
+    if (mode == ITG_MODE_NATIVE) return launch_native<double>(ctx, g, ak, bk);
     if (mode == ITG_MODE_F32) return launch_gett_t<double, ITG_MODE_F32>(ctx, g, ak, bk);
     return launch_gett_t<double, ITG_MODE_BF16X3>(ctx, g, ak, bk);
   }
   if (mode == ITG_MODE_BF16X3) return launch_gett_t<float, ITG_MODE_BF16X3>(ctx, g, ak, bk);
-  return launch_gett_t<float, ITG_MODE_NATIVE>(ctx, g, ak, bk);
+  return launch_native<float>(ctx, g, ak, bk);
 }
 
 // A contraction whose M, N and K modes each merge into one stride is a plain
