@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "dc_core.h"
@@ -1657,6 +1658,100 @@ __global__ __launch_bounds__(256) void jac_round_kernel(double* __restrict__ W, 
   }
 }
 
+// ------------------------------------- orthogonalising nearly orthogonal columns
+// G = W^T W of columns that a preceding eigenbasis left nearly orthogonal.
+// A pair (i, j), i < j, is converged as in jac_round_kernel: its cosine is
+// within tol, or a column is at the rounding level of ||A||. Any other is
+// turned by the angle theta = atan(2 g_ij / (g_jj - g_ii)) / 2 that
+// annihilates it; all small angles are applied at once as a matrix product
+// (columns W X, X = I + K + K^2/2, K antisymmetric), which squares the
+// cosines like a Jacobi sweep. Pairs at a larger angle (near-equal columns,
+// or columns whose directions the eigenbasis did not resolve) are left for
+// a new eigenbasis of the columns from the first of them on.
+constexpr double ORTHO_ANGLE = 0.02;   // largest angle turned by K
+
+__device__ __forceinline__ bool ortho_pair(const double* __restrict__ G, int n, int i, int j,
+                                           double tol, double small2, double* rel,
+                                           double* theta) {
+  const double gi = G[(size_t)i * n + i], gj = G[(size_t)j * n + j];
+  const double g = G[(size_t)j * n + i];
+  *rel = (gi > small2 && gj > small2) ? fabs(g) / sqrt(gi * gj) : 0.0;
+  if (*rel <= tol) return false;
+  const double dd = gj - gi;
+  // |theta| <= pi / 4: the pair's order is kept when the two are equal
+  *theta = dd == 0.0 ? copysign(0.78539816339744831, g) : 0.5 * atan(2.0 * g / dd);
+  return true;
+}
+
+// stat[0] = largest cosine (bits of a non-negative double), stat[1] = first
+// index of a pair at a large angle (initialised to 0 and n); exact, so the
+// order of the atomics does not matter
+__global__ __launch_bounds__(256) void ortho_stat_kernel(const double* __restrict__ G, int n,
+                                                         double tol, double small2,
+                                                         unsigned long long* stat) {
+  const int64_t tot = (int64_t)n * n;
+  double mx = 0.0;
+  int first = n;
+  for (int64_t e = blockIdx.x * 256LL + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256) {
+    const int i = (int)(e % n), j = (int)(e / n);
+    if (i >= j) continue;
+    double rel, th;
+    if (ortho_pair(G, n, i, j, tol, small2, &rel, &th) && fabs(th) > ORTHO_ANGLE)
+      first = min(first, i);
+    mx = fmax(mx, rel);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    mx = fmax(mx, __shfl_xor(mx, o, 64));
+    first = min(first, __shfl_xor(first, o, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMax(stat, (unsigned long long)__double_as_longlong(mx));
+    if (first < n) atomicMin(stat + 1, (unsigned long long)first);
+  }
+}
+
+__global__ void ortho_init_kernel(int n, unsigned long long* stat) {
+  stat[0] = 0;
+  stat[1] = (unsigned long long)n;
+}
+
+// K over the pairs with i < first (stat[1]) and per-block partials of its
+// squared norm
+__global__ __launch_bounds__(256) void ortho_k_kernel(const double* __restrict__ G, int n,
+                                                      double tol, double small2,
+                                                      const unsigned long long* stat,
+                                                      double* __restrict__ K,
+                                                      double* __restrict__ part) {
+  __shared__ double sh4[4];
+  const int first = (int)stat[1];
+  const int64_t tot = (int64_t)n * n;
+  double s = 0.0;
+  for (int64_t e = blockIdx.x * 256LL + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256) {
+    const int r = (int)(e % n), c = (int)(e / n);
+    const int i = min(r, c), j = max(r, c);
+    double rel, th, v = 0.0;
+    if (i != j && i < first && ortho_pair(G, n, i, j, tol, small2, &rel, &th) &&
+        fabs(th) <= ORTHO_ANGLE)
+      v = r < c ? th : -th;
+    K[e] = v;
+    s += v * v;
+  }
+  s = block_sum256(s, sh4);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// X = X + a I + b Y
+__global__ void add_diag_kernel(int n, double a, double b, const double* __restrict__ Y,
+                                double* __restrict__ X) {
+  const int64_t tot = (int64_t)n * n;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    double v = X[e] + (Y ? b * Y[e] : 0.0);
+    if (e % n == e / n) v += a;
+    X[e] = v;
+  }
+}
+
 __global__ __launch_bounds__(256) void col_norm_kernel(const double* __restrict__ W, int m, int ncols,
                                                        double* __restrict__ out) {
   int lane = threadIdx.x & 63;
@@ -1773,6 +1868,109 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   (void)f32;
 }
 
+// Buffers of ortho_columns: W and V with a second buffer each (swapped as
+// they are rotated), and three n x n matrices.
+struct OrthoBufs {
+  double *W, *W2, *V, *V2, *G, *K, *X, *wG;
+  double* part;               // 1024 partials
+  unsigned long long* stat;   // 2
+};
+
+// Makes the columns of W (rows x n, already W = A V with V an eigenbasis of
+// A^T A, columns by descending norm) orthogonal to tol by rotations applied
+// to W and V alike: matrix products while every angle is small, a new
+// eigenbasis of the trailing columns where one is not. *done is false if
+// some pair has to be left to the Jacobi sweeps.
+//
+// Against the sweeps alone: a sweep is n - 1 launches of n / 2 column pairs,
+// ~10 us each whatever they do (2 sweeps, 40 ms, at 2048 x 2048, and one
+// more to see that nothing is left); a pass here is one Gram product and, if
+// it turns anything, four to six more of the same size (0.25 to 0.35 ms each).
+int ortho_columns(itg_ctx* ctx, int rows, int n, double tol, double small2, OrthoBufs& b,
+                  bool* done) {
+  constexpr int PARTS = 1024;
+  *done = false;
+  int last = 0;   // first column of the latest eigenbasis
+  const unsigned gb = (unsigned)itg_blocks((int64_t)n * n, 256, PARTS);
+  for (int pass = 0; pass < 10; ++pass) {
+    int rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', n, n, rows, 1.0, b.W, rows, b.W,
+                      rows, 0.0, b.G, n);
+    if (rc) return rc;
+    ortho_init_kernel<<<1, 1, 0, ctx->stream>>>(n, b.stat);
+    ortho_stat_kernel<<<gb, 256, 0, ctx->stream>>>(b.G, n, tol, small2, b.stat);
+    ortho_k_kernel<<<gb, 256, 0, ctx->stream>>>(b.G, n, tol, small2, b.stat, b.K, b.part);
+    ITG_LAUNCH_CHECK(ctx);
+    unsigned long long st[2];
+    std::vector<double> part(gb);
+    ITG_HIP(ctx, hipMemcpyAsync(st, b.stat, sizeof st, hipMemcpyDeviceToHost, ctx->stream));
+    ITG_HIP(ctx, hipMemcpyAsync(part.data(), b.part, gb * sizeof(double), hipMemcpyDeviceToHost,
+                                ctx->stream));
+    ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    double mx, kf = 0.0;
+    memcpy(&mx, &st[0], sizeof mx);
+    for (double x : part) kf += x;
+    kf = std::sqrt(kf);
+    if (mx <= tol) {
+      *done = true;
+      return ITG_OK;
+    }
+    const int first = (int)st[1];
+    // X^T X - I = K^4 / 4 for X = I + K + K^2 / 2; each polishing step
+    // X (3 I - X^T X) / 2 squares it
+    if (!(kf <= 0.3)) return ITG_OK;
+    if (kf > 0.0) {
+      rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', n, n, n, 0.5, b.K, n, b.K, n,
+                             0.0, b.X, n);
+      if (rc) return rc;
+      add_diag_kernel<<<gb, 256, 0, ctx->stream>>>(n, 1.0, 1.0, b.K, b.X);
+      for (int q = kf <= 1e-4 ? 0 : kf <= 1e-2 ? 1 : 2; q > 0; --q) {
+        rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', n, n, n, -0.5, b.X, n, b.X,
+                               n, 0.0, b.K, n);
+        if (rc) return rc;
+        add_diag_kernel<<<gb, 256, 0, ctx->stream>>>(n, 1.5, 0.0, nullptr, b.K);
+        rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', n, n, n, 1.0, b.X, n, b.K,
+                               n, 0.0, b.G, n);
+        if (rc) return rc;
+        std::swap(b.X, b.G);
+      }
+      rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', rows, n, n, 1.0, b.W, rows,
+                             b.X, n, 0.0, b.W2, rows);
+      if (rc) return rc;
+      rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', n, n, n, 1.0, b.V, n, b.X, n,
+                             0.0, b.V2, n);
+      if (rc) return rc;
+      std::swap(b.W, b.W2);
+      std::swap(b.V, b.V2);
+    }
+    if (first < n) {
+      if (first <= last) return ITG_OK;   // no progress at this scale
+      last = first;
+      const int t = n - first;
+      const size_t wo = (size_t)first * rows, vo = (size_t)first * n;
+      rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', t, t, rows, 1.0, b.W + wo, rows,
+                    b.W + wo, rows, 0.0, b.G, t);
+      if (rc) return rc;
+      int64_t kg = 0;
+      double teg = 0.0, dcg = 0.0;
+      rc = itg_eigh_trunc(ctx, ITG_F64, t, b.G, b.wG, b.X, 0, -1.0, 0, 1, &kg, &teg, &dcg);
+      if (rc) return rc;
+      rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', rows, t, t, 1.0, b.W + wo,
+                             rows, b.X, t, 0.0, b.W2 + wo, rows);
+      if (rc) return rc;
+      rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', n, t, t, 1.0, b.V + vo, n,
+                             b.X, t, 0.0, b.V2 + vo, n);
+      if (rc) return rc;
+      ITG_HIP(ctx, hipMemcpyAsync(b.W2, b.W, wo * sizeof(double), hipMemcpyDeviceToDevice,
+                                  ctx->stream));
+      ITG_HIP(ctx, hipMemcpyAsync(b.V2, b.V, vo * sizeof(double), hipMemcpyDeviceToDevice,
+                                  ctx->stream));
+      std::swap(b.W, b.W2);
+      std::swap(b.V, b.V2);
+    }
+  }
+  return ITG_OK;
+}
+
 // smallest column count at which the Jacobi SVD is preconditioned by the
 // Gram matrix's eigenvectors
 constexpr int SVD_PRECOND_MIN = 64;
@@ -1807,7 +2005,9 @@ extern "C" int itg_svd_trunc(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, 
   const bool precond = cols >= SVD_PRECOND_MIN;
   size_t bytes = ((size_t)rows * cols * 2 + (size_t)cols * cols + (size_t)rows * cols +
                   (size_t)cols * cols + 8 * (size_t)N + 64) * sizeof(double) + 16 * 256 +
-                 (precond ? ((size_t)rows * cols + (size_t)cols * cols + cols) * 8 + 3 * 256 : 0);
+                 (precond ? ((size_t)rows * cols + 4 * (size_t)cols * cols + cols + 1024 + 2) * 8 +
+                                8 * 256
+                          : 0);
   if (bytes > ctx->svd_ws_bytes) {
     if (ctx->svd_ws) {
       ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1838,14 +2038,19 @@ extern "C" int itg_svd_trunc(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, 
   if (rc) return rc;
   if (tr) transpose_kernel<<<itg_blocks((int64_t)m * n, 256, 8192), 256, 0, ctx->stream>>>(m, n, A64, W);
   else ITG_HIP(ctx, hipMemcpyAsync(W, A64, (size_t)m * n * 8, hipMemcpyDeviceToDevice, ctx->stream));
+  OrthoBufs ob = {};
   if (precond) {
     // Jacobi preconditioned by the Gram matrix's eigenvectors: W <- W V0
     // with W^T W = V0 diag(w) V0^T, V <- V0. The columns of W V0 are
-    // orthogonal up to eps ||A||^2 / (s_i s_j), so the one-sided sweeps
-    // below (which keep their relative accuracy) converge in a few sweeps
+    // orthogonal up to eps ||A||^2 / (s_i s_j); ortho_columns turns what is
+    // left by matrix products, and the one-sided sweeps below take over
+    // where it cannot finish
     double* G = cv.take<double>((size_t)cols * cols);
     double* W2 = cv.take<double>((size_t)rows * cols);
     double* wG = cv.take<double>(cols);
+    ob = {W2, W, V, cv.take<double>((size_t)cols * cols), G, cv.take<double>((size_t)cols * cols),
+          cv.take<double>((size_t)cols * cols), wG, cv.take<double>(1024),
+          cv.take<unsigned long long>(2)};
     if (cv.off > bytes) return itg_fail(ctx, ITG_EOOM, "svd: workspace layout overflow");
     // (one operand buffer: the exactly symmetric product)
     rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', cols, cols, rows, 1.0, W, rows, W, rows,
@@ -1858,7 +2063,6 @@ extern "C" int itg_svd_trunc(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, 
     rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', rows, cols, cols, 1.0, W, rows,
                            V, cols, 0.0, W2, rows);
     if (rc) return rc;
-    W = W2;
   } else {
     qr_init_q_kernel<<<itg_blocks((int64_t)cols * cols, 256, 8192), 256, 0, ctx->stream>>>(cols, cols, V);
     ITG_LAUNCH_CHECK(ctx);
@@ -1870,6 +2074,12 @@ extern "C" int itg_svd_trunc(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, 
   double small2 = (ITG_DC_EPS * fro) * (ITG_DC_EPS * fro);
   std::vector<double> hoffs(N / 2);
   bool conv = cols < 2;
+  if (precond) {
+    rc = ortho_columns(ctx, rows, cols, tol, small2, ob, &conv);
+    if (rc) return rc;
+    W = ob.W;
+    V = ob.V;
+  }
   for (int sweep = 0; sweep < 60 && !conv; ++sweep) {
     ITG_HIP(ctx, hipMemsetAsync(offs, 0, (N / 2) * sizeof(double), ctx->stream));
     for (int rnd = 0; rnd < N - 1; ++rnd) {
