@@ -1890,9 +1890,9 @@ int ortho_columns(itg_ctx* ctx, int rows, int n, double tol, double small2, Orth
                   bool* done) {
   constexpr int PARTS = 1024;
   *done = false;
-  int last = 0;   // first column of the latest eigenbasis
+  int64_t fresh = 0;   // columns given a new eigenbasis so far
   const unsigned gb = (unsigned)itg_blocks((int64_t)n * n, 256, PARTS);
-  for (int pass = 0; pass < 10; ++pass) {
+  for (int pass = 0; pass < 14; ++pass) {
     int rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', n, n, rows, 1.0, b.W, rows, b.W,
                       rows, 0.0, b.G, n);
     if (rc) return rc;
@@ -1918,6 +1918,14 @@ int ortho_columns(itg_ctx* ctx, int rows, int n, double tol, double small2, Orth
     // X^T X - I = K^4 / 4 for X = I + K + K^2 / 2; each polishing step
     // X (3 I - X^T X) / 2 squares it
     if (!(kf <= 0.3)) return ITG_OK;
+    // the trailing columns' scale: the eigensolver's deflation is absolute
+    // below unit norm
+    double gf = 1.0;
+    if (first < n) {
+      ITG_HIP(ctx, hipMemcpyAsync(&gf, b.G + (size_t)first * n + first, sizeof(double),
+                                  hipMemcpyDeviceToHost, ctx->stream));
+      ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    }
     if (kf > 0.0) {
       rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', n, n, n, 0.5, b.K, n, b.K, n,
                              0.0, b.X, n);
@@ -1943,12 +1951,14 @@ int ortho_columns(itg_ctx* ctx, int rows, int n, double tol, double small2, Orth
       std::swap(b.V, b.V2);
     }
     if (first < n) {
-      if (first <= last) return ITG_OK;   // no progress at this scale
-      last = first;
+      // a spectrum over the whole range of a double takes about 1.5 n (each
+      // new basis resolves seven digits and disturbs the next ones a little)
       const int t = n - first;
+      fresh += t;
+      if (fresh > 6 * (int64_t)n) return ITG_OK;
       const size_t wo = (size_t)first * rows, vo = (size_t)first * n;
-      rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', t, t, rows, 1.0, b.W + wo, rows,
-                    b.W + wo, rows, 0.0, b.G, t);
+      rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', t, t, rows,
+                    std::ldexp(1.0, -std::ilogb(gf)), b.W + wo, rows, b.W + wo, rows, 0.0, b.G, t);
       if (rc) return rc;
       int64_t kg = 0;
       double teg = 0.0, dcg = 0.0;
