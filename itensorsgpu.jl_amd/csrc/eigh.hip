@@ -425,96 +425,187 @@ __global__ __launch_bounds__(256) void trd_post_kernel(
   }
 }
 
-constexpr int TRD_TAIL = 128;   // trailing blocks this small are reduced in LDS
+// trailing blocks this small are reduced by one workgroup: 192 x 192 doubles
+// are 144 of a thread's 256 registers; 256 rows would not fit
+constexpr int TRD_TAIL = 192;
 
-__device__ __forceinline__ double block_sum1024(double v, double* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double s = 0.0;
-  for (int q = 0; q < 16; ++q) s += red[q];
-  return s;
+// DPP lane exchange of a double within a row of 16 lanes
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
 }
 
-// The trailing block of m = n - p <= TRD_TAIL rows and columns (every
-// earlier update applied, its lower triangle current) reduced to tridiagonal
-// form in LDS by one 1024-thread block, column by column (dsytd2): y = tau
-// A22 v, w = y - tau/2 (y^T v) v, A22 -= v w^T + w v^T. d, e, tau and the
+// sum over each row of 16 lanes, the same bits in all of them
+__device__ __forceinline__ double row16_sum(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  v += dpp_d<0x141>(v);
+  v += dpp_d<0x140>(v);
+  return v;
+}
+
+// The trailing block of m = n - p <= 32 RB rows and columns (every earlier
+// update applied, its lower triangle current) reduced to tridiagonal form by
+// one 512-thread workgroup, column by column (dsytd2): y = tau A22 v,
+// w = y - tau/2 (y^T v) v, A22 -= v w^T + w v^T. d, e, tau and the
 // reflectors (v(j+1) = 1 stored) go where the per-column kernels put them.
-__global__ __launch_bounds__(1024) void trd_tail_kernel(double* __restrict__ A, int n, int p,
-                                                        double* __restrict__ d,
-                                                        double* __restrict__ e,
-                                                        double* __restrict__ tau) {
-  extern __shared__ double S[];
-  __shared__ double yp[8][TRD_TAIL];
-  __shared__ double red[16];
-  const int m = n - p, ld = m + 1;
-  double* a = S;                    // a[r + c ld], both triangles
-  double* v = S + (size_t)m * ld;   // [m]
-  double* w = v + m;                // [m]
-  const int t = threadIdx.x;
-  for (int q = t; q < m * m; q += 1024) {
-    const int r = q % m, c = q / m;
-    const int hi = r > c ? r : c, lo = r > c ? c : r;
-    a[r + c * ld] = A[(size_t)(p + hi) + (size_t)(p + lo) * n];
-  }
-  __syncthreads();
-  for (int k = 0; k + 1 < m; ++k) {
-    double s = 0.0;
-    for (int r = k + 2 + t; r < m; r += 1024) {
-      const double x = a[r + k * ld];
-      s += x * x;
-    }
-    const double xn2 = block_sum1024(s, red);
-    const double alpha = a[k + 1 + k * ld];
-    double beta = alpha, tv = 0.0, scale = 1.0;
-    if (xn2 != 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-      tv = (beta - alpha) / beta;
-      scale = 1.0 / (alpha - beta);
-    }
-    if (t == 0) {
-      d[p + k] = a[k + k * ld];
-      e[p + k] = beta;
-      tau[p + k] = tv;
-    }
-    for (int r = t; r < m; r += 1024) {
-      const double vr = r <= k ? 0.0 : (r == k + 1 ? 1.0 : a[r + k * ld] * scale);
-      v[r] = vr;
-      if (r > k) A[(size_t)(p + r) + (size_t)(p + k) * n] = vr;
-    }
-    __syncthreads();
-    {
-      // A22 v: row r = t % TRD_TAIL, columns c = k + 1 + part (mod 8)
-      const int r = t % TRD_TAIL, part = t / TRD_TAIL;
-      double acc = 0.0;
-      if (r < m && r > k)
-        for (int c = k + 1 + part; c < m; c += 8) acc += a[r + c * ld] * v[c];
-      yp[part][r] = acc;
-    }
-    __syncthreads();
-    double yv = 0.0;
-    if (t < m) {
-      double y = 0.0;
-      if (t > k) {
-        for (int q = 0; q < 8; ++q) y += yp[q][t];
-        y *= tv;
-        yv = y * v[t];
+//
+// Bound: the latency of a column's serial chain. The block stays in
+// registers (both triangles): thread (i, c), i = lane % 32, c = 2 wave +
+// lane / 32, holds rows i + 32 a, a < RB, of columns c + 16 b, b < 2 RB. The
+// columns are taken 32 at a time (phase RA: rows and columns from 32 RA on
+// are live), so that the code of a phase has no tests for finished blocks. A
+// column lies in one half-wave, so its norm is a half-wave sum; A22 v is
+// formed as column sums (the block is symmetric), a lane's partials first
+// halved by one exchange between the half-wave's two rows of 16 lanes; only
+// v, y and the partials of y^T v pass through LDS, two barriers per column.
+// 192 columns take 0.34 ms, 1.8 us each (two launches a column before: 8.5;
+// the LDS-resident tail of 128 rows, eight barriers a column: 5.7).
+template <int RB>
+struct TrdTail {
+  static constexpr int CB = 2 * RB;
+  double* A;
+  double *d, *e, *tau;
+  double *vs, *ys, *part, *scal;   // LDS: 2 x 32 RB, 2 x 32 RB, 2 x 8, 2
+  int n, p, m, lane, wave, i, c;
+  bool up;
+  double x[RB][CB];
+
+  template <int RA>
+  __device__ __forceinline__ void phase() {
+    constexpr int CA = 2 * RA, NC = CB - CA, NR = RB - RA;   // live blocks
+    const int k1 = min(m - 1, 32 * RA + 32);
+    for (int k = 32 * RA; k < k1; ++k) {
+      const int buf = k & 1;
+      double* v = vs + buf * 32 * RB;
+      double* y = ys + buf * 32 * RB;
+      if (c == (k & 15)) {
+        // this half-wave holds column k: block CA or CA + 1
+        const bool hi = (k & 16) != 0;
+        double col[RB];
+#pragma unroll
+        for (int a = RA; a < RB; ++a) col[a] = hi ? x[a][CA + 1] : x[a][CA];
+        double s = 0.0, al = 0.0;
+#pragma unroll
+        for (int a = RA; a < RB; ++a) {
+          const int r = i + 32 * a;
+          if (r > k + 1) s += col[a] * col[a];
+          if (a == ((k + 1) >> 5)) al = col[a];
+        }
+        const double alpha = __shfl(al, (lane & 32) | ((k + 1) & 31), 64);
+        s = row16_sum(s);
+        const double xn2 = s + __shfl_xor(s, 16, 64);
+        double beta = alpha, tv = 0.0, scale = 1.0;
+        if (xn2 != 0.0) {
+          beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
+          tv = (beta - alpha) / beta;
+          scale = 1.0 / (alpha - beta);
+        }
+#pragma unroll
+        for (int a = RA; a < RB; ++a) {
+          const int r = i + 32 * a;
+          const double vr = r <= k ? 0.0 : (r == k + 1 ? 1.0 : col[a] * scale);
+          v[r] = vr;
+          if (r > k && r < m) A[(size_t)(p + r) + (size_t)(p + k) * n] = vr;
+        }
+        if (i == 0) {
+          e[p + k] = beta;
+          tau[p + k] = tv;
+          scal[buf] = tv;
+        }
+        if (i == (k & 31)) d[p + k] = col[RA];
       }
-      w[t] = y;
+      __syncthreads();
+      const double tv = scal[buf];
+      double vr[NR], vc[NC];
+#pragma unroll
+      for (int a = 0; a < NR; ++a) vr[a] = v[i + 32 * (RA + a)];
+#pragma unroll
+      for (int b = 0; b < NC; ++b) vc[b] = v[c + 16 * (CA + b)];
+      // y(q) = sum_r A(r, q) v(r); rows up to k have v = 0
+      double s[NC];
+#pragma unroll
+      for (int b = 0; b < NC; ++b) {
+        s[b] = 0.0;
+#pragma unroll
+        for (int a = 0; a < NR; ++a) s[b] += x[RA + a][CA + b] * vr[a];
+      }
+      // lanes with bit 4 clear end up with the first half of the columns
+      double pv = 0.0;
+#pragma unroll
+      for (int b = 0; b < NR; ++b) {
+        const double send = up ? s[b] : s[b + NR], keep = up ? s[b + NR] : s[b];
+        const double z = row16_sum(keep + __shfl_xor(send, 16, 64));
+        if ((i & 15) == b) y[c + 16 * (CA + b + (up ? NR : 0))] = z;
+        pv += z * (up ? vc[b + NR] : vc[b]);
+      }
+      pv += __shfl_xor(pv, 16, 64);
+      pv += __shfl_xor(pv, 32, 64);
+      if (lane == 0) part[buf * 8 + wave] = pv;
+      __syncthreads();
+      double ytv = 0.0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) ytv += part[buf * 8 + q];
+      const double f = -0.5 * tv * tv * ytv;
+      double wr[NR], wc[NC];
+#pragma unroll
+      for (int a = 0; a < NR; ++a) wr[a] = tv * y[i + 32 * (RA + a)] + f * vr[a];
+#pragma unroll
+      for (int b = 0; b < NC; ++b) wc[b] = tv * y[c + 16 * (CA + b)] + f * vc[b];
+      // finished rows and columns (up to k) have v = 0 but not w; nothing
+      // reads them again
+#pragma unroll
+      for (int b = 0; b < NC; ++b)
+#pragma unroll
+        for (int a = 0; a < NR; ++a)
+          x[RA + a][CA + b] -= vr[a] * wc[b] + wr[a] * vc[b];
     }
-    const double ytv = block_sum1024(yv, red);
-    if (t < m && t > k) w[t] += -0.5 * tv * ytv * v[t];
-    __syncthreads();
-    for (int q = t; q < m * m; q += 1024) {
-      const int r = q % m, c = q / m;
-      if (r > k && c > k) a[r + c * ld] -= v[r] * w[c] + w[r] * v[c];
-    }
-    __syncthreads();
+    if constexpr (RA + 1 < RB)
+      if (k1 < m - 1) phase<RA + 1>();
   }
-  if (t == 0) {
-    d[n - 1] = a[(m - 1) + (m - 1) * ld];
+};
+
+template <int RB>
+__global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, int n, int p,
+                                                       double* __restrict__ d,
+                                                       double* __restrict__ e,
+                                                       double* __restrict__ tau) {
+  __shared__ double sh[2 * 32 * RB + 2 * 32 * RB + 2 * 8 + 2];
+  TrdTail<RB> q;
+  q.A = A;
+  q.d = d;
+  q.e = e;
+  q.tau = tau;
+  q.vs = sh;
+  q.ys = sh + 64 * RB;
+  q.part = sh + 128 * RB;
+  q.scal = sh + 128 * RB + 16;
+  q.n = n;
+  q.p = p;
+  q.m = n - p;
+  q.lane = threadIdx.x & 63;
+  q.wave = threadIdx.x >> 6;
+  q.i = q.lane & 31;
+  q.c = 2 * q.wave + (q.lane >> 5);
+  q.up = (q.lane & 16) != 0;
+#pragma unroll
+  for (int b = 0; b < 2 * RB; ++b)
+#pragma unroll
+    for (int a = 0; a < RB; ++a) {
+      const int r = q.i + 32 * a, c = q.c + 16 * b;
+      const int hi = r > c ? r : c, lo = r > c ? c : r;
+      q.x[a][b] = hi < q.m ? A[(size_t)(p + hi) + (size_t)(p + lo) * n] : 0.0;
+    }
+  q.template phase<0>();
+  const int l = q.m - 1;
+  if (q.c == (l & 15) && q.i == (l & 31)) {
+    double dl = 0.0;
+#pragma unroll
+    for (int b = 0; b < 2 * RB; ++b)
+      if (b == (l >> 4)) dl = q.x[b / 2][b];
+    d[n - 1] = dl;
     tau[n - 1] = 0.0;
   }
 }
@@ -1124,9 +1215,6 @@ int set_lds_limit(itg_ctx* ctx) {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 8192 * 12));
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_final_sort_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 8192 * 12));
-  ITG_HIP(ctx, hipFuncSetAttribute((const void*)trd_tail_kernel,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (TRD_TAIL * (TRD_TAIL + 1) + 2 * TRD_TAIL) * 8));
   done = true;
   return ITG_OK;
 }
@@ -1161,19 +1249,24 @@ static int tridiagonalize(itg_ctx* ctx, int n, double* A, double* d, double* e, 
   double* Vp = VW;
   double* Wp = VW + (size_t)n * NB;
   double* V2 = VW + 2 * (size_t)n * NB;
-  for (int p = 0; p < n; p += NB) {
+  for (int p = 0, nbp; p < n; p += nbp) {
     if (n - p <= TRD_TAIL) {
       // every earlier panel's update is applied: the rest in one block
-      if (n - p >= 2) {
-        const size_t lds = ((size_t)(n - p) * (n - p + 1) + 2 * (size_t)(n - p)) * sizeof(double);
-        trd_tail_kernel<<<1, 1024, lds, ctx->stream>>>(A, n, p, d, e, tau);
+      const int m = n - p;
+      if (m > 128) {
+        trd_tail_kernel<6><<<1, 512, 0, ctx->stream>>>(A, n, p, d, e, tau);
+      } else if (m > 64) {
+        trd_tail_kernel<4><<<1, 512, 0, ctx->stream>>>(A, n, p, d, e, tau);
+      } else if (m >= 2) {
+        trd_tail_kernel<2><<<1, 512, 0, ctx->stream>>>(A, n, p, d, e, tau);
       } else {
         trd_last_kernel<<<1, 1, 0, ctx->stream>>>(A, n, d, tau);
       }
       ITG_LAUNCH_CHECK(ctx);
       return ITG_OK;
     }
-    int nbp = std::min(NB, n - p);
+    // the last panel stops where the tail kernel can take over
+    nbp = std::min(NB, n - TRD_TAIL - p);
     const int npn = (n + TRD_ROWS - 1) / TRD_ROWS;
     int pn_off = 0, pn_cnt = npn;
     if (p < n - 1) {
@@ -1258,10 +1351,14 @@ static int tridiag_dc(itg_ctx* ctx, int n, const double* d, const double* e, dou
                                   (s_lvl <= DC_ZLDS ? sizeof(double) + sizeof(int) : 0));
     dc_prepare_kernel<<<nm, 1024, lds, ctx->stream>>>(n, s_lvl, half, D, Q, e, bufs);
     ITG_LAUNCH_CHECK(ctx);
-    meta.assign(3 * nm, 0);
-    ITG_HIP(ctx, hipMemcpyAsync(meta.data(), bufs.meta, 3 * nm * sizeof(int), hipMemcpyDeviceToHost,
-                                ctx->stream));
-    ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // the host needs the merges' sizes only to launch their products
+    const bool small = s_lvl <= SMALL_MERGE;
+    if (!small) {
+      meta.assign(3 * nm, 0);
+      ITG_HIP(ctx, hipMemcpyAsync(meta.data(), bufs.meta, 3 * nm * sizeof(int),
+                                  hipMemcpyDeviceToHost, ctx->stream));
+      ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    }
     dim3 g256(nm, (s_lvl + 255) / 256);
     dc_rotate_kernel<<<g256, 256, 0, ctx->stream>>>(n, s_lvl, half, Q, bufs);
     dim3 g4(nm, (s_lvl + 3) / 4);
@@ -1269,7 +1366,6 @@ static int tridiag_dc(itg_ctx* ctx, int n, const double* d, const double* e, dou
     dc_zhat_kernel<<<g4, 256, 0, ctx->stream>>>(n, s_lvl, half, bufs);
     dc_vec_kernel<<<dim3(nm, (s_lvl + 3) / 4), 256, 0, ctx->stream>>>(n, s_lvl, half, Vb, bufs);
     ITG_LAUNCH_CHECK(ctx);
-    bool small = s_lvl <= SMALL_MERGE;
     if (!small) {
       for (int m = 0; m < nm; ++m) {
         int r0 = m * s_lvl, s = std::min(s_lvl, n - r0), k = meta[3 * m];
