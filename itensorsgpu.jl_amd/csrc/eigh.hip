@@ -53,6 +53,79 @@ __device__ double block_sum(double v, double* sh) {
   return r;
 }
 
+// ------------------------------------------------------ lane exchanges
+// On the vector unit (DPP within a row of 16 lanes, permlane swaps between
+// rows): __shfl_xor goes through the LDS pipe, which the CU's waves share.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+
+// lanes with bit MASK (32 or 16) clear: a summed over the pair of lanes that
+// differ in it; the others: b
+template <int MASK>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  if constexpr (MASK == 32) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  } else {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+}
+
+// the value of a lane that differs in bit MASK (8, 4, 2 or 1): for 8 and 4 its
+// mirror image in the row or half row, which differs in the lower bits too
+template <int MASK>
+__device__ __forceinline__ double row_partner(double v) {
+  if constexpr (MASK == 8) return dpp_d<0x140>(v);
+  else if constexpr (MASK == 4) return dpp_d<0x141>(v);
+  else if constexpr (MASK == 2) return dpp_d<0x4E>(v);
+  else return dpp_d<0xB1>(v);
+}
+
+// sum over each row of 16 lanes, the same bits in all of them
+__device__ __forceinline__ double row16_sum(double v) {
+  v += row_partner<1>(v);
+  v += row_partner<2>(v);
+  v += row_partner<4>(v);
+  v += row_partner<8>(v);
+  return v;
+}
+
+// N values per lane -> d[0]: value number lane >> (6 - log2 N) summed over the
+// lanes that differ in the bits used (64 / N lanes are left for each); every
+// step halves the values a lane carries. MASK = 32 to begin with.
+template <int N, int MASK, int M>
+__device__ __forceinline__ void fold_halves(double (&d)[M], int lane) {
+  if constexpr (N > 1) {
+#pragma unroll
+    for (int k = 0; k < N / 2; ++k) {
+      if constexpr (MASK >= 16) {
+        d[k] = swap_add<MASK>(d[k], d[k + N / 2]);
+      } else {
+        const bool up = (lane & MASK) != 0;
+        const double send = up ? d[k] : d[k + N / 2], keep = up ? d[k + N / 2] : d[k];
+        d[k] = keep + row_partner<MASK>(send);
+      }
+    }
+    fold_halves<N / 2, MASK / 2>(d, lane);
+  }
+}
+
+// sum of v over the lanes that differ only in bits MASK, MASK / 2, ..., 1
+template <int MASK>
+__device__ __forceinline__ double fold_sum(double v) {
+  if constexpr (MASK >= 16) v = swap_add<MASK>(v, v);
+  else if constexpr (MASK >= 1) v += row_partner<MASK>(v);
+  if constexpr (MASK > 1) return fold_sum<MASK / 2>(v);
+  else return v;
+}
+
 // ------------------------------------------------------- tridiagonalisation
 // Per column j (panel column i) two kernels run across the whole GPU:
 //  trd_symv: one block per 64 x 64 tile on or below the diagonal of A22
@@ -69,10 +142,8 @@ __device__ double block_sum(double v, double* sh) {
 //    squared tail for the next reflector.
 constexpr int TRD_ROWS = 64;   // rows per block of the row-parallel kernels
 
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+// sum over the wave, the same bits in every lane
+__device__ __forceinline__ double wave_sum(double v) { return fold_sum<32>(v); }
 
 // sum over a 256-thread block, the same value returned to every thread and
 // computed in the same order in every block (bitwise identical results)
@@ -180,46 +251,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void t
       const double vl = vr[lane];
 #pragma unroll
       for (int q = 0; q < 16; ++q) x[q] *= vl;
-      // 16 values -> 8 -> 4 -> 2 -> 1 across lane bits 5, 4, 3, 2
-      {
-        const bool hi = (lane & 32) != 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const double send = hi ? x[k] : x[k + 8];
-          const double keep = hi ? x[k + 8] : x[k];
-          x[k] = keep + __shfl_xor(send, 32, 64);
-        }
-      }
-      {
-        const bool hi = (lane & 16) != 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const double send = hi ? x[k] : x[k + 4];
-          const double keep = hi ? x[k + 4] : x[k];
-          x[k] = keep + __shfl_xor(send, 16, 64);
-        }
-      }
-      {
-        const bool hi = (lane & 8) != 0;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const double send = hi ? x[k] : x[k + 2];
-          const double keep = hi ? x[k + 2] : x[k];
-          x[k] = keep + __shfl_xor(send, 8, 64);
-        }
-      }
-      {
-        const bool hi = (lane & 4) != 0;
-        const double send = hi ? x[0] : x[1];
-        const double keep = hi ? x[1] : x[0];
-        x[0] = keep + __shfl_xor(send, 4, 64);
-      }
-      double z = x[0];
-      z += __shfl_xor(z, 2, 64);
-      z += __shfl_xor(z, 1, 64);
-      const int q = ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 +
-                    ((lane >> 2) & 1);
-      const int c = c0 + wv + 4 * q;
+      fold_halves<16, 32>(x, lane);
+      const double z = fold_sum<2>(x[0]);
+      const int c = c0 + wv + 4 * (lane >> 2);
       if ((lane & 3) == 0 && c < m) Ypart[(size_t)I * m + c] = z;
     }
     __syncthreads();
@@ -429,23 +463,6 @@ __global__ __launch_bounds__(256) void trd_post_kernel(
 // are 144 of a thread's 256 registers; 256 rows would not fit
 constexpr int TRD_TAIL = 192;
 
-// DPP lane exchange of a double within a row of 16 lanes
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-
-// sum over each row of 16 lanes, the same bits in all of them
-__device__ __forceinline__ double row16_sum(double v) {
-  v += dpp_d<0xB1>(v);
-  v += dpp_d<0x4E>(v);
-  v += dpp_d<0x141>(v);
-  v += dpp_d<0x140>(v);
-  return v;
-}
-
 // The trailing block of m = n - p <= 32 RB rows and columns (every earlier
 // update applied, its lower triangle current) reduced to tridiagonal form by
 // one 512-thread workgroup, column by column (dsytd2): y = tau A22 v,
@@ -495,8 +512,7 @@ struct TrdTail {
           if (a == ((k + 1) >> 5)) al = col[a];
         }
         const double alpha = __shfl(al, (lane & 32) | ((k + 1) & 31), 64);
-        s = row16_sum(s);
-        const double xn2 = s + __shfl_xor(s, 16, 64);
+        const double xn2 = fold_sum<16>(s);
         double beta = alpha, tv = 0.0, scale = 1.0;
         if (xn2 != 0.0) {
           beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
@@ -536,13 +552,12 @@ struct TrdTail {
       double pv = 0.0;
 #pragma unroll
       for (int b = 0; b < NR; ++b) {
-        const double send = up ? s[b] : s[b + NR], keep = up ? s[b + NR] : s[b];
-        const double z = row16_sum(keep + __shfl_xor(send, 16, 64));
+        const double z = row16_sum(swap_add<16>(s[b], s[b + NR]));
         if ((i & 15) == b) y[c + 16 * (CA + b + (up ? NR : 0))] = z;
         pv += z * (up ? vc[b + NR] : vc[b]);
       }
-      pv += __shfl_xor(pv, 16, 64);
-      pv += __shfl_xor(pv, 32, 64);
+      pv = swap_add<16>(pv, pv);
+      pv = swap_add<32>(pv, pv);
       if (lane == 0) part[buf * 8 + wave] = pv;
       __syncthreads();
       double ytv = 0.0;
@@ -1685,6 +1700,330 @@ __global__ __launch_bounds__(256) void qr_apply_kernel(double* __restrict__ W, i
   for (int r = j + threadIdx.x; r < m; r += 256) col[r] -= f * (r == j ? 1.0 : v[r]);
 }
 
+// ------------------------------------------ QR of up to 8192 rows (blocked)
+// Panels of QW columns: one workgroup factors the panel in registers, then
+// the columns to the right take its block reflector in two launches.
+constexpr int QW = 16;
+constexpr int QR_MAX_ROWS = 8192;   // 16 rows a thread, 4 columns at a time
+typedef double d4v_t __attribute__((ext_vector_type(4)));
+
+// a double of lane l (wave-uniform l), in scalar registers
+__device__ __forceinline__ double read_lane(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+
+// element (l, c) of the panel's V, unit lower trapezoidal with w columns and
+// m2 rows: the load is unconditional (clamped), so that a loop's loads all go
+// out before any is used
+__device__ __forceinline__ double qr_v(const double* __restrict__ A, int ld, int m2, int w, int l,
+                                       int c) {
+  const double v = A[min(l, m2 - 1) + (size_t)min(c, w - 1) * ld];
+  return (l >= m2 || c >= w || l < c) ? 0.0 : (l == c ? 1.0 : v);
+}
+
+// element (l, c) of C (m2 x nc), zero outside
+__device__ __forceinline__ double qr_c(const double* __restrict__ C, int ld, int m2, int nc, int l,
+                                       int c) {
+  const double v = C[min(l, m2 - 1) + (size_t)min(c, nc - 1) * ld];
+  return (l >= m2 || c >= nc) ? 0.0 : v;
+}
+
+// Y = V^T C (QW x 16) over the 64 rows from b on, for one wave: a lane takes
+// four consecutive rows of one column of each operand and spends them on four
+// products; the 32 loads of the four row blocks go out together
+template <typename F>
+__device__ __forceinline__ d4v_t qr_vt_c(const double* __restrict__ A, int ld, int m2, int w,
+                                         int b, int lr, int lg, d4v_t acc, F&& cel) {
+  double va[4][4], vb[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int l = b + 16 * u + 4 * lg + q;
+      va[u][q] = qr_v(A, ld, m2, w, l, lr);
+      vb[u][q] = cel(l, lr);
+    }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(va[u][q], vb[u][q], acc, 0, 0, 0);
+  return acc;
+}
+
+// Householder QR of the w <= QW columns of A = W(p:, p:) (m2 rows, leading
+// dimension ld), in dgeqrf's layout, and tau. One workgroup; thread t keeps
+// rows t + 512 a of CW columns in registers, the panel's columns in QW / CW
+// turns (a turn first applies the reflectors of the ones before it).
+//
+// Bound: the latency of a column's chain, and one barrier per column: the
+// dot products of column j (rows below j) with every column held come from
+// one reduction (a butterfly that halves the values a lane carries, then
+// eight wave partials in LDS), and everything else follows from them and
+// from row j: |x|^2 is one of them and v^T a_c = a_c(j) + s d_c for
+// v = (1, s x). A lane forms one column's coefficient; the others read it
+// from that lane. The column at hand is always register column 0 (a finished
+// one is stored and the rest move down), so that the steps are loops and not
+// QW copies of the code, which took five times as long, all of it
+// instruction fetch.
+template <int RPT, int CW>
+struct QrPanel {
+  double* A;
+  double* tau;
+  double* ts;                     // LDS: tau
+  double (*red)[8][16];           // LDS [2]: wave partials
+  double (*rowv)[16];             // LDS [2]: row j
+  int ld, m2, w, t, lane, wave, buf;
+  double x[RPT][CW];
+
+  // sum over the workgroup of d[lane % NC], NC = 1 << LOG
+  template <int LOG>
+  __device__ __forceinline__ double reduce(double (&d)[1 << LOG]) {
+    fold_halves<1 << LOG, 32>(d, lane);
+    const double z = fold_sum<(32 >> LOG)>(d[0]);
+    if ((lane & ((64 >> LOG) - 1)) == 0) red[buf][wave][lane >> (6 - LOG)] = z;
+    __syncthreads();
+    double g = 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) g += red[buf][q][lane & ((1 << LOG) - 1)];
+    return g;
+  }
+
+  // columns j0 .. j1 - 1, the 1 << LOG columns from j0 on in x
+  template <int LOG>
+  __device__ __forceinline__ void factor(int j0, int j1) {
+    constexpr int NC = 1 << LOG;
+    for (int j = j0; j < j1; ++j) {
+      double d[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) d[c] = 0.0;
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) {
+        const double xj = (a > 0 || t > j) ? x[a][0] : 0.0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) d[c] += xj * x[a][c];
+      }
+      if (t == j) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) rowv[buf][c] = x[0][c];
+      }
+      const double g = reduce<LOG>(d);
+      const double rv = rowv[buf][lane & (NC - 1)];
+      buf ^= 1;
+      const double alpha = read_lane(rv, 0), xn2 = read_lane(g, 0);
+      // a column whose squares underflow has no direction left: it is dropped
+      double beta = alpha, tj = 0.0, scale = 0.0;
+      if (xn2 >= 0x1p-1010) {
+        beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
+        tj = (beta - alpha) / beta;
+        scale = 1.0 / (alpha - beta);
+      }
+      if (t == 0) {
+        tau[j] = tj;
+        ts[j] = tj;
+      }
+      const double f = tj * (rv + scale * g);
+      double v[RPT];
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) {
+        const bool below = a > 0 || t > j;
+        v[a] = below ? x[a][0] * scale : (t == j ? 1.0 : 0.0);
+        const double s = below ? v[a] : (t == j ? beta : x[a][0]);
+        if (t + 512 * a < m2) A[t + 512 * a + (size_t)j * ld] = s;
+      }
+#pragma unroll
+      for (int c = 1; c < NC; ++c) {
+        const double fc = read_lane(f, c);
+#pragma unroll
+        for (int a = 0; a < RPT; ++a) x[a][c - 1] = x[a][c] - fc * v[a];
+      }
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) x[a][NC - 1] = 0.0;
+    }
+  }
+
+  // the reflector of an earlier column j, applied to the CW columns held
+  template <int LOG>
+  __device__ __forceinline__ void apply(int j) {
+    double v[RPT], d[CW];
+#pragma unroll
+    for (int a = 0; a < RPT; ++a) v[a] = qr_v(A, ld, m2, w, t + 512 * a, j);
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+      d[c] = 0.0;
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) d[c] += v[a] * x[a][c];
+    }
+    const double f = ts[j] * reduce<LOG>(d);
+    buf ^= 1;
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+      const double fc = read_lane(f, c);
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) x[a][c] -= fc * v[a];
+    }
+  }
+};
+
+template <int RPT, int CW>
+__global__ __launch_bounds__(512) void qr_panel_kernel(double* __restrict__ A, int ld, int m2,
+                                                       int w, double* __restrict__ tau) {
+  __shared__ double red[2][8][16], rowv[2][16], ts[QW];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  QrPanel<RPT, CW> q;
+  q.A = A;
+  q.tau = tau;
+  q.ts = ts;
+  q.red = red;
+  q.rowv = rowv;
+  q.ld = ld;
+  q.m2 = m2;
+  q.w = w;
+  q.t = t;
+  q.lane = lane;
+  q.wave = wave;
+  q.buf = 0;
+  for (int c0 = 0; c0 < w; c0 += CW) {
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) q.x[a][c] = qr_c(A, ld, m2, w, t + 512 * a, c0 + c);
+    constexpr int LOG = CW == 16 ? 4 : CW == 8 ? 3 : 2;
+    for (int j = 0; j < c0; ++j) q.template apply<LOG>(j);
+    // the columns in hand halve as they are finished
+    int j = c0;
+    if constexpr (LOG >= 4) {
+      q.template factor<4>(j, min(w, j + 8));
+      j += 8;
+    }
+    if constexpr (LOG >= 3) {
+      if (j < w) q.template factor<3>(j, min(w, j + 4));
+      j += 4;
+    }
+    if (j < w) q.template factor<2>(j, min(w, j + 4));
+    __syncthreads();   // the next turn reads what was stored
+  }
+}
+
+// C <- H^T C (trans) or H C, H = H_0 ... H_{w-1} = I - V T V^T of the panel in
+// A (m2 rows), in two launches over 256 rows x 16 columns per workgroup:
+// partials of Y = V^T C, and of G = V^T V as one more column block; then
+// X = T^T Y or T Y and C -= V X. T is not formed: T^-1 = diag(1 / tau) + the
+// upper triangle of G, so X comes from substitution, x_i = tau_i (y_i -
+// sum_{k<i} G(k, i) x_k) upwards for T^T, from k > i downwards for T. A memory
+// round trip bounds either launch (the matrix is in the Infinity Cache, not
+// in the writer's L2), so a wave's loads all go out together and the grid
+// spans rows as well as columns: one workgroup per 16 columns, walking the
+// rows, took 42 us a panel against 9 + 14 (2000 x 1000).
+constexpr int QR_ROWS = 256;
+
+__global__ __launch_bounds__(256) void qr_y_kernel(const double* __restrict__ A, int ld, int m2,
+                                                   int w, const double* __restrict__ C, int ldc,
+                                                   int nc, double* __restrict__ Yp) {
+  __shared__ double ys[4][QW * 16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int b = (int)blockIdx.y * QR_ROWS + 64 * wave;
+  d4v_t acc = {0.0, 0.0, 0.0, 0.0};
+  if (blockIdx.x + 1 < gridDim.x) {
+    const int cols = min(16, nc - (int)blockIdx.x * 16);
+    C += (size_t)blockIdx.x * 16 * ldc;
+    acc = qr_vt_c(A, ld, m2, w, b, lr, lg, acc,
+                  [&](int l, int c) { return qr_c(C, ldc, m2, cols, l, c); });
+  } else {
+    acc = qr_vt_c(A, ld, m2, w, b, lr, lg, acc,
+                  [&](int l, int c) { return qr_v(A, ld, m2, w, l, c); });
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) ys[wave][(4 * r + lg) + QW * lr] = acc[r];
+  __syncthreads();
+  Yp[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + t] =
+      (ys[0][t] + ys[1][t]) + (ys[2][t] + ys[3][t]);
+}
+
+__global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict__ A, int ld,
+                                                        int m2, int w,
+                                                        const double* __restrict__ tau, int trans,
+                                                        double* __restrict__ C, int ldc, int nc,
+                                                        const double* __restrict__ Yp) {
+  __shared__ double ys[QW * 16], gs[QW * QW], xs[QW * 16], ts[QW];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int cols = min(16, nc - (int)blockIdx.x * 16);
+  C += (size_t)blockIdx.x * 16 * ldc;
+  // this wave's four 16-row blocks: loads and stores run along the rows (the
+  // product is issued transposed)
+  const int b0 = (int)blockIdx.y * QR_ROWS + 64 * wave;
+  double vb[4][4];
+  d4v_t z[4];   // C(l, 4 r + lg)
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      vb[u][q] = qr_v(A, ld, m2, w, b0 + 16 * u + lr, 4 * q + lg);
+      z[u][q] = qr_c(C, ldc, m2, cols, b0 + 16 * u + lr, 4 * q + lg);
+    }
+  if (t < QW) ts[t] = t < w ? tau[t] : 0.0;
+  double y = 0.0, g = 0.0;
+  const size_t nb = gridDim.x + 1;
+  for (int q0 = 0; q0 < (int)gridDim.y; q0 += 8) {
+    double yq[8], gq[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const size_t s = min(q0 + q, (int)gridDim.y - 1);
+      yq[q] = Yp[(s * nb + blockIdx.x) * 256 + t];
+      gq[q] = Yp[(s * nb + gridDim.x) * 256 + t];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (q0 + q < (int)gridDim.y) {
+        y += yq[q];
+        g += gq[q];
+      }
+  }
+  ys[t] = y;
+  gs[t] = g;
+  __syncthreads();
+  if (t < 16) {
+    double x[QW];   // y, less the terms of the x found so far
+#pragma unroll
+    for (int i = 0; i < QW; ++i) x[i] = ys[i + QW * t];
+    if (trans) {
+#pragma unroll
+      for (int i = 0; i < QW; ++i) {
+        x[i] *= ts[i];
+#pragma unroll
+        for (int k = i + 1; k < QW; ++k) x[k] -= gs[i + QW * k] * x[i];
+      }
+    } else {
+#pragma unroll
+      for (int i = QW - 1; i >= 0; --i) {
+        x[i] *= ts[i];
+#pragma unroll
+        for (int k = 0; k < i; ++k) x[k] -= gs[k + QW * i] * x[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < QW; ++i) xs[i + QW * t] = -x[i];
+  }
+  __syncthreads();
+  double xa[4];   // -X(4 q + lg, lr), the left operand X^T(column, k)
+#pragma unroll
+  for (int q = 0; q < 4; ++q) xa[q] = xs[(4 * q + lg) + QW * lr];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int l = b0 + 16 * u + lr;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      z[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[q], vb[u][q], z[u], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (l < m2 && 4 * r + lg < cols) C[l + (size_t)(4 * r + lg) * ldc] = z[u][r];
+  }
+}
+
 __global__ void qr_init_q_kernel(int m, int r, double* __restrict__ Q) {
   int64_t tot = (int64_t)m * r;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot;
@@ -1892,6 +2231,50 @@ __global__ void transpose_kernel(int m, int n, const double* __restrict__ A, dou
 
 }  // namespace
 
+// doubles of the partials of V^T C (nc columns) and V^T V
+static size_t qr_yp_doubles(int m, int nc) {
+  return (size_t)((m + QR_ROWS - 1) / QR_ROWS) * ((nc + 15) / 16 + 1) * 256;
+}
+
+static int qr_block_apply(itg_ctx* ctx, const double* A, int ld, int m2, int w, const double* tau,
+                          int trans, double* C, int ldc, int nc, double* Yp) {
+  const unsigned nb = (nc + 15) / 16, ns = (m2 + QR_ROWS - 1) / QR_ROWS;
+  qr_y_kernel<<<dim3(nb + 1, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, C, ldc, nc, Yp);
+  qr_update_kernel<<<dim3(nb, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, tau, trans, C, ldc, nc,
+                                                          Yp);
+  ITG_LAUNCH_CHECK(ctx);
+  return ITG_OK;
+}
+
+// W (m x n, m <= QR_MAX_ROWS) <- its QR in dgeqrf's layout and Q (m x r,
+// column-major) formed; Yp holds qr_yp_doubles(m, n)
+static int qr_blocked(itg_ctx* ctx, int m, int n, double* W, double* Q, double* tau, double* Yp) {
+  const int r = std::min(m, n);
+  for (int p = 0; p < r; p += QW) {
+    const int w = std::min(QW, r - p), m2 = m - p, nt = n - p - w;
+    double* A = W + (size_t)p * m + p;
+    hipStream_t st = ctx->stream;
+    // rows a thread x columns a turn: at most 64 doubles of the panel
+    if (m2 <= 1024) qr_panel_kernel<2, 16><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
+    else if (m2 <= 2048) qr_panel_kernel<4, 16><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
+    else if (m2 <= 4096) qr_panel_kernel<8, 8><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
+    else qr_panel_kernel<16, 4><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
+    ITG_LAUNCH_CHECK(ctx);
+    if (nt <= 0) continue;
+    int rc = qr_block_apply(ctx, A, m, m2, w, tau + p, 1, A + (size_t)w * m, m, nt, Yp);
+    if (rc) return rc;
+  }
+  qr_init_q_kernel<<<itg_blocks((int64_t)m * r, 256, 8192), 256, 0, ctx->stream>>>(m, r, Q);
+  ITG_LAUNCH_CHECK(ctx);
+  for (int p = (r - 1) / QW * QW; p >= 0; p -= QW) {
+    // columns before p are still those of the identity
+    int rc = qr_block_apply(ctx, W + (size_t)p * m + p, m, m - p, std::min(QW, r - p), tau + p, 0,
+                            Q + (size_t)p * m + p, m, r - p, Yp);
+    if (rc) return rc;
+  }
+  return ITG_OK;
+}
+
 extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const void* Ain, void* Qo,
                       void* Ro) {
   ITG_CHECK_CTX(ctx);
@@ -1903,7 +2286,7 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   int m = (int)m64, n = (int)n64, r = std::min(m, n);
   bool f32 = dtype == ITG_F32;
   size_t bytes = ((size_t)m * n + (size_t)m * r + (size_t)r * n + (size_t)m * NB + 2 * (size_t)NB * n +
-                  2 * NB * NB + (size_t)r + 64) * sizeof(double) + 16 * 256;
+                  2 * NB * NB + (size_t)r + (m <= QR_MAX_ROWS ? qr_yp_doubles(m, n) : 0) + 64) * sizeof(double) + 16 * 256;
   void* ws;
   int rc = eig_workspace(ctx, bytes, &ws);
   if (rc) return rc;
@@ -1919,7 +2302,16 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   double* tau = cv.take<double>(r);
   rc = itg_convert(ctx, (int64_t)m * n, dtype, Ain, ITG_F64, W);
   if (rc) return rc;
-  // blocked Householder QR (dgeqrf): each panel of NB columns is factored
+  if (m <= QR_MAX_ROWS) {
+    rc = qr_blocked(ctx, m, n, W, Q, tau, cv.take<double>(qr_yp_doubles(m, n)));
+    if (rc) return rc;
+    qr_extract_r_kernel<<<itg_blocks((int64_t)r * n, 256, 8192), 256, 0, ctx->stream>>>(m, n, r, W, R);
+    ITG_LAUNCH_CHECK(ctx);
+    rc = itg_convert(ctx, (int64_t)m * r, ITG_F64, Q, dtype, Qo);
+    if (rc) return rc;
+    return itg_convert(ctx, (int64_t)r * n, ITG_F64, R, dtype, Ro);
+  }
+  // taller matrices: blocked Householder QR (dgeqrf): each panel of NB columns is factored
   // column by column within itself, then the trailing columns take the
   // panel's block reflector, W2 -= V T^T (V^T W2), as GEMMs
   for (int p = 0; p < r; p += NB) {
