@@ -815,22 +815,14 @@ __global__ __launch_bounds__(256) void bt_group_solve_kernel(int nbg, int k,
 }
 
 // --------------------------------------------------------- divide & conquer
-// Q = I and Qn = 0: every merge rewrites whole block squares, and entries
+// Q = Qn = 0: the leaves and every merge write whole block squares, and entries
 // outside the current squares of both ping-pong buffers must stay zero
-__global__ void dc_init_kernel(int n, const double* d, const double* e, double* D, double* Q,
-                               double* Qn) {
+__global__ void dc_init_kernel(int n, double* Q, double* Qn) {
   int64_t tot = (int64_t)n * n;
   for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < tot;
        x += (int64_t)gridDim.x * blockDim.x) {
-    int r = (int)(x % n), c = (int)(x / n);
-    Q[x] = (r == c) ? 1.0 : 0.0;
+    Q[x] = 0.0;
     Qn[x] = 0.0;
-    if (r == 0) {
-      double v = d[c];
-      if (c > 0) v -= fabs(e[c - 1]);
-      if (c < n - 1) v -= fabs(e[c]);
-      D[c] = v;
-    }
   }
 }
 
@@ -1100,6 +1092,325 @@ __global__ __launch_bounds__(256) void dc_zhat_kernel(int n, int s_lvl, int half
   }
 }
 
+// --------------------------------------------- the first levels in one launch
+// Rows [DC_LEAF b, ...) of the tridiagonal from 1 x 1 blocks to one block of
+// at most DC_LEAF, everything in LDS, one workgroup per leaf. A level costs
+// six launches when it runs on the whole matrix, whatever its size (60 us a
+// level up to 64); here it costs six barriers, 96 us for the six levels
+// against 370. Four lanes per root, per entry of zhat and per eigenvector; the
+// merges' deflation passes by one wave together; their products on MFMA with
+// the deflated columns as unit columns of V (blocks below 16 padded with
+// zeros).
+constexpr int DC_LEAF = 64;
+
+struct DcLeaf {
+  static constexpr int LD = DC_LEAF + 1;
+  double Q[2][DC_LEAF * LD], V[DC_LEAF * LD];
+  double D[2][DC_LEAF], ds[DC_LEAF], zs[DC_LEAF], dl[DC_LEAF], w[DC_LEAF], dval[DC_LEAF];
+  double tau[DC_LEAF], zh[DC_LEAF], rcs[2 * DC_LEAF], rho[DC_LEAF], w2[DC_LEAF];
+  int col[DC_LEAF], src[DC_LEAF], org[DC_LEAF], rcol[2 * DC_LEAF];
+  int k[DC_LEAF], nrot[DC_LEAF];   // of the merge that starts at this row
+};
+
+// sum over the four lanes of a quad, the same bits in each
+__device__ __forceinline__ double quad_sum(double v) {
+  v += row_partner<1>(v);
+  v += row_partner<2>(v);
+  return v;
+}
+
+// The deflation pass of every merge of a level (aligned groups of s rows, s
+// <= 64) by one wave, lane = sorted position. The rules are dc_deflate's: an
+// entry with a negligible z is dropped, and consecutive kept entries that
+// nearly coincide are rotated into one, which carries N = sum d z^2 and
+// Z2 = sum z^2 of its run. Tests of neighbours with their own values find
+// where a run starts; sums from that start on (a scan) give every later test
+// of the run at once, and the first that fails ends it. One turn of the loop
+// per run of two or more, against one step per entry (22 us for 64).
+__device__ __forceinline__ void dc_leaf_deflate(DcLeaf& L, int lane, int s, int half, int nl) {
+  const int r0 = lane / s * s, sm = min(s, nl - r0);
+  const bool in = sm > half && lane < nl;
+  const unsigned long long seg = (s == 64 ? ~0ull : ((1ull << s) - 1)) << r0;
+  const unsigned long long below = (1ull << lane) - 1;
+  const double d = in ? L.ds[lane] : 0.0, z = in ? L.zs[lane] : 0.0;
+  const double rho = in ? L.rho[r0] : 0.0;
+  double dm = fabs(d), zm = fabs(z);
+  for (int o = 1; o < s; o <<= 1) {
+    dm = fmax(dm, __shfl_xor(dm, o, 64));
+    zm = fmax(zm, __shfl_xor(zm, o, 64));
+  }
+  const double tol = 8.0 * ITG_DC_EPS * fmax(dm, zm), tol2 = tol * tol;
+  const bool kept = in && rho * fabs(z) > tol;
+  const unsigned long long km = __ballot(kept) & seg;
+  const double z2 = z * z;
+  // the kept entry before this one (its lane; -1: none)
+  const int pv = (km & below) ? 63 - __clzll(km & below) : -1;
+  const double dp0 = __shfl(d, pv < 0 ? lane : pv, 64), zp0 = __shfl(z, pv < 0 ? lane : pv, 64);
+  auto close = [&](double N, double Z2) {
+    const double T2 = Z2 + z2, x = d * Z2 - N;
+    return x * x * z2 <= tol2 * Z2 * T2 * T2;
+  };
+  const bool pair = kept && pv >= 0 && close(dp0 * (zp0 * zp0), zp0 * zp0);
+  const unsigned long long pm = __ballot(pair) & seg;
+  unsigned long long rot = 0;     // entries rotated onto (this group's)
+  double N = d * z2, Z2 = z2;     // sums of the run up to this entry
+  double Np = 0.0, Zp = 0.0;      // and before it
+  int cur = r0;                   // entries up to here are settled
+  while (true) {
+    const unsigned long long m = cur >= 64 ? 0 : pm & (~0ull << cur) & ~(1ull << cur);
+    // a start needs its predecessor at or after cur, which holds for any
+    // kept entry after cur (cur itself is kept once a run has ended there)
+    if (!__any(m != 0)) break;
+    const bool have = m != 0;
+    const int j0 = have ? __ffsll(m) - 1 : 0;
+    const int s0 = have ? 63 - __clzll(km & ((1ull << j0) - 1)) : 0;
+    double sn = have && kept && lane >= s0 ? d * z2 : 0.0;
+    double sz = have && kept && lane >= s0 ? z2 : 0.0;
+    for (int o = 1; o < s; o <<= 1) {
+      const double un = __shfl_up(sn, o, 64), uz = __shfl_up(sz, o, 64);
+      if (lane - r0 >= o) {
+        sn += un;
+        sz += uz;
+      }
+    }
+    // the sums before this entry: those of the kept entry before it
+    const double en = __shfl(sn, pv < 0 ? lane : pv, 64), ez = __shfl(sz, pv < 0 ? lane : pv, 64);
+    const bool fail = have && kept && lane > s0 && !close(en, ez);
+    const unsigned long long fm = __ballot(fail) & seg;
+    if (have) {
+      const int jf = fm ? __ffsll(fm) - 1 : r0 + s;   // first entry past the run
+      const unsigned long long upto = jf >= 64 ? ~0ull : (1ull << jf) - 1;
+      rot |= km & upto & ~((2ull << s0) - 1);
+      if (kept && lane > s0 && lane < jf) {
+        N = sn;
+        Z2 = sz;
+        Np = en;
+        Zp = ez;
+      }
+      cur = jf;
+    }
+  }
+  const bool myrot = (rot >> lane) & 1;
+  // a kept entry survives unless the next kept one is rotated onto
+  const unsigned long long later = km & ~below & ~(1ull << lane);
+  const int nx = later ? __ffsll(later) - 1 : 64;
+  const bool out = kept && !(nx < 64 && ((rot >> nx) & 1));
+  const unsigned long long om = __ballot(out) & seg;
+  const bool drop = in && !kept;
+  const unsigned long long dm2 = __ballot(drop || myrot) & seg;
+  const int col = in ? L.col[lane] : lane;
+  const int pcol = __shfl(col, pv < 0 ? lane : pv, 64);
+  const bool psingle = pv >= 0 && !((rot >> pv) & 1);   // a run of one before this entry
+  const int k = __popcll(om);
+  if (out) {
+    const int q = r0 + __popcll(om & below);
+    L.dl[q] = myrot ? N / Z2 : d;
+    L.w[q] = myrot ? sqrt(Z2) : z;
+    L.src[q] = col;
+  }
+  if (drop || myrot) {
+    const int q = __popcll(dm2 & below);
+    double v = d;
+    if (myrot) {
+      const double it = 1.0 / sqrt(Zp + z2);
+      const double c = z * it, sg = -(psingle ? zp0 : sqrt(Zp)) * it;
+      const double dp = psingle ? dp0 : Np / Zp;
+      const int x = r0 + __popcll(rot & below);
+      L.rcol[2 * x] = pcol;
+      L.rcol[2 * x + 1] = col;
+      L.rcs[2 * x] = c;
+      L.rcs[2 * x + 1] = sg;
+      v = dp * c * c + d * sg * sg;
+    }
+    L.dval[r0 + q] = v;
+    L.src[r0 + k + q] = myrot ? pcol : col;
+  }
+  double w2 = out ? Z2 : 0.0;
+  for (int o = 1; o < s; o <<= 1) w2 += __shfl_xor(w2, o, 64);
+  if (in && lane == r0) {
+    L.k[r0] = k;
+    L.nrot[r0] = __popcll(rot);
+    L.w2[r0] = w2;
+  }
+}
+
+__global__ __launch_bounds__(256) void dc_leaf_kernel(int n, const double* __restrict__ d,
+                                                      const double* __restrict__ e,
+                                                      double* __restrict__ Qg,
+                                                      double* __restrict__ Dg) {
+  extern __shared__ __attribute__((aligned(16))) char dc_leaf_lds[];
+  DcLeaf& L = *(DcLeaf*)dc_leaf_lds;
+  constexpr int LD = DcLeaf::LD;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int r00 = blockIdx.x * DC_LEAF, nl = min(DC_LEAF, n - r00);
+  const int g = t >> 2, q4 = t & 3;   // row / root / column of four lanes
+  for (int x = t; x < DC_LEAF * LD; x += 256) {
+    L.Q[0][x] = x % LD == x / LD ? 1.0 : 0.0;
+    L.Q[1][x] = 0.0;
+  }
+  if (t < DC_LEAF) {
+    double v = 0.0;
+    const int c = r00 + t;
+    if (t < nl) {
+      v = d[c];
+      if (c > 0) v -= fabs(e[c - 1]);
+      if (c < n - 1) v -= fabs(e[c]);
+    }
+    L.D[0][t] = v;
+  }
+  __syncthreads();
+  int cur = 0;
+  for (int half = 1; half < nl; half *= 2, cur ^= 1) {
+    const int s = 2 * half;
+    const int r0 = g / s * s, sm = min(s, nl - r0);   // this row's merge
+    const bool act = sm > half;
+    const int i = g - r0;
+    double* Q = L.Q[cur];
+    double* D = L.D[cur];
+    // z and the position in the merge's ascending order
+    if (act && g < nl) {
+      int before = 0;
+      const double dg = D[g];
+      for (int c = q4; c < sm; c += 4) {
+        const double dc = D[r0 + c];
+        before += (dc < dg || (dc == dg && c < i)) ? 1 : 0;
+      }
+      before += __builtin_amdgcn_mov_dpp(before, 0xB1, 0xF, 0xF, false);
+      before += __builtin_amdgcn_mov_dpp(before, 0x4E, 0xF, 0xF, false);
+      if (q4 == 0) {
+        const double beta = e[r00 + r0 + half - 1];
+        const double sg = beta >= 0.0 ? 1.0 : -1.0;
+        const double z = i < half ? Q[g * LD + r0 + half - 1] : sg * Q[g * LD + r0 + half];
+        L.ds[r0 + before] = dg;
+        L.zs[r0 + before] = z * 0.7071067811865476;
+        L.col[r0 + before] = g;
+        if (i == 0) L.rho[r0] = 2.0 * fabs(beta);
+      }
+    }
+    __syncthreads();
+    if (wave == 0) dc_leaf_deflate(L, lane, s, half, nl);
+    __syncthreads();
+    const int k = act ? L.k[r0] : 0;
+    if (t < nl) {
+      // the deflation's rotations, thread = row of Q
+      const int b0 = t / s * s;
+      if (min(s, nl - b0) > half) {
+        const int nr = L.nrot[b0];
+        for (int x = 0; x < nr; ++x) {
+          const int pc = L.rcol[2 * b0 + 2 * x], qc = L.rcol[2 * b0 + 2 * x + 1];
+          const double c = L.rcs[2 * b0 + 2 * x], sn = L.rcs[2 * b0 + 2 * x + 1];
+          const double u = Q[pc * LD + t], v = Q[qc * LD + t];
+          Q[pc * LD + t] = c * u + sn * v;
+          Q[qc * LD + t] = c * v - sn * u;
+        }
+      }
+    }
+    const double* dl = L.dl + r0;
+    const double* w = L.w + r0;
+    if (act && i < k) {
+      const double rho = L.rho[r0];
+      auto ev = [&](int o, double tau, int side, double* dpo, double* dpf, double* absum) {
+        double f = 0.0, po = 0.0, pf = 0.0, ab = 0.0;
+        const double dlo = dl[o];
+#pragma unroll 4
+        for (int j = q4; j < k; j += 4) {
+          const double del = (dl[j] - dlo) - tau;
+          const double u = w[j] / del;
+          const double term = rho * w[j] * u;
+          f += term;
+          ab += fabs(term);
+          const double dt = rho * u * u;
+          const bool origin_side = side > 0 ? (j <= o) : (j >= o);
+          if (origin_side) po += dt; else pf += dt;
+        }
+        *dpo = quad_sum(po);
+        *dpf = quad_sum(pf);
+        *absum = 1.0 + quad_sum(ab);
+        return 1.0 + quad_sum(f);
+      };
+      int o;
+      double tv;
+      dc_secular_root_with(i, k, dl, rho, L.w2[r0], ev, &o, &tv);
+      if (q4 == 0) {
+        L.org[g] = o;
+        L.tau[g] = tv;
+      }
+    }
+    __syncthreads();
+    const int* org = L.org + r0;
+    const double* tau = L.tau + r0;
+    if (act && i < k) {
+      // zhat_i (Gu-Eisenstat, as dc_zhat)
+      const double dli = dl[i];
+      double p = 1.0;
+#pragma unroll 4
+      for (int j = q4; j < k; j += 4)
+        if (j != i) p *= ((dli - dl[org[j]]) - tau[j]) / (dli - dl[j]);
+      p *= row_partner<1>(p);
+      p *= row_partner<2>(p);
+      p *= (dli - dl[org[i]]) - tau[i];
+      if (q4 == 0) L.zh[g] = copysign(sqrt(p < 0.0 ? -p : 0.0), w[i]);
+    }
+    __syncthreads();
+    {
+      // column g of V: an eigenvector of the rank-one update, or a unit
+      // column (deflated, or a block without a sibling at this level)
+      const int S = s < 16 ? 16 : s, b0 = g / S * S;
+      double lamo = 0.0, tj = 0.0, inv = 0.0;
+      const bool root = act && g < nl && i < k;
+      if (root) {
+        lamo = dl[org[i]];
+        tj = tau[i];
+        double s2 = 0.0;
+#pragma unroll 4
+        for (int j = q4; j < k; j += 4) {
+          const double v = L.zh[r0 + j] / ((dl[j] - lamo) - tj);
+          s2 += v * v;
+        }
+        inv = 1.0 / sqrt(quad_sum(s2));
+      }
+#pragma unroll 4
+      for (int x = b0 + q4; x < b0 + S; x += 4) {
+        const int j = x - r0;
+        double v;
+        if (root) v = j >= 0 && j < k ? L.zh[x] / ((dl[j] - lamo) - tj) * inv : 0.0;
+        else v = x == g ? 1.0 : 0.0;
+        L.V[g * LD + x] = v;
+      }
+      if (q4 == 0) {
+        L.D[cur ^ 1][g] = root ? lamo + tj : act && g < nl ? L.dval[r0 + i - k] : D[g];
+        if (!act || g >= nl) L.src[g] = g;
+      }
+    }
+    __syncthreads();
+    {
+      // Q' = Q(:, src) V, blocks of S on the diagonal
+      const int S = s < 16 ? 16 : s, ts = S / 16;
+      const int lr = lane & 15, lg = lane >> 4;
+      for (int tile = wave; tile < DC_LEAF / S * ts * ts; tile += 4) {
+        const int b0 = tile / (ts * ts) * S, in = tile % (ts * ts);
+        const int row = b0 + in % ts * 16, cj = b0 + in / ts * 16;
+        typedef double d4 __attribute__((ext_vector_type(4)));
+        d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int x = b0; x < b0 + S; x += 4) {
+          const double a = Q[L.src[x + lg] * LD + row + lr];
+          const double b = L.V[(cj + lr) * LD + x + lg];
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) L.Q[cur ^ 1][(cj + lr) * LD + row + 4 * r + lg] = acc[r];
+      }
+    }
+    __syncthreads();
+  }
+  for (int x = t; x < nl * nl; x += 256) {
+    const int r = x % nl, c = x / nl;
+    Qg[(size_t)(r00 + c) * n + r00 + r] = L.Q[cur][c * LD + r];
+  }
+  if (t < nl) Dg[r00 + t] = L.D[cur][t];
+}
+
 // column j of the rank-one eigenvector matrix, normalised (one wave per column)
 __global__ __launch_bounds__(256) void dc_vec_kernel(int n, int s_lvl, int half, double* __restrict__ Vb,
                                                      DcBufs b) {
@@ -1228,6 +1539,8 @@ int set_lds_limit(itg_ctx* ctx) {
   if (done) return ITG_OK;
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_prepare_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 8192 * 12));
+  ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_leaf_kernel,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(DcLeaf)));
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_final_sort_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 8192 * 12));
   done = true;
@@ -1355,11 +1668,12 @@ static int tridiag_dc(itg_ctx* ctx, int n, const double* d, const double* e, dou
                       double* Qb, double* Da, double* Db, double* Vb, DcBufs bufs, int64_t* tab,
                       double** Qout, double** Dout, GettArgs* top) {
   if (top) top->M = 0;
-  dc_init_kernel<<<itg_blocks((int64_t)n * n, 256, 16384), 256, 0, ctx->stream>>>(n, d, e, Da, Qa, Qb);
+  dc_init_kernel<<<itg_blocks((int64_t)n * n, 256, 16384), 256, 0, ctx->stream>>>(n, Qa, Qb);
+  dc_leaf_kernel<<<(n + DC_LEAF - 1) / DC_LEAF, 256, sizeof(DcLeaf), ctx->stream>>>(n, d, e, Qa, Da);
   ITG_LAUNCH_CHECK(ctx);
   double *Q = Qa, *Qn = Qb, *D = Da, *Dn = Db;
   std::vector<int> meta;
-  for (int half = 1; half < n; half *= 2) {
+  for (int half = DC_LEAF; half < n; half *= 2) {
     int s_lvl = 2 * half;
     int nm = (n + s_lvl - 1) / s_lvl;
     size_t lds = (size_t)s_lvl * (sizeof(double) + sizeof(int) +
