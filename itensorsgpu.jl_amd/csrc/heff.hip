@@ -15,6 +15,7 @@
 // split-operand GEMM (bf16x3.hip).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "bf16x3.h"
@@ -40,43 +41,10 @@ __global__ void heff_x_kernel(int64_t WL, int64_t WM, int64_t WR, int64_t d, con
   }
 }
 
-// one block: 64 consecutive a' for one b; tile T1(a', q) staged in LDS
-template <typename T>
-__global__ __launch_bounds__(256) void heff_wpass_kernel(int64_t chiL, int64_t Q, int64_t O,
-                                                         const T* __restrict__ T1,
-                                                         const double* __restrict__ X,
-                                                         T* __restrict__ T3) {
-  extern __shared__ double sh[];
-  double* tile = sh;            // [Q][64]
-  double* xs = sh + Q * 64;     // [Q][O]
-  int64_t tiles_a = (chiL + 63) / 64;
-  int64_t b = blockIdx.x / tiles_a;
-  int64_t a0 = (blockIdx.x % tiles_a) * 64;
-  int t = threadIdx.x;
-  for (int64_t e = t; e < Q * O; e += 256) xs[e] = X[e];
-  const T* src = T1 + Q * chiL * b;
-  for (int64_t e = t; e < Q * 64; e += 256) {
-    int64_t q = e / 64, al = e % 64;
-    int64_t a = a0 + al;
-    tile[e] = a < chiL ? (double)src[a + chiL * q] : 0.0;
-  }
-  __syncthreads();
-  int al = t & 63, part = t >> 6;
-  int64_t a = a0 + al;
-  if (a < chiL) {
-    T* dst = T3 + O * chiL * b;
-    for (int64_t o = part; o < O; o += 4) {
-      double acc = 0.0;
-      for (int64_t q = 0; q < Q; ++q) acc += tile[q * 64 + al] * xs[q + Q * o];
-      dst[a + chiL * o] = (T)acc;
-    }
-  }
-}
-
-// The same pass for fixed Q x O (the chain's w = 5, d = 2: 20 x 20): one
-// thread per row a' for WPASS_B consecutive b, T1(a', q, b) loaded and
-// T3(a', o, b) stored along a' (256 consecutive rows per block), X read from
-// LDS by broadcast. The sum over q runs in the order of heff_wpass_kernel.
+// The W pass for fixed Q x O (the chain's w = 5, d = 2: 20 x 20) at large chi,
+// where HBM bounds it: one thread per row a' for WPASS_B consecutive b,
+// T1(a', q, b) loaded and T3(a', o, b) stored along a' (256 consecutive rows
+// per block), X read from LDS by broadcast, the sum over q in order.
 constexpr int WPASS_B = 4;
 
 template <typename T, int QC, int OC>
@@ -107,6 +75,127 @@ __global__ __launch_bounds__(256) void heff_wpass_fixed_kernel(int64_t chiL, int
       for (int q = 0; q < QC; ++q) acc += t[q] * xs[q + QC * o];
       dst[chiL * o] = (T)acc;
     }
+  }
+}
+
+// The pass on FP64 MFMA for any Q x O: one wave per 16 AT rows a' of one b,
+// issued as X^T (o x q) times T1^T (q x a'), so that loads of T1 and stores of
+// T3 run along a'. X sits in LDS, zero padded to whole products (rows of the
+// four lane groups offset by half the banks); O outputs of the Oall are
+// formed (X and T3 start at the first). Latency bounds it at small chi
+// and L2 traffic at large; before it a block staged 64 rows of T1 in LDS and
+// one thread summed an output at a time. Measured (us, before -> now):
+//   Q = O = 56, 300 x 277 FP64: 84 -> 28; 500 x 500 FP32: 187 -> 54
+//   Q = O = 45, 300 x 300 FP64: 56 -> 25; Q = O = 20, 20 x 20 FP64: 20 -> 8
+typedef double d4w_t __attribute__((ext_vector_type(4)));
+
+__host__ __device__ constexpr int wpass_ldo(int O) {
+  return ((O + 15) / 16 * 16) % 32 == 0 ? (O + 15) / 16 * 16 + 16 : (O + 15) / 16 * 16;
+}
+
+template <typename T, int NT, int AT>
+__global__ __launch_bounds__(256) void heff_wpass_mfma_kernel(int chiL, int chiR, int Q,
+                                                              int64_t Oall, int O,
+                                                              const T* __restrict__ T1,
+                                                              const double* __restrict__ X,
+                                                              T* __restrict__ T3) {
+  extern __shared__ double xs[];
+  const int t = threadIdx.x, lane = t & 63, lr = lane & 15, lg = lane >> 4;
+  const int kt = (Q + 3) / 4, ldo = wpass_ldo(O), ot = (O + 15) / 16;
+  for (int e = t; e < 4 * kt * ldo; e += 256) {
+    const int q = e / ldo, o = e % ldo;
+    xs[e] = q < Q && o < O ? X[q + Q * o] : 0.0;
+  }
+  __syncthreads();
+  constexpr int KC = 8 / AT;   // k steps whose loads go out together
+  const int ta = (chiL + 16 * AT - 1) / (16 * AT);
+  const int64_t units = (int64_t)ta * chiR;
+  for (int64_t u = (int64_t)blockIdx.x * 4 + (t >> 6); u < units; u += (int64_t)gridDim.x * 4) {
+    const int a0 = (int)(u % ta) * 16 * AT + lr;
+    const int64_t b = u / ta;
+    const T* src[AT];
+#pragma unroll
+    for (int s = 0; s < AT; ++s)
+      src[s] = T1 + (int64_t)Q * chiL * b + (a0 + 16 * s < chiL ? a0 + 16 * s : chiL - 1);
+    T* dst = T3 + Oall * chiL * b + a0;
+    for (int o0 = 0; o0 < ot; o0 += NT) {
+      d4w_t acc[AT][NT];
+#pragma unroll
+      for (int s = 0; s < AT; ++s)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[s][j] = d4w_t{0.0, 0.0, 0.0, 0.0};
+      for (int k0 = 0; k0 < kt; k0 += KC) {
+        T v[KC][AT];
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+          const int q = 4 * (k0 + i) + lg;
+#pragma unroll
+          for (int s = 0; s < AT; ++s)
+            v[i][s] = src[s][(int64_t)chiL * (q < Q ? q : Q - 1)];   // X is zero past Q
+        }
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+          if (k0 + i >= kt) break;
+          const double* x = xs + (4 * (k0 + i) + lg) * ldo + 16 * o0 + lr;
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            const double xj = x[16 * j];
+#pragma unroll
+            for (int s = 0; s < AT; ++s)
+              acc[s][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(xj, (double)v[i][s], acc[s][j], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int o = 16 * (o0 + j) + 4 * r + lg;
+#pragma unroll
+          for (int s = 0; s < AT; ++s)
+            if (o < O && a0 + 16 * s < chiL) dst[(int64_t)chiL * o + 16 * s] = (T)acc[s][j][r];
+        }
+    }
+  }
+}
+
+template <typename T>
+static void wpass(itg_ctx* ctx, int64_t chiL, int64_t chiR, int64_t Q, int64_t O, const T* T1,
+                  const double* X, T* T3) {
+  // 20 x 20 beyond the caches: whole rows of 256 reach HBM's rate (2048^2
+  // FP32: 145 us, 4.6 TB/s), 32-row pieces do not (211 us); below 800 x 800
+  // the MFMA form is faster (700^2 FP32: 26.5 against 28.9, 200^2: 11 against 22)
+  if (Q == 20 && O == 20 && chiL * chiR >= 800 * 800) {
+    const int64_t fb = ((chiL + 255) / 256) * ((chiR + WPASS_B - 1) / WPASS_B);
+    heff_wpass_fixed_kernel<T, 20, 20><<<(unsigned)fb, 256, 0, ctx->stream>>>(chiL, chiR, T1, X,
+                                                                              T3);
+    return;
+  }
+  // outputs per launch: as many as X has room for in 64 KB of LDS (all of
+  // them but for an MPO of thousands of channels and d = 1)
+  const int64_t rows = (Q + 3) / 4 * 4;
+  int64_t os = O;
+  while (rows * wpass_ldo((int)os) * 8 > 65536) os = (os / 2 + 15) / 16 * 16;
+  const size_t lds = (size_t)rows * wpass_ldo((int)os) * sizeof(double);
+  const int nt = (O + 15) / 16 <= 1 ? 1 : (O + 15) / 16 == 2 ? 2 : 4;
+  // two row tiles a wave once there are enough of them
+  const int at = chiL >= 200 ? 2 : 1;
+  const int64_t units = (chiL + 16 * at - 1) / (16 * at) * chiR;
+  const unsigned nb =
+      (unsigned)std::min<int64_t>((units + 3) / 4, 4 * (int64_t)std::max(ctx->num_cu, 1));
+  auto go = [&](auto kernel) {
+    for (int64_t o = 0; o < O; o += os)
+      kernel<<<nb, 256, lds, ctx->stream>>>((int)chiL, (int)chiR, (int)Q, O,
+                                            (int)std::min(os, O - o), T1, X + Q * o, T3 + chiL * o);
+  };
+  if (at == 2) {
+    if (nt == 1) go(heff_wpass_mfma_kernel<T, 1, 2>);
+    else if (nt == 2) go(heff_wpass_mfma_kernel<T, 2, 2>);
+    else go(heff_wpass_mfma_kernel<T, 4, 2>);
+  } else {
+    if (nt == 1) go(heff_wpass_mfma_kernel<T, 1, 1>);
+    else if (nt == 2) go(heff_wpass_mfma_kernel<T, 2, 1>);
+    else go(heff_wpass_mfma_kernel<T, 4, 1>);
   }
 }
 
@@ -256,24 +345,11 @@ int apply(itg_ctx* ctx, int dtype, int mode, const HeffDims& h, const void* L, c
   }
   if (rc) return rc;
   // C23: W pass
-  int64_t blocks = ((h.chiL + 63) / 64) * h.chiR;
-  size_t lds = (size_t)(h.Q * 64 + h.Q * h.O) * sizeof(double);
   int tk = itg_tstart(ctx, ITG_K_WPASS);
-  if (h.Q == 20 && h.O == 20) {
-    const int64_t fb = ((h.chiL + 255) / 256) * ((h.chiR + WPASS_B - 1) / WPASS_B);
-    if (idt == ITG_F64)
-      heff_wpass_fixed_kernel<double, 20, 20><<<(unsigned)fb, 256, 0, ctx->stream>>>(
-          h.chiL, h.chiR, (const double*)w.T1, P.X, (double*)w.T3);
-    else
-      heff_wpass_fixed_kernel<float, 20, 20><<<(unsigned)fb, 256, 0, ctx->stream>>>(
-          h.chiL, h.chiR, (const float*)w.T1, P.X, (float*)w.T3);
-  } else if (idt == ITG_F64) {
-    heff_wpass_kernel<double><<<(unsigned)blocks, 256, lds, ctx->stream>>>(
-        h.chiL, h.Q, h.O, (const double*)w.T1, P.X, (double*)w.T3);
-  } else {
-    heff_wpass_kernel<float><<<(unsigned)blocks, 256, lds, ctx->stream>>>(
-        h.chiL, h.Q, h.O, (const float*)w.T1, P.X, (float*)w.T3);
-  }
+  if (idt == ITG_F64)
+    wpass<double>(ctx, h.chiL, h.chiR, h.Q, h.O, (const double*)w.T1, P.X, (double*)w.T3);
+  else
+    wpass<float>(ctx, h.chiL, h.chiR, h.Q, h.O, (const float*)w.T1, P.X, (float*)w.T3);
   ITG_LAUNCH_CHECK(ctx);
   itg_tstop(ctx, tk, ITG_K_WPASS, 2.0 * h.Q * h.O * h.chiL * h.chiR,
             (double)(h.Q + h.O) * h.chiL * h.chiR * itg_dtype_size(idt));
