@@ -1185,6 +1185,16 @@ static int launch_gett(itg_ctx* ctx, int dtype, int mode, GettArgs& g, bool ak, 
   return launch_native<float>(ctx, g, ak, bk);
 }
 
+// The library does not split K: a product with fewer 64 x 64 tiles than half
+// the CUs and a long K leaves most of the chip idle there, and the native
+// kernel's K split is faster. FP64, us, library against native: 1200 x 277 x
+// 3878: 123 / 70, 600 x 600 x 6000: 182 / 105, 300 x 300 x 10000: 274 to 1074 /
+// 72, 700 x 277 x 1500: 34 to 86 / 27; on the other side 512^3: 12 / 18,
+// 256 x 1280 x 512: 19 / 21, 2000 x 400 x 5000 (224 tiles): 157 / 179.
+static bool split_k_wins(const itg_ctx* ctx, int64_t m, int64_t n, int64_t k) {
+  return ((m + 63) / 64) * ((n + 63) / 64) * 2 < std::max(ctx->num_cu, 1) && k >= 1024;
+}
+
 // A contraction whose M, N and K modes each merge into one stride is a plain
 // product C(m, n) = alpha sum_k A(m, k) B(k, n) + beta C(m, n), elements at
 // m sAm + k sAk, k sBk + n sBn, m sCm + n sCn. It runs as a column-major
@@ -1308,7 +1318,7 @@ extern "C" int itg_contract(itg_ctx* ctx, int dtype, int mode, int rA, const int
   g.alpha = alpha;
   g.beta = beta;
   if (!g.tAm && !g.tAk && !g.tBk && !g.tBn && !g.tCm && !g.tCn &&
-      itg_libgemm_ok(ctx, dtype, mode, g.M, g.N, g.K)) {
+      itg_libgemm_ok(ctx, dtype, mode, g.M, g.N, g.K) && !split_k_wins(ctx, g.M, g.N, g.K)) {
     int rc = contract_on_lib(ctx, g);
     if (rc != 1) return rc;
   }
@@ -1329,7 +1339,7 @@ int itg_gemm_internal(itg_ctx* ctx, int dtype, int mode, char ta, char tb, int64
   }
   bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
   if (!lower_band && lda >= (tA ? k : m) && ldb >= (tB ? n : k) && ldc >= m &&
-      itg_libgemm_ok(ctx, dtype, mode, m, n, k))
+      itg_libgemm_ok(ctx, dtype, mode, m, n, k) && !split_k_wins(ctx, m, n, k))
     return itg_libgemm(ctx, ta, tb, m, n, k, alpha, (const double*)A, lda, (const double*)B, ldb,
                        beta, (double*)C, ldc);
   GettArgs g;
