@@ -1,8 +1,8 @@
 // Davidson eigensolver for one bond's two-site effective Hamiltonian, on the
 // device: ITensors-style Krylov/Davidson (the eigsolve dmrg runs per bond,
-// test/dmrg.jl:27) with the FP64 Krylov basis, batched FP64 dot products
-// (one read-back per Gram-Schmidt pass), device-side Ritz combinations and
-// the small projected eigenproblem on the host (cyclic Jacobi). In split-BF16
+// test/dmrg.jl:27) with the FP64 Krylov basis, Gram-Schmidt and Ritz
+// combinations in fused passes on the device and the small projected
+// eigenproblem on the host (cyclic Jacobi). In split-BF16
 // mode the prepared Heff apply (five launches) is captured once into a HIP
 // graph per (dims, basis slot) and replayed.
 #include <hip/hip_runtime.h>
@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "itg_internal.h"
@@ -20,24 +21,48 @@ namespace {
 
 constexpr int kMaxBasis = 17;   // maxiter + 1 <= 17
 
-// part[b * cnt + k] = sum over this block's range of V_k . x (V_k = V + k n)
-__global__ __launch_bounds__(256) void multidot_kernel(int64_t n, const double* __restrict__ V,
-                                                       int cnt, const double* __restrict__ x,
-                                                       double* __restrict__ part) {
-  __shared__ double sh[4][kMaxBasis];
-  double s[kMaxBasis];
+// The vector work of a step is a chain of passes over the basis, each needing
+// the dot products of the one before. A pass leaves per-block partials, and
+// every block of the next one sums them itself (in the same order, so all
+// agree), so a Gram-Schmidt pass, its dot products and the norm never go
+// through the host: per step eight launches and two read-backs (the projected
+// matrix's new column and the residual norm) against 22 and five; a bond of
+// 300 x 277, w = 14 with three Krylov vectors 0.87 -> 0.61 ms.
+// Partials: nb x cnt, block b's k-th at part[b cnt + k].
+
+// the cnt sums over nb blocks, in LDS (tot), for a 256-thread block
+template <int MB>
+__device__ __forceinline__ void block_totals(const double* __restrict__ part, int nb, int cnt,
+                                             double (&sh)[4][MB], double (&tot)[MB]) {
+  double s[MB];
 #pragma unroll
-  for (int k = 0; k < kMaxBasis; ++k) s[k] = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double xi = x[i];
+  for (int k = 0; k < MB; ++k) s[k] = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 256)
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k)
-      if (k < cnt) s[k] += V[(size_t)k * n + i] * xi;
-  }
+    for (int k = 0; k < MB; ++k)
+      if (k < cnt) s[k] += part[(size_t)b * cnt + k];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
-  for (int k = 0; k < kMaxBasis; ++k) {
+  for (int k = 0; k < MB; ++k) {
+    if (k >= cnt) break;
+    double v = s[k];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) sh[w][k] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < cnt)
+    tot[threadIdx.x] = (sh[0][threadIdx.x] + sh[1][threadIdx.x]) +
+                       (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
+  __syncthreads();
+}
+
+// this block's cnt sums -> part
+template <int MB>
+__device__ __forceinline__ void write_partials(double (&s)[MB], int cnt, double (&sh)[4][MB],
+                                               double* __restrict__ part) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < MB; ++k) {
     if (k >= cnt) break;
     double v = s[k];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -49,59 +74,205 @@ __global__ __launch_bounds__(256) void multidot_kernel(int64_t n, const double* 
         (sh[0][threadIdx.x] + sh[1][threadIdx.x]) + (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
 }
 
-// out[k] = sum_b part[b][k]: wave w sums the dots k = w (mod 4), its lanes
-// striding over the block partials (a fixed order, so every call agrees)
-__global__ __launch_bounds__(256) void multidot_sum_kernel(int nb, int cnt,
-                                                           const double* __restrict__ part,
-                                                           double* __restrict__ out) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int k = wv; k < cnt; k += 4) {
-    double s = 0.0;
-    for (int b = lane; b < nb; b += 64) s += part[(size_t)b * cnt + k];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) out[k] = s;
+// partials of V_k . x (V_k = V + k n), k < cnt
+template <int MB>
+__global__ __launch_bounds__(256) void dots_kernel(int64_t n, const double* __restrict__ V,
+                                                   int cnt, const double* __restrict__ x,
+                                                   double* __restrict__ part) {
+  __shared__ double sh[4][MB];
+  double s[MB];
+#pragma unroll
+  for (int k = 0; k < MB; ++k) s[k] = 0.0;
+  for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) {
+    const double xi = x[i];
+#pragma unroll
+    for (int k = 0; k < MB; ++k)
+      if (k < cnt) s[k] += V[(size_t)k * n + i] * xi;
   }
+  write_partials<MB>(s, cnt, sh, part);
+}
+
+// y = x - sum_k h_k V_k, h the totals of `pin`; then partials of V_k . y
+// (norm 0) or of y . y (norm 1)
+template <int MB>
+__global__ __launch_bounds__(256) void project_kernel(int64_t n, const double* __restrict__ V,
+                                                      int cnt, const double* x, double* y,
+                                                      const double* __restrict__ pin, int nb,
+                                                      int norm, double* __restrict__ pout) {
+  __shared__ double sh[4][MB], h[MB];
+  block_totals<MB>(pin, nb, cnt, sh, h);
+  double s[MB];
+#pragma unroll
+  for (int k = 0; k < MB; ++k) s[k] = 0.0;
+  for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) {
+    double v[MB], yi = x[i];
+#pragma unroll
+    for (int k = 0; k < MB; ++k) {
+      v[k] = k < cnt ? V[(size_t)k * n + i] : 0.0;
+      if (k < cnt) yi -= h[k] * v[k];
+    }
+    y[i] = yi;
+    if (norm) {
+      s[0] += yi * yi;
+    } else {
+#pragma unroll
+      for (int k = 0; k < MB; ++k) s[k] += v[k] * yi;
+    }
+  }
+  __syncthreads();   // sh is reused
+  write_partials<MB>(s, norm ? 1 : cnt, sh, pout);
+}
+
+// y = x / sqrt(total of pin); the total goes to *out
+__global__ __launch_bounds__(256) void normalise_kernel(int64_t n, const double* x, double* y,
+                                                        const double* __restrict__ pin, int nb,
+                                                        double* out) {
+  __shared__ double sh[4][1], h[1];
+  block_totals<1>(pin, nb, 1, sh, h);
+  const double f = 1.0 / sqrt(h[0]);
+  for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) y[i] = f * x[i];
+  if (blockIdx.x == 0 && threadIdx.x == 0 && out) *out = h[0];
 }
 
 struct Coefs {
   double c[kMaxBasis];
 };
 
-// y = beta * y + sum_k c_k V_k  (V_k = V + k n)
-__global__ void lincomb_kernel(int64_t n, const double* __restrict__ V, int cnt, Coefs c,
-                               double beta, double* __restrict__ y) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double s = beta == 0.0 ? 0.0 : beta * y[i];
+// phi = sum_k u_k V_k and, if q, q = sum_k u_k AV_k - lam phi; partials of
+// (phi . phi, q . q)
+template <int MB>
+__global__ __launch_bounds__(256) void ritz_kernel(int64_t n, const double* __restrict__ V,
+                                                   const double* __restrict__ AV, int cnt,
+                                                   Coefs u, double lam, double* __restrict__ phi,
+                                                   double* __restrict__ q,
+                                                   double* __restrict__ part) {
+  __shared__ double sh[4][2];
+  double s[2] = {0.0, 0.0};
+  for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) {
+    double p = 0.0, r = 0.0;
 #pragma unroll
-    for (int k = 0; k < kMaxBasis; ++k)
-      if (k < cnt) s += c.c[k] * V[(size_t)k * n + i];
-    y[i] = s;
+    for (int k = 0; k < MB; ++k)
+      if (k < cnt) {
+        p += u.c[k] * V[(size_t)k * n + i];
+        if (q) r += u.c[k] * AV[(size_t)k * n + i];
+      }
+    phi[i] = p;
+    s[0] += p * p;
+    if (q) {
+      r -= lam * p;
+      q[i] = r;
+      s[1] += r * r;
+    }
   }
+  write_partials<2>(s, 2, sh, part);
 }
 
-// dots of x against V_0..V_{cnt-1}, read back to the host
-int multidot(itg_ctx* ctx, int64_t n, const double* V, int cnt, const double* x, double* host) {
-  unsigned nb = itg_blocks(n, 256, 512);
-  double* part = ctx->red + 32;
-  multidot_kernel<<<nb, 256, 0, ctx->stream>>>(n, V, cnt, x, part);
-  multidot_sum_kernel<<<1, 256, 0, ctx->stream>>>((int)nb, cnt, part, ctx->red);
-  ITG_LAUNCH_CHECK(ctx);
-  ITG_HIP(ctx, hipMemcpyAsync(ctx->red_host, ctx->red, cnt * sizeof(double),
-                              hipMemcpyDeviceToHost, ctx->stream));
-  ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  std::memcpy(host, ctx->red_host, cnt * sizeof(double));
-  return ITG_OK;
+// q = a - lam v with lam the total of `pin` (also to out[0]); partials of q . q
+__global__ __launch_bounds__(256) void residual_kernel(int64_t n, const double* __restrict__ a,
+                                                       const double* __restrict__ v,
+                                                       const double* __restrict__ pin, int nb,
+                                                       double* __restrict__ q,
+                                                       double* __restrict__ pout, double* out) {
+  __shared__ double sh[4][1], h[1];
+  block_totals<1>(pin, nb, 1, sh, h);
+  double s[1] = {0.0};
+  for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) {
+    const double r = a[i] - h[0] * v[i];
+    q[i] = r;
+    s[0] += r * r;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *out = h[0];
+  __syncthreads();   // sh is reused
+  write_partials<1>(s, 1, sh, pout);
 }
 
-int lincomb(itg_ctx* ctx, int64_t n, const double* V, int cnt, const double* c, double beta,
-            double* y) {
-  Coefs cf;
-  for (int k = 0; k < kMaxBasis; ++k) cf.c[k] = k < cnt ? c[k] : 0.0;
-  lincomb_kernel<<<itg_blocks(n, 256, 8192), 256, 0, ctx->stream>>>(n, V, cnt, cf, beta, y);
-  ITG_LAUNCH_CHECK(ctx);
-  return ITG_OK;
+__global__ __launch_bounds__(256) void totals_kernel(int nb, int cnt,
+                                                     const double* __restrict__ part,
+                                                     double* out) {
+  __shared__ double sh[4][kMaxBasis], tot[kMaxBasis];
+  block_totals<kMaxBasis>(part, nb, cnt, sh, tot);
+  if (threadIdx.x < cnt) out[threadIdx.x] = tot[threadIdx.x];
 }
+
+// y = beta * y + alpha x
+__global__ void axpby_kernel(int64_t n, double alpha, const double* __restrict__ x, double beta,
+                             double* __restrict__ y) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    y[i] = alpha * x[i] + (beta == 0.0 ? 0.0 : beta * y[i]);
+}
+
+// Launches of the passes on one context. Results for the host are written by
+// the kernels into the context's pinned buffer: slots 0.. from totals, 20 and
+// 21 from normalise and residual.
+struct Passes {
+  itg_ctx* ctx;
+  int64_t n;
+  static constexpr int kPart = 5000;   // doubles per partial buffer
+  double* part(int i) const { return ctx->red + 32 + i * kPart; }
+  double* host() const { return ctx->red_host; }
+  // blocks of a pass with cnt sums: about 1024 elements each, at most 1024
+  // (enough to stream from HBM) and at most the partial buffer's room
+  int blocks(int cnt) const {
+    const int64_t b = std::min<int64_t>({(n + 1023) / 1024, 1024, kPart / cnt});
+    return (int)std::max<int64_t>(b, 1);
+  }
+  template <typename F>
+  static void by_size(int cnt, F&& f) {   // f(integral constant >= cnt)
+    if (cnt <= 2) f(std::integral_constant<int, 2>());
+    else if (cnt <= 4) f(std::integral_constant<int, 4>());
+    else if (cnt <= 8) f(std::integral_constant<int, 8>());
+    else f(std::integral_constant<int, kMaxBasis>());
+  }
+  int dots(const double* V, int cnt, const double* x, int pout) const {
+    by_size(cnt, [&](auto mb) {
+      dots_kernel<mb()><<<blocks(cnt), 256, 0, ctx->stream>>>(n, V, cnt, x, part(pout));
+    });
+    ITG_LAUNCH_CHECK(ctx);
+    return ITG_OK;
+  }
+  int project(const double* V, int cnt, const double* x, double* y, int pin, bool norm,
+              int pout) const {
+    by_size(cnt, [&](auto mb) {
+      // the output partials hold cnt or one sum; one grid serves both
+      project_kernel<mb()><<<blocks(cnt), 256, 0, ctx->stream>>>(n, V, cnt, x, y, part(pin),
+                                                                 blocks(cnt), norm ? 1 : 0,
+                                                                 part(pout));
+    });
+    ITG_LAUNCH_CHECK(ctx);
+    return ITG_OK;
+  }
+  // nb: blocks that left the partials
+  int normalise(const double* x, double* y, int pin, int nb) const {
+    normalise_kernel<<<blocks(1), 256, 0, ctx->stream>>>(n, x, y, part(pin), nb, host() + 20);
+    ITG_LAUNCH_CHECK(ctx);
+    return ITG_OK;
+  }
+  int residual(const double* a, const double* v, int pin, double* q, int pout) const {
+    residual_kernel<<<blocks(1), 256, 0, ctx->stream>>>(n, a, v, part(pin), blocks(1), q,
+                                                        part(pout), host() + 21);
+    ITG_LAUNCH_CHECK(ctx);
+    return ITG_OK;
+  }
+  int ritz(const double* V, const double* AV, int cnt, const double* u, double lam, double* phi,
+           double* q, int pout) const {
+    Coefs c;
+    for (int k = 0; k < kMaxBasis; ++k) c.c[k] = k < cnt ? u[k] : 0.0;
+    by_size(cnt, [&](auto mb) {
+      ritz_kernel<mb()><<<blocks(2), 256, 0, ctx->stream>>>(n, V, AV, cnt, c, lam, phi, q,
+                                                            part(pout));
+    });
+    ITG_LAUNCH_CHECK(ctx);
+    return ITG_OK;
+  }
+  // totals of cnt partials to the host's slots 0.., and wait
+  int fetch(int pin, int cnt) const {
+    totals_kernel<<<1, 256, 0, ctx->stream>>>(blocks(cnt), cnt, part(pin), host());
+    ITG_LAUNCH_CHECK(ctx);
+    ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return ITG_OK;
+  }
+};
 
 // lowest eigenpair of the symmetric m x m matrix M (row-major) by cyclic
 // Jacobi; u normalised with u[0] >= 0
@@ -241,12 +412,16 @@ static int learned_correction(itg_ctx* ctx, const LearnedStep& ls, int64_t chiL,
     if (rc) return rc;
     sv = ls.tskip;
   }
-  double h[kMaxBasis];
-  rc = multidot(ctx, n, sv, 1, sv, h);
+  const Passes ps{ctx, n};
+  rc = ps.dots(sv, 1, sv, 0);
   if (rc) return rc;
-  const double sn = std::sqrt(h[0]);
+  rc = ps.fetch(0, 1);
+  if (rc) return rc;
+  const double sn = std::sqrt(ps.host()[0]);
   double sc = sn > 0.0 ? std::sqrt((double)n) / sn : 0.0;
-  return lincomb(ctx, n, sv, 1, &sc, 1.0, t);
+  axpby_kernel<<<itg_blocks(n, 256, 8192), 256, 0, ctx->stream>>>(n, sc, sv, 1.0, t);
+  ITG_LAUNCH_CHECK(ctx);
+  return ITG_OK;
 }
 
 // ITensors' davidson on one bond with the basis on the device. With a
@@ -276,36 +451,24 @@ static int davidson2_core(itg_ctx* ctx, int dtype, int mode, int64_t chiL, int64
   double* q = AV + (size_t)(maxiter + 1) * n;       // residual
   double* t = q + n;                                // correction
   double* phi = t + n;                              // Ritz vector
-  double h[kMaxBasis], u[kMaxBasis];
+  double u[kMaxBasis];
   int rc;
-  // V0 = psi / |psi|
-  rc = multidot(ctx, n, (const double*)psi, 1, (const double*)psi, h);
-  if (rc) return rc;
-  double nrm = std::sqrt(h[0]);
-  if (!(nrm > 0.0)) return itg_fail(ctx, ITG_EARG, "davidson2: zero start vector");
-  double one = 1.0 / nrm;
-  rc = lincomb(ctx, n, (const double*)psi, 1, &one, 0.0, V);
-  if (rc) return rc;
+  const Passes ps{ctx, n};
+  const double* h = ps.host();   // slots valid after a fetch
+  // V0 = psi / |psi|, AV0, lam = V0 . AV0, q = AV0 - lam V0
+  if ((rc = ps.dots((const double*)psi, 1, (const double*)psi, 0))) return rc;
+  if ((rc = ps.normalise((const double*)psi, V, 0, ps.blocks(1)))) return rc;
   rc = heff_apply_graph(ctx, dtype, mode, dims, L, R, prep, V, AV, work);
   if (rc) return rc;
+  if ((rc = ps.dots(V, 1, AV, 0))) return rc;
+  if ((rc = ps.residual(AV, V, 0, q, 1))) return rc;
+  if ((rc = ps.fetch(1, 1))) return rc;
+  if (!(h[20] > 0.0)) return itg_fail(ctx, ITG_EARG, "davidson2: zero start vector");
+  double lam = h[21], last = NAN, qn = std::sqrt(h[0]);
   int nmv = 1, m = 1, nrev = 0;
-  rc = multidot(ctx, n, V, 1, AV, h);
-  if (rc) return rc;
-  double lam = h[0], last = NAN;
   std::vector<double> M(kMaxBasis * kMaxBasis, 0.0);
   M[0] = lam;
-  // q = AV0 - lam V0
-  {
-    double c1 = 1.0, cl = -lam;
-    rc = lincomb(ctx, n, AV, 1, &c1, 0.0, q);
-    if (rc) return rc;
-    rc = lincomb(ctx, n, V, 1, &cl, 1.0, q);
-    if (rc) return rc;
-  }
   u[0] = 1.0;
-  rc = multidot(ctx, n, q, 1, q, h);
-  if (rc) return rc;
-  double qn = std::sqrt(h[0]);
   for (int ni = 1; ni <= maxiter; ++ni) {
     bool conv = (qn < errgoal && std::fabs(lam - last) < errgoal) ||
                 qn < std::max(1e-12, errgoal * 1e-3);
@@ -318,21 +481,25 @@ static int davidson2_core(itg_ctx* ctx, int dtype, int mode, int64_t chiL, int64
       const bool net = try_net && att == 0;
       const bool guarded = net;   // the diagonal step is the fallback
       // correction
+      const double* t0 = t;
+      rc = ITG_OK;
       if (net) rc = learned_correction(ctx, *ls, chiL, d, chiR, q, (const double*)diag, lam, t);
       else if (diag) rc = itg_precond_diag(ctx, ITG_F64, n, q, diag, lam, 1e-8, t);
-      else rc = itg_memcpy_d2d(ctx, t, q, (size_t)n * sizeof(double));
+      else t0 = q;
       if (rc) return rc;
-      // two Gram-Schmidt passes against the basis
-      for (int pass = 0; pass < 2; ++pass) {
-        rc = multidot(ctx, n, V, m, t, h);
-        if (rc) return rc;
-        for (int k = 0; k < m; ++k) h[k] = -h[k];
-        rc = lincomb(ctx, n, V, m, h, 1.0, t);
-        if (rc) return rc;
-      }
-      rc = multidot(ctx, n, t, 1, t, h);
+      // two Gram-Schmidt passes against the basis, then V_m = t / |t|
+      if ((rc = ps.dots(V, m, t0, 0))) return rc;
+      if ((rc = ps.project(V, m, t0, t, 0, false, 1))) return rc;
+      if ((rc = ps.project(V, m, t, t, 1, true, 2))) return rc;
+      if ((rc = ps.normalise(t, V + (size_t)m * n, 2, ps.blocks(m)))) return rc;
+      rc = heff_apply_graph(ctx, dtype, mode, dims, L, R, prep, V + (size_t)m * n,
+                            AV + (size_t)m * n, work);
       if (rc) return rc;
-      double tn = std::sqrt(h[0]);
+      if ((rc = ps.dots(V, m + 1, AV + (size_t)m * n, 0))) return rc;
+      if ((rc = ps.fetch(0, m + 1))) return rc;
+      // a correction inside the basis: its product (in flight by now) is
+      // dropped
+      const double tn = std::sqrt(h[20]);
       if (tn < 1e-14 * std::max(1.0, qn)) {
         if (guarded) {
           ++nrev;
@@ -345,15 +512,7 @@ static int davidson2_core(itg_ctx* ctx, int dtype, int mode, int64_t chiL, int64
       const double lamprev = lam;
       double uprev[kMaxBasis];
       for (int k = 0; k < m; ++k) uprev[k] = u[k];
-      double sc = 1.0 / tn;
-      rc = lincomb(ctx, n, t, 1, &sc, 0.0, V + (size_t)m * n);
-      if (rc) return rc;
-      rc = heff_apply_graph(ctx, dtype, mode, dims, L, R, prep, V + (size_t)m * n,
-                            AV + (size_t)m * n, work);
-      if (rc) return rc;
       ++nmv;
-      rc = multidot(ctx, n, V, m + 1, AV + (size_t)m * n, h);
-      if (rc) return rc;
       ++m;
       std::vector<double> Mn(m * m);
       for (int a = 0; a < m - 1; ++a)
@@ -361,45 +520,33 @@ static int davidson2_core(itg_ctx* ctx, int dtype, int mode, int64_t chiL, int64
       for (int k = 0; k < m; ++k) Mn[k * m + (m - 1)] = Mn[(m - 1) * m + k] = h[k];
       M.assign(Mn.begin(), Mn.end());
       small_lowest(m, M.data(), &lam, u);
-      // phi = sum u_k V_k, q = sum u_k AV_k - lam phi
-      rc = lincomb(ctx, n, V, m, u, 0.0, phi);
-      if (rc) return rc;
-      rc = lincomb(ctx, n, AV, m, u, 0.0, q);
-      if (rc) return rc;
-      double ml = -lam;
-      rc = lincomb(ctx, n, phi, 1, &ml, 1.0, q);
-      if (rc) return rc;
-      rc = multidot(ctx, n, q, 1, q, h);
-      if (rc) return rc;
-      const double qn_new = std::sqrt(h[0]);
-      if (guarded && !(qn_new < qn)) {
-        // the learned step did not lower the residual: drop it
-        --m;
-        M.assign(Mprev.begin(), Mprev.end());
-        lam = lamprev;
-        for (int k = 0; k < m; ++k) u[k] = uprev[k];
-        rc = lincomb(ctx, n, V, m, u, 0.0, phi);
-        if (rc) return rc;
-        rc = lincomb(ctx, n, AV, m, u, 0.0, q);
-        if (rc) return rc;
-        ml = -lam;
-        rc = lincomb(ctx, n, phi, 1, &ml, 1.0, q);
-        if (rc) return rc;
-        ++nrev;
-        continue;
+      // phi = sum u_k V_k, q = sum u_k AV_k - lam phi; nothing reads the
+      // residual of the last step
+      const bool lastq = ni == maxiter && !guarded;
+      if ((rc = ps.ritz(V, AV, m, u, lam, phi, lastq ? nullptr : q, 0))) return rc;
+      if (!lastq) {
+        if ((rc = ps.fetch(0, 2))) return rc;
+        const double qn_new = std::sqrt(h[1]);
+        if (guarded && !(qn_new < qn)) {
+          // the learned step did not lower the residual: drop it
+          --m;
+          M.assign(Mprev.begin(), Mprev.end());
+          lam = lamprev;
+          for (int k = 0; k < m; ++k) u[k] = uprev[k];
+          if ((rc = ps.ritz(V, AV, m, u, lam, phi, q, 0))) return rc;
+          ++nrev;
+          continue;
+        }
+        qn = qn_new;
       }
-      qn = qn_new;
       stepped = true;
     }
     if (!stepped) break;
   }
   // psi = Ritz vector (V0 when no step was taken), normalised
   const double* src = (m == 1) ? V : phi;
-  rc = multidot(ctx, n, src, 1, src, h);
-  if (rc) return rc;
-  double inv = 1.0 / std::sqrt(h[0]);
-  rc = lincomb(ctx, n, src, 1, &inv, 0.0, (double*)psi);
-  if (rc) return rc;
+  if ((rc = ps.dots(src, 1, src, 0))) return rc;
+  if ((rc = ps.normalise(src, (double*)psi, 0, ps.blocks(1)))) return rc;
   *energy = lam;
   if (matvecs) *matvecs = nmv;
   if (reverted) *reverted = nrev;
