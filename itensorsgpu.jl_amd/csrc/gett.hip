@@ -621,22 +621,59 @@ __global__ __launch_bounds__(256, TS == 128 ? 2 : 4) void gett_native_kernel(Get
   }
 }
 
-// split-K reduction + epilogue
-template <typename T, typename CT>
+// split-K reduction + epilogue. A block takes 64 (or, with few partials, 256)
+// consecutive outputs; ZW waves share an output's partials (z = wave mod ZW,
+// eight loads in flight each) and meet in LDS in a fixed order. One thread
+// per output, walking the partials, was latency-bound: 12.7 us for 64 of
+// 256 x 256 FP32, 3.6 now.
+template <typename T, typename CT, int ZW>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(GettArgs g, int nsplit) {
-  int64_t MN = g.M * g.N;
-  const CT* P = (const CT*)g.partial;
+  constexpr int EB = 256 / ZW;   // outputs per block and turn
+  __shared__ double sh[ZW][EB];
+  const int64_t MN = g.M * g.N;
+  const CT* __restrict__ P = (const CT*)g.partial;
   T* C = (T*)g.C;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < MN;
-       e += (int64_t)gridDim.x * blockDim.x) {
+  const int ei = threadIdx.x % EB, zi = threadIdx.x / EB;
+  for (int64_t e0 = blockIdx.x * (int64_t)EB; e0 < MN; e0 += (int64_t)gridDim.x * EB) {
+    const int64_t e = e0 + ei;
     double s = 0.0;
-    for (int z = 0; z < nsplit; ++z) s += (double)P[z * MN + e];
-    int64_t n = e % g.N, m = e / g.N;
-    int64_t o = goff(g.tCm, g.sCm, m) + goff(g.tCn, g.sCn, n);
+    if (e < MN) {
+      const CT* p = P + e;
+      int z = zi;
+      for (; z + 7 * ZW < nsplit; z += 8 * ZW) {
+        CT v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = p[(int64_t)(z + q * ZW) * MN];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += (double)v[q];
+      }
+      for (; z < nsplit; z += ZW) s += (double)p[(int64_t)z * MN];
+    }
+    if constexpr (ZW > 1) {
+      __syncthreads();
+      sh[zi][ei] = s;
+      __syncthreads();
+      if (zi != 0) continue;
+      s = sh[0][ei];
+#pragma unroll
+      for (int q = 1; q < ZW; ++q) s += sh[q][ei];
+    }
+    if (e >= MN) continue;
+    const int64_t n = e % g.N, m = e / g.N;
+    const int64_t o = goff(g.tCm, g.sCm, m) + goff(g.tCn, g.sCn, n);
     double v = g.alpha * s;
     if (g.beta != 0.0) v += g.beta * (double)C[o];
     C[o] = (T)v;
   }
+}
+
+template <typename T, typename CT>
+static void splitk_reduce(itg_ctx* ctx, const GettArgs& g, int nsplit) {
+  const int64_t MN = g.M * g.N;
+  if (nsplit >= 8)
+    splitk_reduce_kernel<T, CT, 4><<<itg_blocks(MN, 64, 8192), 256, 0, ctx->stream>>>(g, nsplit);
+  else
+    splitk_reduce_kernel<T, CT, 1><<<itg_blocks(MN, 256, 4096), 256, 0, ctx->stream>>>(g, nsplit);
 }
 
 // Contractions with at most 16 outputs (scalars, short vectors; dot-like):
@@ -725,58 +762,96 @@ struct itg_plan {
   SicArgs sa = {};
 };
 
-template <typename T, int GM>
+// blockIdx.y takes GM of the G outputs (its own part of Y in LDS), so that a
+// small F still fills the chip; X is then read once per part, from L2.
+// F = 305000, K = G = 8 FP64: 24 us with 64-bit index arithmetic and every
+// output in one thread, 19 now; the operator products of a DMRG sweep on a
+// 4 x 6 cylinder take 8.6 us on average.
+template <typename T, int GM, typename I>
 __global__ __launch_bounds__(256) void sic_kernel(SicArgs a) {
-  __shared__ T ys[SIC_KMAX * SIC_GMAX];   // Y(k, g) at k G + g
-  __shared__ int64_t kox[SIC_KMAX];       // offset of k in X
-  __shared__ int64_t goc[SIC_GMAX];       // offset of g in C
+  __shared__ T ys[SIC_KMAX * GM];      // Y(k, g0 + g) at k GM + g
+  __shared__ int64_t kox[SIC_KMAX];    // offset of k in X
+  __shared__ int64_t goc[GM];          // offset of g0 + g in C
   const int t = threadIdx.x;
+  const int g0 = (int)blockIdx.y * GM, ng = min(GM, a.G - g0);
   const T* __restrict__ Y = (const T*)a.Y;
-  for (int e = t; e < a.K * a.G; e += 256) {
-    int64_t rk = e / a.G, rg = e % a.G, o = 0;
-    for (int q = 0; q < a.nk; ++q) { o += (rk % a.kd[q]) * a.ky[q]; rk /= a.kd[q]; }
-    for (int q = 0; q < a.ng; ++q) { o += (rg % a.gd[q]) * a.gy[q]; rg /= a.gd[q]; }
-    ys[e] = Y[o];
+  for (int e = t; e < a.K * GM; e += 256) {
+    int rk = e / GM, rg = g0 + e % GM;
+    int64_t o = 0;
+    const bool live = e % GM < ng;
+    for (int q = 0; q < a.nk; ++q) { o += (rk % (int)a.kd[q]) * a.ky[q]; rk /= (int)a.kd[q]; }
+    for (int q = 0; q < a.ng; ++q) { o += (rg % (int)a.gd[q]) * a.gy[q]; rg /= (int)a.gd[q]; }
+    ys[e] = live ? Y[o] : (T)0;
   }
   for (int k = t; k < a.K; k += 256) {
-    int64_t r = k, o = 0;
-    for (int q = 0; q < a.nk; ++q) { o += (r % a.kd[q]) * a.kx[q]; r /= a.kd[q]; }
+    int r = k;
+    int64_t o = 0;
+    for (int q = 0; q < a.nk; ++q) { o += (r % (int)a.kd[q]) * a.kx[q]; r /= (int)a.kd[q]; }
     kox[k] = o;
   }
-  for (int g = t; g < a.G; g += 256) {
-    int64_t r = g, o = 0;
-    for (int q = 0; q < a.ng; ++q) { o += (r % a.gd[q]) * a.gc[q]; r /= a.gd[q]; }
+  for (int g = t; g < ng; g += 256) {
+    int r = g0 + g;
+    int64_t o = 0;
+    for (int q = 0; q < a.ng; ++q) { o += (r % (int)a.gd[q]) * a.gc[q]; r /= (int)a.gd[q]; }
     goc[g] = o;
   }
   __syncthreads();
   const int64_t f = (int64_t)blockIdx.x * 256 + t;
   if (f >= a.F) return;
-  int64_t ox = 0, oc = 0, r = f;
+  int64_t ox = 0, oc = 0;
+  I r = (I)f;
   for (int q = 0; q < a.nf; ++q) {
-    const int64_t i = r % a.fd[q];
-    r /= a.fd[q];
-    ox += i * a.fx[q];
-    oc += i * a.fc[q];
+    const I dq = (I)a.fd[q], rq = r / dq, i = r - rq * dq;
+    r = rq;
+    ox += (int64_t)i * a.fx[q];
+    oc += (int64_t)i * a.fc[q];
   }
   const T* __restrict__ X = (const T*)a.X + ox;
   T acc[GM];
 #pragma unroll
   for (int g = 0; g < GM; ++g) acc[g] = (T)0;
-#pragma unroll 4
-  for (int k = 0; k < a.K; ++k) {
+  int k = 0;
+  for (; k + 8 <= a.K; k += 8) {
+    T xv[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) xv[q] = X[kox[k + q]];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+#pragma unroll
+      for (int g = 0; g < GM; ++g) acc[g] += xv[q] * ys[(k + q) * GM + g];
+  }
+  for (; k < a.K; ++k) {
     const T xv = X[kox[k]];
 #pragma unroll
-    for (int g = 0; g < GM; ++g)
-      if (g < a.G) acc[g] += xv * ys[k * a.G + g];
+    for (int g = 0; g < GM; ++g) acc[g] += xv * ys[k * GM + g];
   }
   T* __restrict__ C = (T*)a.C + oc;
 #pragma unroll
   for (int g = 0; g < GM; ++g) {
-    if (g < a.G) {
+    if (g < ng) {
       T v = (T)a.alpha * acc[g];
       if (a.beta != 0.0) v += (T)a.beta * C[goc[g]];
       C[goc[g]] = v;
     }
+  }
+}
+
+template <typename T>
+static void launch_sic_t(itg_ctx* ctx, const SicArgs& a, unsigned nblk) {
+  // outputs per thread: all of them for a large F, fewer until the grid has
+  // four workgroups per CU
+  int gm = a.G <= 4 ? 4 : a.G <= 8 ? 8 : a.G <= 16 ? 16 : 32;
+  const int64_t want = 4 * (int64_t)std::max(ctx->num_cu, 1);
+  while (gm > 4 && (int64_t)nblk * ((a.G + gm - 1) / gm) < want) gm /= 2;
+  const dim3 grid(nblk, (a.G + gm - 1) / gm);
+  auto go = [&](auto kernel) { kernel<<<grid, 256, 0, ctx->stream>>>(a); };
+  if (a.F <= 0x7fffffff) {
+    if (gm == 4) go(sic_kernel<T, 4, uint32_t>);
+    else if (gm == 8) go(sic_kernel<T, 8, uint32_t>);
+    else if (gm == 16) go(sic_kernel<T, 16, uint32_t>);
+    else go(sic_kernel<T, SIC_GMAX, uint32_t>);
+  } else {
+    go(sic_kernel<T, SIC_GMAX, int64_t>);
   }
 }
 
@@ -791,14 +866,8 @@ static int launch_sic(itg_ctx* ctx, int dtype, const itg_plan* p, const void* A,
   const int64_t nblk = (a.F + 255) / 256;
   if (nblk > 0x7fffffff) return itg_fail(ctx, ITG_EUNSUPPORTED, "contraction too large");
   const int tk = itg_tstart(ctx, ITG_K_GETT);
-  const bool small = a.G <= 16;
-  if (dtype == ITG_F64) {
-    if (small) sic_kernel<double, 16><<<(unsigned)nblk, 256, 0, ctx->stream>>>(a);
-    else sic_kernel<double, SIC_GMAX><<<(unsigned)nblk, 256, 0, ctx->stream>>>(a);
-  } else {
-    if (small) sic_kernel<float, 16><<<(unsigned)nblk, 256, 0, ctx->stream>>>(a);
-    else sic_kernel<float, SIC_GMAX><<<(unsigned)nblk, 256, 0, ctx->stream>>>(a);
-  }
+  if (dtype == ITG_F64) launch_sic_t<double>(ctx, a, (unsigned)nblk);
+  else launch_sic_t<float>(ctx, a, (unsigned)nblk);
   ITG_LAUNCH_CHECK(ctx);
   const double es = dtype == ITG_F64 ? 8.0 : 4.0;
   itg_tstop(ctx, tk, ITG_K_GETT, 2.0 * a.F * a.G * a.K,
@@ -1047,7 +1116,7 @@ static int launch_gett_t(itg_ctx* ctx, GettArgs& g, bool ak, bool bk) {
   itg_tstop(ctx, tk, ITG_K_GETT, 2.0 * g.M * g.N * g.K,
             (double)sizeof(T) * (g.M * g.K + g.K * g.N + g.M * g.N * (g.beta != 0.0 ? 2 : 1)));
   if (nsplit > 1) {
-    splitk_reduce_kernel<T, CT><<<itg_blocks(g.M * g.N, 256, 4096), 256, 0, ctx->stream>>>(g, nsplit);
+    splitk_reduce<T, CT>(ctx, g, nsplit);
     ITG_LAUNCH_CHECK(ctx);
   }
   return ITG_OK;
@@ -1155,8 +1224,7 @@ static int launch_native(itg_ctx* ctx, GettArgs& g, bool ak, bool bk) {
   itg_tstop(ctx, tk, ITG_K_GETT, 2.0 * g.M * g.N * g.K,
             (double)sizeof(T) * (g.M * g.K + g.K * g.N + g.M * g.N * (g.beta != 0.0 ? 2 : 1)));
   if (nsplit > 1) {
-    splitk_reduce_kernel<T, T><<<itg_blocks(g.M * g.N, 256, 4096), 256, 0, ctx->stream>>>(
-        g, (int)nsplit);
+    splitk_reduce<T, T>(ctx, g, (int)nsplit);
     ITG_LAUNCH_CHECK(ctx);
   }
   return ITG_OK;
