@@ -2,11 +2,14 @@
 // preconditioner: forward, MSE backward and Adam, FP32. No counterpart in the
 // reference. Activations are feature-major (column-major features x rows, i.e.
 // row-major rows x features); weights are packed row-major
-// [W1(h x in), b1, W2(h x h), b2, W3(out x h), b3]. The matrix products run
-// on FP32 MFMA through the contraction kernel; bias, GELU and the loss are
-// fused elementwise kernels.
+// [W1(h x in), b1, W2(h x h), b2, W3(out x h), b3]. The hidden x hidden
+// products run on FP32 MFMA through the contraction kernel; layers 1 and 3
+// with their biases, GELUs and gradients are fused passes over the
+// activations, or products and elementwise kernels when they have many
+// inputs or outputs.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "itg_internal.h"
@@ -82,6 +85,287 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(int f, int64_t rows, con
   if (threadIdx.x == 0) gb[feat] = (float)(sh[0] + sh[1] + sh[2] + sh[3]);
 }
 
+// ------------------------------------------- fused outer layers (training)
+// With few inputs and outputs (in <= 32, out <= 16: the preconditioner has 12
+// and 4, or 27 and 9) layers 1 and 3 and their gradients are a few
+// multiply-adds per hidden unit and row, far below the traffic of the
+// activations they read and write, so they ride along with the bias, GELU and
+// GELU' passes instead of being products of their own; only the hidden x
+// hidden products stay on MFMA. Thread = hidden unit (blockIdx.y: groups of
+// 256), block = a range of rows; layer 3's sums over the hidden units take a
+// wave per row instead. Weight and bias gradients leave one partial per block,
+// summed in one last launch. Forward and backward of 4096 rows at 12 -> 256 ->
+// 256 -> 4 take 10 launches and 97 us; as products and elementwise passes,
+// 142. At the limit: in = 32, out = 16 122 us, past it 154 to 158 (200 rows:
+// 87 against 130; 65536 rows: 722 against 960 to 999).
+constexpr int MLP_IN = 32, MLP_OUT = 16, MLP_TILE = 16;   // rows staged in LDS
+
+bool mlp_outer_fused(int in, int out) { return in <= MLP_IN && out <= MLP_OUT; }
+
+// Z1 = W1 X + b1, A1 = gelu(Z1)
+template <int IN>
+__global__ __launch_bounds__(256) void mlp_layer1_kernel(int64_t rows, int in, int h, int64_t rpb,
+                                                         const float* __restrict__ W1,
+                                                         const float* __restrict__ b1,
+                                                         const float* __restrict__ X,
+                                                         float* __restrict__ Z1,
+                                                         float* __restrict__ A1) {
+  __shared__ float xs[MLP_TILE][IN];
+  const int t = threadIdx.x, f = blockIdx.y * 256 + t;
+  float w[IN];
+#pragma unroll
+  for (int k = 0; k < IN; ++k) w[k] = (f < h && k < in) ? W1[(int64_t)f * in + k] : 0.0f;
+  const float b = f < h ? b1[f] : 0.0f;
+  const int64_t r0 = blockIdx.x * rpb, r1 = r0 + rpb < rows ? r0 + rpb : rows;
+  for (int64_t rt = r0; rt < r1; rt += MLP_TILE) {
+    const int nr = (int)(r1 - rt < MLP_TILE ? r1 - rt : MLP_TILE);
+    __syncthreads();
+    for (int e = t; e < MLP_TILE * IN; e += 256) {
+      const int r = e / IN, k = e % IN;
+      xs[r][k] = (r < nr && k < in) ? X[(rt + r) * in + k] : 0.0f;
+    }
+    __syncthreads();
+    if (f >= h) continue;
+    for (int r = 0; r < nr; ++r) {
+      float z = b;
+#pragma unroll
+      for (int k = 0; k < IN; ++k) z += xs[r][k] * w[k];
+      Z1[(rt + r) * h + f] = z;
+      A1[(rt + r) * h + f] = gelu_f(z);
+    }
+  }
+}
+
+// Z2 += b2, A2 = gelu(Z2), Y = W3 A2 + b3; a wave takes two rows at a time
+// (W3 is read from L1 for both), its lanes the hidden units
+template <int OUT>
+__global__ __launch_bounds__(256) void mlp_layer3_kernel(int64_t rows, int h, int out,
+                                                         const float* __restrict__ b2,
+                                                         const float* __restrict__ W3,
+                                                         const float* __restrict__ b3,
+                                                         float* __restrict__ Z2,
+                                                         float* __restrict__ A2,
+                                                         float* __restrict__ Y) {
+  constexpr int R = 2;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int64_t rt = ((int64_t)blockIdx.x * 4 + wv) * R; rt < rows; rt += (int64_t)gridDim.x * 4 * R) {
+    const int nr = (int)(rows - rt < R ? rows - rt : R);
+    float acc[R][OUT];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) acc[r][o] = 0.0f;
+#pragma unroll 4
+    for (int f = lane; f < h; f += 64) {
+      const float b = b2[f];
+      float w[OUT];
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) w[o] = o < out ? W3[(int64_t)o * h + f] : 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (r >= nr) continue;
+        const int64_t e = (rt + r) * h + f;
+        const float z = Z2[e] + b;
+        const float a = gelu_f(z);
+        Z2[e] = z;
+        A2[e] = a;
+#pragma unroll
+        for (int o = 0; o < OUT; ++o) acc[r][o] += a * w[o];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) {
+        if (r >= nr || o >= out) continue;
+        float v = acc[r][o];
+        for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s, 64);
+        if (lane == 0) Y[(rt + r) * out + o] = b3[o] + v;
+      }
+  }
+}
+
+// dY = 2 (Y - T) scale; per block the sums over its rows of dY (out of them)
+// and of (Y - T)^2: part[block (out + 1) + ..]
+__global__ __launch_bounds__(256) void mlp_mse_kernel(int64_t rows, int out, int64_t rpb,
+                                                      const float* __restrict__ Y,
+                                                      const float* __restrict__ T, float scale,
+                                                      float* __restrict__ dY,
+                                                      double* __restrict__ part) {
+  __shared__ double sb[256], sl[256];
+  const int t = threadIdx.x, per = 256 / out;   // rows a turn
+  const int o = t % out, rr = t / out;
+  const int64_t r0 = blockIdx.x * rpb, r1 = r0 + rpb < rows ? r0 + rpb : rows;
+  double b = 0.0, l = 0.0;
+  if (rr < per)
+    for (int64_t r = r0 + rr; r < r1; r += per) {
+      const float d = Y[r * out + o] - T[r * out + o];
+      const float g = 2.0f * d * scale;
+      dY[r * out + o] = g;
+      b += (double)g;
+      l += (double)d * d;
+    }
+  sb[t] = b;
+  sl[t] = l;
+  __syncthreads();
+  if (t < out) {
+    double s = 0.0;
+    for (int q = 0; q < per; ++q) s += sb[q * out + t];
+    part[(int64_t)blockIdx.x * (out + 1) + t] = s;
+  }
+  for (int s = 128; s > 0; s >>= 1) {
+    if (t < s) sl[t] += sl[t + s];
+    __syncthreads();
+  }
+  if (t == 0) part[(int64_t)blockIdx.x * (out + 1) + out] = sl[0];
+}
+
+// dZ2 = (W3^T dY) gelu'(Z2), and this block's partials of dW3 (out x h) and db2
+template <int OUT>
+__global__ __launch_bounds__(256) void mlp_back3_kernel(int64_t rows, int h, int out, int64_t rpb,
+                                                        const float* __restrict__ W3,
+                                                        const float* __restrict__ dY,
+                                                        const float* __restrict__ Z2,
+                                                        const float* __restrict__ A2,
+                                                        float* __restrict__ dZ2,
+                                                        float* __restrict__ pw,
+                                                        float* __restrict__ pb) {
+  __shared__ float ds[MLP_TILE][OUT];
+  const int t = threadIdx.x, f = blockIdx.y * 256 + t;
+  float w[OUT], gw[OUT];
+  double gb = 0.0;
+#pragma unroll
+  for (int o = 0; o < OUT; ++o) {
+    w[o] = (f < h && o < out) ? W3[(int64_t)o * h + f] : 0.0f;
+    gw[o] = 0.0f;
+  }
+  const int64_t r0 = blockIdx.x * rpb, r1 = r0 + rpb < rows ? r0 + rpb : rows;
+  for (int64_t rt = r0; rt < r1; rt += MLP_TILE) {
+    const int nr = (int)(r1 - rt < MLP_TILE ? r1 - rt : MLP_TILE);
+    __syncthreads();
+    for (int e = t; e < MLP_TILE * OUT; e += 256) {
+      const int r = e / OUT, o = e % OUT;
+      ds[r][o] = (r < nr && o < out) ? dY[(rt + r) * out + o] : 0.0f;
+    }
+    __syncthreads();
+    if (f >= h) continue;
+#pragma unroll 4
+    for (int r = 0; r < nr; ++r) {
+      const int64_t e = (rt + r) * h + f;
+      const float a = A2[e];
+      float d = 0.0f;
+#pragma unroll
+      for (int o = 0; o < OUT; ++o) {
+        d += w[o] * ds[r][o];
+        gw[o] += ds[r][o] * a;
+      }
+      d *= gelu_grad_f(Z2[e]);
+      dZ2[e] = d;
+      gb += (double)d;
+    }
+  }
+  if (f >= h) return;
+#pragma unroll
+  for (int o = 0; o < OUT; ++o)
+    if (o < out) pw[((int64_t)blockIdx.x * out + o) * h + f] = gw[o];
+  pb[(int64_t)blockIdx.x * h + f] = (float)gb;
+}
+
+// with dZ1 = dA1 gelu'(Z1): this block's partials of dW1 (in x h here) and db1
+template <int IN>
+__global__ __launch_bounds__(256) void mlp_back1_kernel(int64_t rows, int in, int h, int64_t rpb,
+                                                        const float* __restrict__ X,
+                                                        const float* __restrict__ Z1,
+                                                        const float* __restrict__ dA1,
+                                                        float* __restrict__ pw,
+                                                        float* __restrict__ pb) {
+  __shared__ float xs[MLP_TILE][IN];
+  const int t = threadIdx.x, f = blockIdx.y * 256 + t;
+  float gw[IN];
+  double gb = 0.0;
+#pragma unroll
+  for (int k = 0; k < IN; ++k) gw[k] = 0.0f;
+  const int64_t r0 = blockIdx.x * rpb, r1 = r0 + rpb < rows ? r0 + rpb : rows;
+  for (int64_t rt = r0; rt < r1; rt += MLP_TILE) {
+    const int nr = (int)(r1 - rt < MLP_TILE ? r1 - rt : MLP_TILE);
+    __syncthreads();
+    for (int e = t; e < MLP_TILE * IN; e += 256) {
+      const int r = e / IN, k = e % IN;
+      xs[r][k] = (r < nr && k < in) ? X[(rt + r) * in + k] : 0.0f;
+    }
+    __syncthreads();
+    if (f >= h) continue;
+#pragma unroll 4
+    for (int r = 0; r < nr; ++r) {
+      const int64_t e = (rt + r) * h + f;
+      const float d = dA1[e] * gelu_grad_f(Z1[e]);
+      gb += (double)d;
+#pragma unroll
+      for (int k = 0; k < IN; ++k) gw[k] += d * xs[r][k];
+    }
+  }
+  if (f >= h) return;
+#pragma unroll
+  for (int k = 0; k < IN; ++k)
+    if (k < in) pw[((int64_t)blockIdx.x * in + k) * h + f] = gw[k];
+  pb[(int64_t)blockIdx.x * h + f] = (float)gb;
+}
+
+struct GradSums {
+  const float *w1, *b1, *w3, *b2;   // nb partials each of in x h, h, out x h, h
+  const double* y;                  // ny partials of out + 1
+  int nb, ny, in, h, out;
+  float *gw1, *gb1, *gw3, *gb2, *gb3;
+  double* loss;
+};
+
+// every sum over partials in one launch: blockIdx.y = dW1, db1, dW3, db2, or
+// db3 and the loss; 64 outputs a block, sixteen waves over the partials
+__global__ __launch_bounds__(1024) void mlp_grad_sum_kernel(GradSums g) {
+  __shared__ double sh[16][64];
+  const int ei = threadIdx.x & 63, zi = threadIdx.x >> 6, job = blockIdx.y;
+  const int64_t e = (int64_t)blockIdx.x * 64 + ei;
+  const int64_t cnt = job == 0   ? (int64_t)g.in * g.h
+                      : job == 2 ? (int64_t)g.out * g.h
+                      : job == 4 ? g.out + 1
+                                 : g.h;
+  if ((int64_t)blockIdx.x * 64 >= cnt) return;   // whole block
+  double s = 0.0;
+  if (e < cnt) {
+    if (job == 4) {
+      for (int z = zi; z < g.ny; z += 16) s += g.y[(int64_t)z * cnt + e];
+    } else {
+      const float* p = (job == 0 ? g.w1 : job == 1 ? g.b1 : job == 2 ? g.w3 : g.b2) + e;
+      int z = zi;
+      for (; z + 112 < g.nb; z += 128) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = p[(int64_t)(z + 16 * q) * cnt];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += (double)v[q];
+      }
+      for (; z < g.nb; z += 16) s += (double)p[(int64_t)z * cnt];
+    }
+  }
+  sh[zi][ei] = s;
+  __syncthreads();
+  if (zi != 0 || e >= cnt) return;
+#pragma unroll
+  for (int q = 1; q < 16; ++q) s += sh[q][ei];
+  if (job == 0) g.gw1[(e % g.h) * g.in + e / g.h] = (float)s;
+  else if (job == 1) g.gb1[e] = (float)s;
+  else if (job == 2) g.gw3[e] = (float)s;
+  else if (job == 3) g.gb2[e] = (float)s;
+  else if (e < g.out) g.gb3[e] = (float)s;
+  else if (g.loss) *g.loss = s;
+}
+
+// rows per block for about two blocks per CU
+int64_t mlp_rpb(const itg_ctx* ctx, int64_t rows, int h) {
+  const int64_t nb = std::max<int64_t>(1, 2 * (int64_t)std::max(ctx->num_cu, 1) / ((h + 255) / 256));
+  return std::max<int64_t>(1, (rows + nb - 1) / nb);
+}
+
 __global__ void adam_kernel(int64_t n, float* __restrict__ p, const float* __restrict__ g,
                             float* __restrict__ m, float* __restrict__ v, float lr, float b1,
                             float b2, float eps, float c1, float c2) {
@@ -135,6 +419,21 @@ extern "C" int itg_mlp_forward(itg_ctx* ctx, int rows, int in, int h, int out, c
   float* A1 = acts + rh;
   float* Z2 = acts + 2 * rh;
   float* A2 = acts + 3 * rh;
+  if (mlp_outer_fused(in, out)) {
+    const int64_t rpb = mlp_rpb(ctx, rows, h);
+    const dim3 grid((unsigned)((rows + rpb - 1) / rpb), (h + 255) / 256);
+    hipStream_t st = ctx->stream;
+    if (in <= 16) mlp_layer1_kernel<16><<<grid, 256, 0, st>>>(rows, in, h, rpb, P + L.W1, P + L.b1, X, Z1, A1);
+    else mlp_layer1_kernel<32><<<grid, 256, 0, st>>>(rows, in, h, rpb, P + L.W1, P + L.b1, X, Z1, A1);
+    rc = itg_gemm_internal(ctx, ITG_F32, ITG_MODE_NATIVE, 'T', 'N', h, rows, h, 1.0, P + L.W2, h,
+                           A1, h, 0.0, Z2, h);
+    if (rc) return rc;
+    const unsigned nb = itg_blocks(rows, 8, 8 * (int64_t)std::max(ctx->num_cu, 1));
+    if (out <= 4) mlp_layer3_kernel<4><<<nb, 256, 0, st>>>(rows, h, out, P + L.b2, P + L.W3, P + L.b3, Z2, A2, Y);
+    else mlp_layer3_kernel<16><<<nb, 256, 0, st>>>(rows, h, out, P + L.b2, P + L.W3, P + L.b3, Z2, A2, Y);
+    ITG_LAUNCH_CHECK(ctx);
+    return ITG_OK;
+  }
   rc = itg_gemm_internal(ctx, ITG_F32, ITG_MODE_NATIVE, 'T', 'N', h, rows, in, 1.0, P + L.W1, in,
                          X, in, 0.0, Z1, h);
   if (rc) return rc;
@@ -368,6 +667,47 @@ extern "C" int itg_mlp_backward(itg_ctx* ctx, int rows, int in, int h, int out, 
   const float* Z2 = acts + 2 * rh;
   const float* A2 = acts + 3 * rh;
   void* ws;
+  if (mlp_outer_fused(in, out)) {
+    const int64_t rpb = mlp_rpb(ctx, rows, h), nbr = (rows + rpb - 1) / rpb;
+    const int64_t rpy = std::max<int64_t>(16, (rows + 511) / 512), ny = (rows + rpy - 1) / rpy;
+    const size_t floats = (size_t)ro + 2 * rh + (size_t)nbr * h * (in + out + 2);
+    rc = mlp_workspace(ctx, floats * sizeof(float) + (size_t)ny * (out + 1) * sizeof(double) + 256,
+                       &ws);
+    if (rc) return rc;
+    float* dY = (float*)ws;
+    float* dZ2 = dY + ro;
+    float* dA1 = dZ2 + rh;
+    float* pw1 = dA1 + rh;
+    float* pb1 = pw1 + nbr * h * in;
+    float* pw3 = pb1 + nbr * h;
+    float* pb2 = pw3 + nbr * h * out;
+    double* py = (double*)(((uintptr_t)(pb2 + nbr * h) + 255) & ~(uintptr_t)255);
+    hipStream_t st = ctx->stream;
+    const dim3 grid((unsigned)nbr, (h + 255) / 256);
+    mlp_mse_kernel<<<(unsigned)ny, 256, 0, st>>>(rows, out, rpy, Y, T, 1.0f / (float)ro, dY, py);
+    if (out <= 4) mlp_back3_kernel<4><<<grid, 256, 0, st>>>(rows, h, out, rpb, P + L.W3, dY, Z2, A2, dZ2, pw3, pb2);
+    else mlp_back3_kernel<16><<<grid, 256, 0, st>>>(rows, h, out, rpb, P + L.W3, dY, Z2, A2, dZ2, pw3, pb2);
+    ITG_LAUNCH_CHECK(ctx);
+    rc = itg_gemm_internal(ctx, ITG_F32, ITG_MODE_NATIVE, 'N', 'T', h, h, rows, 1.0, A1, h, dZ2, h,
+                           0.0, G + L.W2, h);
+    if (rc) return rc;
+    rc = itg_gemm_internal(ctx, ITG_F32, ITG_MODE_NATIVE, 'N', 'N', h, rows, h, 1.0, P + L.W2, h,
+                           dZ2, h, 0.0, dA1, h);
+    if (rc) return rc;
+    if (in <= 16) mlp_back1_kernel<16><<<grid, 256, 0, st>>>(rows, in, h, rpb, X, Z1, dA1, pw1, pb1);
+    else mlp_back1_kernel<32><<<grid, 256, 0, st>>>(rows, in, h, rpb, X, Z1, dA1, pw1, pb1);
+    const GradSums gs = {pw1, pb1, pw3, pb2, py, (int)nbr, (int)ny, in, h, out, G + L.W1,
+                         G + L.b1, G + L.W3, G + L.b2, G + L.b3,
+                         loss ? ctx->red_host : nullptr};
+    const int64_t most = (int64_t)h * std::max(in, out);
+    mlp_grad_sum_kernel<<<dim3((unsigned)((most + 63) / 64), 5), 1024, 0, st>>>(gs);
+    ITG_LAUNCH_CHECK(ctx);
+    if (loss) {
+      ITG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      *loss = ctx->red_host[0] / (double)ro;
+    }
+    return ITG_OK;
+  }
   size_t nb = 1024;
   rc = mlp_workspace(ctx, (size_t)(ro + 2 * rh) * sizeof(float) + nb * sizeof(double) + 256, &ws);
   if (rc) return rc;
