@@ -354,7 +354,9 @@ __global__ __launch_bounds__(256, 2) void gett_kernel(GettArgs g) {
 // FP64 storage with FP64 MFMA and FP32 storage with FP32 MFMA. TS x TS
 // tile per 256-thread workgroup (2 x 2 waves of TS/2 x TS/2, 16x16x4
 // blocks), K staged 16 deep through two LDS buffers with one barrier per
-// stage.
+// stage, the loads of two more stages in flight in registers (one in flight:
+// 4096^3 FP64 61.3 TFLOP/s, 66.1 now; FP32 125 and 130; a stage of a lone
+// 32 x 32 workgroup 0.44 us and 0.27, FP64).
 //
 // Bound: the matrix pipe, if the loader and the fragment reads stay out of
 // its way. A wave issues (TS/32)^2 products per 4 k, 64 (FP64) or 32 (FP32)
@@ -397,7 +399,7 @@ struct NativeLoader {
   int64_t kn[TAB ? NKO : 1]; // offsets of the next stage's k (!TAB: of its first)
   int kf;                    // KF: k of this thread in a stage; else its first k
   int klen;
-  T r[NPT];
+  T r[2][NPT];               // two stages in flight
 
   __device__ __forceinline__ void init(const T* X, int64_t r0, int64_t rows, const int64_t* tr,
                                        int64_t sr, const int64_t* tkk, int64_t skk, int64_t kbeg,
@@ -435,36 +437,36 @@ struct NativeLoader {
     }
   }
   // the stage at k0; stages are loaded in order
-  __device__ __forceinline__ void load(int k0) {
+  __device__ __forceinline__ void load(int k0, int set) {
     if (TAB || k0 + BK <= klen) {
 #pragma unroll
       for (int i = 0; i < NPT; ++i)
-        r[i] = p[KF ? i : 0][KF ? kn[0] : TAB ? kn[TAB ? i % NKO : 0] : kn[0] + (STEP * i) * sk];
+        r[set][i] = p[KF ? i : 0][KF ? kn[0] : TAB ? kn[TAB ? i % NKO : 0] : kn[0] + (STEP * i) * sk];
     } else {
 #pragma unroll
       for (int i = 0; i < NPT; ++i) {
         const int k = k0 + kf + (KF ? 0 : STEP * i);
-        r[i] = k < klen ? p[KF ? i : 0][k * sk] : (T)0;
+        r[set][i] = k < klen ? p[KF ? i : 0][k * sk] : (T)0;
       }
     }
     if constexpr (TAB) {
       if (k0 + BK > klen) {
 #pragma unroll
         for (int i = 0; i < NPT; ++i)
-          if (k0 + kf + (KF ? 0 : STEP * i) >= klen) r[i] = (T)0;
+          if (k0 + kf + (KF ? 0 : STEP * i) >= klen) r[set][i] = (T)0;
       }
       offsets(k0 + BK);
     } else {
       kn[0] += BK * sk;
     }
   }
-  __device__ __forceinline__ void store(T* s) const {
+  __device__ __forceinline__ void store(T* s, int set) const {
     const int t = threadIdx.x;
 #pragma unroll
     for (int i = 0; i < NPT; ++i) {
       const int m = KF ? t / BK + STEP * i : t % TS;
       const int k = KF ? kf : kf + STEP * i;
-      s[k * TS + (m ^ (native_sw<T>(k) & MASK))] = r[i];
+      s[k * TS + (m ^ (native_sw<T>(k) & MASK))] = r[set][i];
     }
   }
 };
@@ -506,19 +508,24 @@ __global__ __launch_bounds__(256, TS == 128 ? 2 : 4) void gett_native_kernel(Get
 
   const int lr = lane & 15, lg = lane >> 4;
   const int ma = wm * WH + WT * lr, nb = wn * WH + WT * lr;
-  la.load(0);
-  lb.load(0);
-  la.store(smem[0][0]);
-  lb.store(smem[0][1]);
+  la.load(0, 0);
+  lb.load(0, 0);
   if (BK < klen) {
-    la.load(BK);
-    lb.load(BK);
+    la.load(BK, 1);
+    lb.load(BK, 1);
+  }
+  la.store(smem[0][0], 0);
+  lb.store(smem[0][1], 0);
+  if (2 * BK < klen) {
+    la.load(2 * BK, 0);
+    lb.load(2 * BK, 0);
   }
   __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < klen; k0 += BK) {
-    const T* As = smem[buf][0];
-    const T* Bs = smem[buf][1];
+  // the stage at k0, P = its number mod 2
+  auto stage = [&](int k0, auto par) {
+    constexpr int P = decltype(par)::value;
+    const T* As = smem[P][0];
+    const T* Bs = smem[P][1];
     typedef typename NativeVec<T, WT>::vec vec;
     vec a[2], b[2];
     auto frag = [&](int kk) {
@@ -533,14 +540,14 @@ __global__ __launch_bounds__(256, TS == 128 ? 2 : 4) void gett_native_kernel(Get
       if (kk == 1) {
         // the first products are in the matrix pipe: store the next stage
         // (the other buffer was last read before the barrier that ended
-        // the previous stage) and start the loads of the one after
+        // the previous stage) and start the loads of the one two after it
         __builtin_amdgcn_sched_barrier(0);
         if (k0 + BK < klen) {
-          la.store(smem[buf ^ 1][0]);
-          lb.store(smem[buf ^ 1][1]);
-          if (k0 + 2 * BK < klen) {
-            la.load(k0 + 2 * BK);
-            lb.load(k0 + 2 * BK);
+          la.store(smem[P ^ 1][0], P ^ 1);
+          lb.store(smem[P ^ 1][1], P ^ 1);
+          if (k0 + 3 * BK < klen) {
+            la.load(k0 + 3 * BK, P ^ 1);
+            lb.load(k0 + 3 * BK, P ^ 1);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -558,7 +565,10 @@ __global__ __launch_bounds__(256, TS == 128 ? 2 : 4) void gett_native_kernel(Get
         }
     }
     __syncthreads();
-    buf ^= 1;
+  };
+  for (int k0 = 0; k0 < klen; k0 += 2 * BK) {
+    stage(k0, std::integral_constant<int, 0>());
+    if (k0 + BK < klen) stage(k0 + BK, std::integral_constant<int, 1>());
   }
 
   // lane holds D[q][lr] of each block, q = 4 lg + r (FP32) or 4 r + lg
@@ -1143,9 +1153,9 @@ static void native_kernel(itg_ctx* ctx, const GettArgs& g, dim3 grid, bool ak, b
 // what each further one adds; a split adds a launch and its partials'
 // traffic. Measured on MI355X (us; one workgroup per CU and many):
 //            FP64 lat  mf      FP32 lat  mf
-//   32 x 32       0.44 0.23         0.30 0.146
-//   64 x 64       0.97 0.55         0.50 0.31
-// 128 x 128          -    -         1.29 1.0
+//   32 x 32       0.27 0.175        0.21 0.108
+//   64 x 64       0.77 0.50         0.41 0.315
+// 128 x 128          -    -         1.23 1.05
 // FP64 at 128 x 128 gains nothing over 64 x 64 (59 against 61 TFLOP/s at
 // 4096^3: 64 cycles per product hide the smaller tile's reads) and rounds
 // worse, so it is not built. The estimates are within 15% of the measured
@@ -1159,8 +1169,8 @@ static NativeChoice choose_native(const itg_ctx* ctx, const GettArgs& g, bool f6
     int ts;
     double lat, mf;
   };
-  static const Tile t64[] = {{32, 0.44, 0.23}, {64, 0.97, 0.55}};
-  static const Tile t32[] = {{32, 0.30, 0.146}, {64, 0.50, 0.31}, {128, 1.29, 1.0}};
+  static const Tile t64[] = {{32, 0.27, 0.175}, {64, 0.77, 0.50}};
+  static const Tile t32[] = {{32, 0.21, 0.108}, {64, 0.41, 0.315}, {128, 1.23, 1.05}};
   const Tile* tiles = f64 ? t64 : t32;
   const int nt = f64 ? 2 : 3;
   const double cus = std::max(ctx->num_cu, 1);
