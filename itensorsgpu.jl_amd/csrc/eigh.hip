@@ -23,6 +23,7 @@
 #include <cstdlib>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "dc_core.h"
@@ -622,6 +623,259 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
       if (b == (l >> 4)) dl = q.x[b / 2][b];
     d[n - 1] = dl;
     tau[n - 1] = 0.0;
+  }
+}
+
+// -------------------------------------------- resident reduction (m <= 2560)
+// The trailing block of m = n - p <= 512 K rows and columns (every earlier
+// update applied, its lower triangle current) reduced by `cols` columns by
+// workgroups that keep it in registers: workgroup g owns rows 16 g .. 16 g + 15
+// (whole rows, both triangles), thread t of 512 columns t + 512 k, k < K.
+//
+// Bound: the latency of one exchange per column between the workgroups (write
+// to memory, poll, read); the rest is the chain of
+// three barriers and two sums over the block. The chip-wide kernels pay two
+// launches and three dependent passes over memory per column instead. A column
+// takes 3.1, 3.7, 4.5, 5.2 us for K = 1, 2, 3, 4 (8.2 to 13 before); whole
+// eigendecompositions: n = 512 3.68 -> 2.13 ms, 1000 8.3 -> 4.5, 2048 20.4 ->
+// 10.9, 2560 (K = 5) 18.9 -> 15.5 over K = 4 alone, 4096 61.6 -> 48.6.
+//
+// Column j, every workgroup alike: from a = A(:, j) (known to all) the norm,
+// the reflector v and tau; one pass over the workgroup's rows applies the
+// previous column's A -= v w^T + w v^T and forms y = A v; the workgroup
+// publishes y(r) and A(r, j + 1) for its rows, and reads both for all rows.
+// Then w = tau y - tau^2/2 (y^T v) v, and the next column is A(:, j + 1) -
+// v w(j+1) - w v(j+1): one exchange gives all that the next column needs, and
+// every workgroup computes the same bits from it.
+//
+// The exchange is data that validates itself: a slot holds MID_EMPTY until its
+// value is there (a result with these very bits is published with the last bit
+// flipped; both are NaNs). Three slots take turns: at column j a workgroup
+// empties its part of slot (j + 1) mod 3, last used at column j - 2; all that
+// read that have published column j - 1 since, which has just been gathered.
+// Values go through agent-scope atomics (past the L2 of the XCD); the emptying
+// store is waited for before the same thread publishes. A workgroup whose rows
+// are done leaves before it would gather (nothing waits for it any more).
+//
+// All workgroups have to be resident at once: at most 160 of one per CU. The
+// host lets one such reduction run at a time on a device. Against other
+// processes on it every wait is bounded by `limit` ticks (100 MHz): then
+// *stop is set, every workgroup leaves, and the host starts over without this
+// kernel.
+constexpr int MID_ROWS = 16, MID_MAX = 2560;
+constexpr unsigned long long MID_EMPTY = 0x7FF8A5A5C3C35A5AULL;
+typedef unsigned long long mid_t;
+
+__device__ __forceinline__ mid_t mid_get(const mid_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void mid_put(mid_t* p, mid_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void trd_mid_clear_kernel(mid_t* ring, int count, int* stop, bool first) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e < count) ring[e] = MID_EMPTY;
+  if (e == 0 && first) *stop = 0;
+}
+
+template <int K>
+__global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, int n, int p, int cols,
+                                                      double* __restrict__ d,
+                                                      double* __restrict__ e,
+                                                      double* __restrict__ tau, mid_t* ring,
+                                                      int* stop, long long limit) {
+  constexpr int R = MID_ROWS, MP = 512 * K;
+  __shared__ double red1[8], red2[8], part[8][R], ncol[R], rv[R], rw[R], sc[2];
+  __shared__ int bad;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int m = n - p, row0 = (int)blockIdx.x * R;
+  const bool writer = blockIdx.x + 1 == gridDim.x;   // its rows are the last ones done
+  double* Ap = A + (size_t)p * n + p;
+  double x[K][R];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = t + 512 * k;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int r = row0 + i, hi = r > c ? r : c, lo = r > c ? c : r;
+      x[k][i] = hi < m ? Ap[(size_t)lo * n + hi] : 0.0;
+    }
+  }
+  // a: column j; v, w: column j - 1's until the pass, then j's
+  double a[K], v[K], w[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = t + 512 * k;
+    a[k] = c < m ? Ap[c] : 0.0;
+    v[k] = w[k] = 0.0;
+  }
+  if (t < R) rv[t] = rw[t] = 0.0;
+  if (t == 0) bad = 0;
+  for (int j = 0; j < cols; ++j) {
+    mid_t* slot = ring + (size_t)(j % 3) * 2 * MP;
+    if (t < 2 * R && row0 + (t & (R - 1)) > j) {
+      mid_t* old = ring + (size_t)((j + 1) % 3) * 2 * MP;
+      mid_put(old + (t / R) * MP + row0 + (t & (R - 1)), MID_EMPTY);
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = t + 512 * k;
+      if (c >= j + 2) s += a[k] * a[k];   // a is 0 from m on
+      if (c == j + 1) sc[0] = a[k];
+    }
+    s = wave_sum(s);
+    if (lane == 0) red1[wv] = s;
+    __syncthreads();
+    const double alpha = sc[0];
+    const double xn2 = ((red1[0] + red1[1]) + (red1[2] + red1[3])) +
+                       ((red1[4] + red1[5]) + (red1[6] + red1[7]));
+    double beta = alpha, tv = 0.0, scale = 1.0;
+    if (xn2 != 0.0) {
+      beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
+      tv = (beta - alpha) / beta;
+      scale = 1.0 / (alpha - beta);
+    }
+    double vn[K], y[R];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = t + 512 * k;
+      vn[k] = c <= j ? 0.0 : c == j + 1 ? 1.0 : a[k] * scale;
+      if (writer && c == j) d[p + j] = a[k];
+    }
+    if (writer && t == 0) {
+      e[p + j] = beta;
+      tau[p + j] = tv;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const double pr = rv[i], qr = rw[i];
+      y[i] = 0.0;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        x[k][i] -= pr * w[k] + qr * v[k];
+        y[i] += x[k][i] * vn[k];
+      }
+    }
+    if (t == ((j + 1) & 511)) {
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (k == (j + 1) / 512) {
+#pragma unroll
+          for (int i = 0; i < R; ++i) ncol[i] = x[k][i];
+        }
+    }
+    fold_halves<R, 32>(y, lane);
+    const double z = fold_sum<2>(y[0]);
+    if ((lane & 3) == 0) part[wv][lane >> 2] = z;
+    __syncthreads();
+    if (t < 2 * R) {
+      const int i = t & (R - 1), r = row0 + i;
+      double q = ncol[i];
+      if (t < R)
+        q = ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) +
+            ((part[4][i] + part[5][i]) + (part[6][i] + part[7][i]));
+      // the emptying store above is done before this one starts
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (r > j && r < m) {
+        mid_t b = (mid_t)__double_as_longlong(q);
+        if (b == MID_EMPTY) b ^= 1;
+        mid_put(slot + (t / R) * MP + r, b);
+      }
+    }
+    // whole workgroup: no row after j + 1 and none to hand back
+    if (row0 + R - 1 <= j + 1 && row0 + R - 1 < cols) return;
+    mid_t yb[K], ab[K];
+    {
+      long long t0 = 0;
+      for (int spins = 0;; ++spins) {
+        bool all = true;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const int c = t + 512 * k;
+          yb[k] = ab[k] = 0;
+          if (c > j && c < m) {
+            yb[k] = mid_get(slot + c);
+            ab[k] = mid_get(slot + MP + c);
+            all = all && yb[k] != MID_EMPTY && ab[k] != MID_EMPTY;
+          }
+        }
+        if (all) break;
+        if (spins == 0) t0 = wall_clock64();
+        if ((spins & 63) == 63 || limit == 0) {
+          if (__hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
+              wall_clock64() - t0 >= limit) {
+            __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bad = 1;
+            break;
+          }
+        }
+      }
+    }
+    double g = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = t + 512 * k;
+      v[k] = vn[k];
+      w[k] = __longlong_as_double((long long)yb[k]);
+      a[k] = __longlong_as_double((long long)ab[k]);
+      g += c > j ? w[k] * v[k] : 0.0;
+      if (c == j + 1) sc[1] = w[k];
+    }
+    g = wave_sum(g);
+    if (lane == 0) red2[wv] = g;
+    __syncthreads();
+    if (bad) return;   // whole workgroup
+    if (writer) {
+      // only now, past the barrier: every workgroup has published, so has
+      // read the column that is overwritten
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int c = t + 512 * k;
+        if (c > j && c < m) Ap[(size_t)j * n + c] = v[k];
+      }
+    }
+    const double ytv = ((red2[0] + red2[1]) + (red2[2] + red2[3])) +
+                       ((red2[4] + red2[5]) + (red2[6] + red2[7]));
+    const double f = -0.5 * tv * tv * ytv, w1 = tv * sc[1] + f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = t + 512 * k;
+      w[k] = c > j ? tv * w[k] + f * v[k] : 0.0;
+      a[k] = c > j ? a[k] - (v[k] * w1 + w[k]) : 0.0;
+      if (c >= row0 && c < row0 + R) {
+        rv[c - row0] = v[k];
+        rw[c - row0] = w[k];
+      }
+    }
+  }
+  __syncthreads();
+  // the last update, and the rest back: row r's part right of the diagonal
+  // into column r
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = row0 + i;
+    const double pr = rv[i], qr = rw[i];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = t + 512 * k;
+      if (r >= cols && c >= r && c < m)
+        Ap[(size_t)r * n + c] = x[k][i] - (pr * w[k] + qr * v[k]);
+    }
+  }
+}
+
+// A's rows and columns from p on, to or from a copy
+__global__ void trd_copy_kernel(double* __restrict__ A, int n, int p, double* __restrict__ B,
+                                bool back) {
+  const int m = n - p;
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < (int64_t)m * m;
+       q += (int64_t)gridDim.x * blockDim.x) {
+    const int r = (int)(q % m), c = (int)(q / m);
+    double* x = A + (size_t)(p + c) * n + p + r;
+    if (back) *x = B[q];
+    else B[q] = *x;
   }
 }
 
@@ -1567,17 +1821,73 @@ static int eig_workspace(itg_ctx* ctx, size_t bytes, void** out) {
   return ITG_OK;
 }
 
+// From this many trailing rows on: the copy, the loads and the read-back cost
+// 31 us, a column of the chip-wide kernels 5 us more than one of these (n = 220
+// whole: 1045 us without, 934 with; even at six columns). Up to MID_MAX rows:
+// K = 6 would not fit the registers.
+constexpr int MID_MIN = TRD_TAIL + 8;
+
+// Columns p .. n - TRD_TAIL - 1 by the resident kernels, the trailing block
+// handed from one to the next as it shrinks; *ok = false if a wait ran out
+// (A as before the call).
+static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double* e, double* tau,
+                        double* copy, mid_t* ring, bool* ok) {
+  static std::mutex turn[64];   // one reduction at a time on a device
+  const char* env = getenv("ITG_TRD_WAIT_MS");
+  const long long limit = (env ? atoll(env) : 2000) * 100000LL;
+  int dev = 0;
+  ITG_HIP(ctx, hipGetDevice(&dev));
+  int* stop = (int*)(ring + 3 * 2 * MID_MAX);
+  hipStream_t st = ctx->stream;
+  const int m0 = n - p, p0 = p;
+  trd_copy_kernel<<<itg_blocks((int64_t)m0 * m0, 256, 8192), 256, 0, st>>>(A, n, p, copy, false);
+  int stopped = 0;
+  {
+    std::lock_guard<std::mutex> lock(turn[dev & 63]);
+    for (int end; p < n - TRD_TAIL; p = end) {
+      const int m = n - p, K = (m + 511) / 512;
+      end = K == 1 ? n - TRD_TAIL : n - 512 * (K - 1);
+      const int count = 3 * 2 * 512 * K, G = (m + MID_ROWS - 1) / MID_ROWS;
+      trd_mid_clear_kernel<<<(count + 255) / 256, 256, 0, st>>>(ring, count, stop, p == p0);
+      auto go = [&](auto kernel) {
+        kernel<<<G, 512, 0, st>>>(A, n, p, end - p, d, e, tau, ring, stop, limit);
+      };
+      if (K == 1) go(trd_mid_kernel<1>);
+      else if (K == 2) go(trd_mid_kernel<2>);
+      else if (K == 3) go(trd_mid_kernel<3>);
+      else if (K == 4) go(trd_mid_kernel<4>);
+      else go(trd_mid_kernel<5>);
+      ITG_LAUNCH_CHECK(ctx);
+    }
+    ITG_HIP(ctx, hipMemcpyAsync(&stopped, stop, sizeof(int), hipMemcpyDeviceToHost, st));
+    ITG_HIP(ctx, hipStreamSynchronize(st));
+  }
+  *ok = stopped == 0;
+  if (stopped) {
+    trd_copy_kernel<<<itg_blocks((int64_t)m0 * m0, 256, 8192), 256, 0, st>>>(A, n, p0, copy, true);
+    ITG_LAUNCH_CHECK(ctx);
+  }
+  return ITG_OK;
+}
+
 // Tridiagonalise A (n x n FP64, full symmetric storage) in place: d, e out;
 // reflectors left in A's strictly lower part (v_j(j+1) = 1 explicit), tau out.
 static int tridiagonalize(itg_ctx* ctx, int n, double* A, double* d, double* e, double* tau,
                           double* VW, double* Ypart, double* ab, double* pnorm, double* pyv,
-                          double* sc) {
+                          double* sc, double* copy, double* ring) {
   // VW = [V | W | V], n x NB each: the trailing update of a full panel is one
   // K = 2 NB product A22 -= [V W] [W V]^T
   double* Vp = VW;
   double* Wp = VW + (size_t)n * NB;
   double* V2 = VW + 2 * (size_t)n * NB;
+  bool resident = copy != nullptr;
   for (int p = 0, nbp; p < n; p += nbp) {
+    if (resident && n - p <= MID_MAX && n - p >= MID_MIN) {
+      int rc = trd_resident(ctx, n, p, A, d, e, tau, copy, (mid_t*)ring, &resident);
+      if (rc) return rc;
+      if (resident) p = n - TRD_TAIL;
+      resident = false;
+    }
     if (n - p <= TRD_TAIL) {
       // every earlier panel's update is applied: the rest in one block
       const int m = n - p;
@@ -1892,7 +2202,15 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   // 1. tridiagonalise
   if (cplx) rc = itg_zhetrd(ctx, n, Ain, d, e, ztau, zscr);
   else if (two) rc = eig2::reduce(ctx, n, A, d, e, eb);
-  else rc = tridiagonalize(ctx, n, A, d, e, tau, VW, Ypart, ab, pnorm, pyv, trd_sc);
+  else {
+    // the resident reduction reads its outcome back: not under capture, and
+    // with every CU its workgroups need
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    ITG_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
+    const bool resident = cap == hipStreamCaptureStatusNone && ctx->num_cu >= MID_MAX / MID_ROWS;
+    rc = tridiagonalize(ctx, n, A, d, e, tau, VW, Ypart, ab, pnorm, pyv, trd_sc,
+                        resident ? Qa : nullptr, Qb);
+  }
   if (rc) return rc;
   // 2. divide and conquer
   double *Q, *D;
