@@ -943,129 +943,107 @@ __global__ void bt_clear_upper_kernel(double* __restrict__ A, int n) {
   }
 }
 
-// All compact-WY factors at once: block b forms G = V_b^T V_b of panel b
-// (columns p = NB b .. p+nb, rows p+1..n-1, staged through LDS in 64-row
-// chunks) and runs the dlarft recurrence on it in LDS; T_b goes to
-// Tall[b * NB * NB] (nb x nb, column-major with leading dimension nb).
-__global__ __launch_bounds__(256) void bt_tall_kernel(const double* __restrict__ A, int n,
-                                                      int nrefl, const double* __restrict__ tau,
-                                                      double* __restrict__ Tall) {
-  __shared__ double Vs[64][NB + 1];
-  __shared__ double Gs[NB][NB + 1];
-  __shared__ double Ts[NB][NB + 1];
-  __shared__ double ts[NB];
-  __shared__ double tmp[NB];
-  const int t = threadIdx.x;
-  const int p = blockIdx.x * NB;
-  const int nb = min(NB, nrefl - p);
-  if (nb <= 0) return;
-  double g0 = 0.0, g1 = 0.0, g2 = 0.0, g3 = 0.0;   // pairs t, t+256, t+512, t+768
-  for (int r0 = p + 1; r0 < n; r0 += 64) {
-    __syncthreads();
-    for (int x = t; x < 64 * NB; x += 256) {
-      int rr = x % 64, c = x / 64, r = r0 + rr;
-      Vs[rr][c] = (r < n && c < nb) ? A[r + (size_t)(p + c) * n] : 0.0;
-    }
-    __syncthreads();
-    int rows = min(64, n - r0);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      int pr = t + 256 * q, ca = pr % NB, cb = pr / NB;
-      double s = 0.0;
-      for (int rr = 0; rr < rows; ++rr) s += Vs[rr][ca] * Vs[rr][cb];
-      if (q == 0) g0 += s; else if (q == 1) g1 += s; else if (q == 2) g2 += s; else g3 += s;
-    }
-  }
-  {
-    double gq[4] = {g0, g1, g2, g3};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      int pr = t + 256 * q;
-      Gs[pr % NB][pr / NB] = gq[q];
-      Ts[pr % NB][pr / NB] = 0.0;
-    }
-  }
-  if (t < nb) ts[t] = tau[p + t];
-  __syncthreads();
-  for (int i = 0; i < nb; ++i) {
-    if (t < i) tmp[t] = -ts[i] * Gs[t][i];
-    __syncthreads();
-    if (t < i) {
-      double acc = 0.0;
-      for (int m = t; m < i; ++m) acc += Ts[t][m] * tmp[m];
-      Ts[t][i] = acc;
-    }
-    if (t == i) Ts[i][i] = ts[i];
-    __syncthreads();
-  }
-  double* T = Tall + (size_t)blockIdx.x * NB * NB;
-  for (int e = t; e < nb * nb; e += 256) T[e] = Ts[e % nb][e / nb];
-}
-
-// X2 = T X for one panel: T nb x nb upper triangular, X nb x k (ld nb);
-// one thread per element, eight columns per block (rows along lanes)
-__global__ __launch_bounds__(256) void bt_apply_t_kernel(int nb, int k, const double* __restrict__ T,
-                                                         const double* __restrict__ X,
-                                                         double* __restrict__ X2) {
-  __shared__ double Tsh[NB * NB];
-  __shared__ double Xs[8][NB];
-  const int t = threadIdx.x, r = t % NB, cl = t / NB;
-  const int c = blockIdx.x * 8 + cl;
-  for (int e = t; e < nb * nb; e += 256) Tsh[e] = T[e];
-  Xs[cl][r] = (c < k && r < nb) ? X[(size_t)c * nb + r] : 0.0;
-  __syncthreads();
-  if (c >= k || r >= nb) return;
-  double s = 0.0;
-  for (int q = r; q < nb; ++q) s += Tsh[r + q * nb] * Xs[cl][q];
-  X2[(size_t)c * nb + r] = s;
-}
-
-// Back-transform of a group of BTG consecutive panels (up to BTG*NB
-// reflectors) at once. With Y = V_G^T U (the group's rows of U before the
-// group is applied) and the Gram matrix Gg = V_G^T V_G, the panels applied
-// last-to-first give X_b = Y_b - sum_{b' > b} Gg(b, b') X2_b' and
-// X2_b = T_b X_b; then U -= V_G X2 in one product. One block: 8 columns of
-// U x the 32 rows of the current panel; X2 of the later panels in LDS.
-constexpr int BTG = 4;
+// Back-transform of a group of up to BT_GROUP consecutive reflectors at once:
+// with Y = V^T U (the group's rows of U) and G = V^T V, U <- H_0 .. H_{b-1} U =
+// U - V X, X = T Y, where T is never formed: T^-1 = diag(1 / tau) + the strict
+// upper triangle of G (forward columnwise compact WY, any tau), so that
+// X_i = tau_i (Y_i - sum_{q>i} G(i, q) X_q).
+//
+// One workgroup per 16 columns of U, 16 rows of X a step, last to first: the
+// later rows' terms on MFMA, their k split over the four waves, then the
+// 16 x 16 triangle by its inverse (T of the 16 reflectors), formed beforehand
+// for all steps at once. Bound by latency: everything is loaded up front (the
+// fragments of G in registers) and a step is three barriers. 128 reflectors:
+// 14 us for 100 columns, 15 for 1000; with 32-row steps of dot products in LDS
+// and T formed by a kernel of its own 17 and 23, and for that kernel 46 (n =
+// 200) to 216 (n = 2048).
+constexpr int BT_GROUP = 128;
+typedef double btv_t __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void bt_group_solve_kernel(int nbg, int k,
                                                              const double* __restrict__ Y,
                                                              const double* __restrict__ Gg,
-                                                             const double* __restrict__ Tall,
+                                                             const double* __restrict__ tau,
                                                              double* __restrict__ X2) {
-  __shared__ double X2s[8][BTG * NB];
-  __shared__ double xs[8][NB];
-  __shared__ double Gs[NB][(BTG - 1) * NB + 1];   // Gg rows of panel b, later columns
-  __shared__ double Ts[NB][NB + 1];
-  const int t = threadIdx.x, r = t % NB, cl = t / NB;
-  const int c = blockIdx.x * 8 + cl;
-  const bool live = c < k;
-  const int npb = (nbg + NB - 1) / NB;
-  for (int b = npb - 1; b >= 0; --b) {
-    const int r0 = b * NB, nb = min(NB, nbg - r0), q0 = r0 + nb, nq = nbg - q0;
-    // stage Gg(r0.., q0..) and T_b (group-relative panel b)
-    for (int e = t; e < NB * nq; e += 256) {
-      int rr = e % NB, qq = e / NB;
-      Gs[rr][qq] = rr < nb ? Gg[(r0 + rr) + (size_t)(q0 + qq) * nbg] : 0.0;
+  constexpr int S = BT_GROUP / 16;
+  __shared__ double gs[S][257], Ts[S][16][17], xs[BT_GROUP][16], part[4][256], xt[256];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int lr = lane & 15, lg = lane >> 4, ti = t & 15, tc = t >> 4;
+  const int c = (int)blockIdx.x * 16 + tc;
+  btv_t f[S - 1][2];   // wave wv's fragments of G, S - 1 - b of step b used
+  double y[S];
+#pragma unroll
+  for (int b = 0; b < S; ++b) {
+    const int r = 16 * b + ti, q = 16 * b + tc;
+    y[b] = (c < k && r < nbg) ? Y[(size_t)c * nbg + r] : 0.0;
+    double g = 0.0;
+    if (ti < tc && q < nbg) g = Gg[r + (size_t)q * nbg];
+    if (ti == tc && q < nbg) g = tau[q];
+    gs[b][ti + 16 * tc] = g;
+  }
+#pragma unroll
+  for (int b = 0; b < S - 1; ++b)
+#pragma unroll
+    for (int u = 0; u < S - 1 - b; ++u) {
+      const int r = 16 * b + lr, q = 16 * (b + 1) + 4 * (wv + 4 * u) + lg;
+      f[b][u / 4][u % 4] = (r < nbg && q < nbg) ? Gg[r + (size_t)q * nbg] : 0.0;
     }
-    const double* T = Tall + (size_t)b * NB * NB;
-    for (int e = t; e < nb * nb; e += 256) Ts[e % nb][e / nb] = T[e];
-    __syncthreads();
-    double x = 0.0;
-    if (live && r < nb) {
-      x = Y[(size_t)c * nbg + r0 + r];
-      for (int qq = 0; qq < nq; ++qq) x -= Gs[r][qq] * X2s[cl][q0 + qq];
+  __syncthreads();
+  if (t < 16 * S) {
+    // column ti of step tc's T
+    const double* g = gs[tc];
+    double x[16];
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+      const double ta = g[i + 16 * i];
+      double s = 0.0;
+#pragma unroll
+      for (int q = i + 1; q < 16; ++q) s += g[i + 16 * q] * x[q];
+      x[i] = i == ti ? ta : -ta * s;
+      if (i > ti) x[i] = 0.0;
+      Ts[tc][i][ti] = x[i];
     }
-    xs[cl][r] = x;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int b = S - 1; b >= 0; --b) {
+    double x = y[b];
+    if (b < S - 1) {
+      btv_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int u = 0; u < S - 1 - b; ++u)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
+            f[b][u / 4][u % 4], xs[16 * (b + 1) + 4 * (wv + 4 * u) + lg][lr], acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[wv][4 * r + lg + 16 * lr] = acc[r];
+      __syncthreads();
+      x -= (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
+    }
+    xt[t] = x;
     __syncthreads();
-    if (live && r < nb) {
-      double v = 0.0;
-      for (int q = r; q < nb; ++q) v += Ts[r][q] * xs[cl][q];
-      X2s[cl][r0 + r] = v;
-      X2[(size_t)c * nbg + r0 + r] = v;
+    if (wv == 0) {
+      btv_t d = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(Ts[b][lr][4 * q + lg], xt[4 * q + lg + 16 * lr], d,
+                                                 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) xs[16 * b + 4 * r + lg][lr] = d[r];
     }
     __syncthreads();
   }
+  if (c >= k) return;
+#pragma unroll
+  for (int b = 0; b < S; ++b)
+    if (16 * b + ti < nbg) X2[(size_t)c * nbg + 16 * b + ti] = xs[16 * b + ti][tc];
+}
+
+// tau of every reflector from the panels' compact-WY factors (their diagonals)
+__global__ void bt_tau_kernel(const double* __restrict__ Tall, int nrefl, double* __restrict__ tau) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nrefl) return;
+  const int p = i / NB, nb = min(NB, nrefl - p * NB);
+  tau[i] = Tall[(size_t)p * NB * NB + (size_t)(i % NB) * (nb + 1)];
 }
 
 // --------------------------------------------------------- divide & conquer
@@ -2045,73 +2023,30 @@ static int tridiag_dc(itg_ctx* ctx, int n, const double* d, const double* e, dou
   return ITG_OK;
 }
 
-// U (n x k, FP64) <- Q U with Q = H_0 H_1 ... H_{nrefl-1}, reflectors stored
-// in A (ld n) as described at bt_build_v_kernel
-static int back_transform(itg_ctx* ctx, int n, int nrefl, int off, int k, const double* A,
-                          const double* tau, double* U, double* Vb, double* G, double* T,
-                          double* X, double* X2) {
-  if (nrefl < 1) return ITG_OK;
-  int last = ((nrefl - 1) / NB) * NB;
-  for (int p = last; p >= 0; p -= NB) {
-    int nbp = std::min(NB, nrefl - p);
-    int m2 = n - p - off;
-    if (nbp <= 0 || m2 <= 0) continue;
-    bt_build_v_kernel<<<itg_blocks((int64_t)n * nbp, 256, 4096), 256, 0, ctx->stream>>>(A, n, p, nbp, off, Vb);
-    ITG_LAUNCH_CHECK(ctx);
-    const double* V1 = Vb + (p + off);
-    int rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', nbp, nbp, m2, 1.0, V1, n,
-                               V1, n, 0.0, G, nbp);
-    if (rc) return rc;
-    bt_larft_kernel<<<1, 64, 0, ctx->stream>>>(nbp, G, tau + p, T);
-    ITG_LAUNCH_CHECK(ctx);
-    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', nbp, k, m2, 1.0, V1, n,
-                           U + (p + off), n, 0.0, X, nbp);
-    if (rc) return rc;
-    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', nbp, k, nbp, 1.0, T, nbp, X,
-                           nbp, 0.0, X2, nbp);
-    if (rc) return rc;
-    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', m2, k, nbp, -1.0, V1, n, X2,
-                           nbp, 1.0, U + (p + off), n);
-    if (rc) return rc;
-  }
-  return ITG_OK;
-}
-
-// U (n x k) <- Q U for Q = H_0 ... H_{n-off-1}, reflector j stored in
-// column j of A from row j + off on (the tridiagonalisation: off = 1, its
-// rows 0..j cleared here and every T formed up front by bt_tall_kernel; the
-// two-stage band reduction: off = its bandwidth, A already laid out and
-// Tall given). Groups of BTG panels go last-to-first: Y = V_G^T U,
-// Gg = V_G^T V_G, the group solve for X2, U -= V_G X2.
-static int back_transform_trd(itg_ctx* ctx, int n, int k, double* A, const double* tau,
-                              double* U, double* Tall, double* Y, double* X2, double* Gg,
-                              int off = 1, bool have_t = false) {
-  int nrefl = n - off;
+// U (m x k) <- H_0 ... H_{nrefl-1} U, reflector j in column j of A (leading
+// dimension m) from row j + off on, v(j + off) = 1 stored and zeros above
+// within its group. Groups of BT_GROUP reflectors go last to first: Y = V^T U,
+// G = V^T V, the group solve for X, U -= V X. `eye`: U is the identity's first
+// k = nrefl columns (columns before a group's first are still untouched).
+static int back_transform_groups(itg_ctx* ctx, int m, int nrefl, int off, int k, const double* A,
+                                 const double* tau, double* U, bool eye, double* Y, double* X2,
+                                 double* Gg) {
   if (nrefl < 1 || k < 1) return ITG_OK;
-  if (!have_t) {
-    bt_clear_upper_kernel<<<itg_blocks((int64_t)n * n, 256, 16384), 256, 0, ctx->stream>>>(A, n);
-    int npan = (nrefl + NB - 1) / NB;
-    bt_tall_kernel<<<npan, 256, 0, ctx->stream>>>(A, n, nrefl, tau, Tall);
-    ITG_LAUNCH_CHECK(ctx);
-  }
-  const int gsz = BTG * NB;
-  int ngrp = (nrefl + gsz - 1) / gsz;
-  for (int g = ngrp - 1; g >= 0; --g) {
-    int p0 = g * gsz;
-    int nbg = std::min(gsz, nrefl - p0);
-    int m2 = n - p0 - off;
-    const double* VG = A + (size_t)p0 * n + (p0 + off);   // rows p0+off.., columns p0..p0+nbg
-    int rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', nbg, k, m2, 1.0, VG, n,
-                               U + (p0 + off), n, 0.0, Y, nbg);
+  for (int p0 = (nrefl - 1) / BT_GROUP * BT_GROUP; p0 >= 0; p0 -= BT_GROUP) {
+    const int nbg = std::min(BT_GROUP, nrefl - p0);
+    const int m2 = m - p0 - off, c0 = eye ? p0 : 0, kc = k - c0;
+    const double* VG = A + (size_t)p0 * m + (p0 + off);   // rows p0+off.., columns p0..p0+nbg
+    double* UG = U + (size_t)c0 * m + (p0 + off);
+    int rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', nbg, kc, m2, 1.0, VG, m, UG,
+                               m, 0.0, Y, nbg);
     if (rc) return rc;
-    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', nbg, nbg, m2, 1.0, VG, n, VG,
-                           n, 0.0, Gg, nbg);
+    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', nbg, nbg, m2, 1.0, VG, m, VG,
+                           m, 0.0, Gg, nbg);
     if (rc) return rc;
-    bt_group_solve_kernel<<<(k + 7) / 8, 256, 0, ctx->stream>>>(
-        nbg, k, Y, Gg, Tall + (size_t)(p0 / NB) * NB * NB, X2);
+    bt_group_solve_kernel<<<(kc + 15) / 16, 256, 0, ctx->stream>>>(nbg, kc, Y, Gg, tau + p0, X2);
     ITG_LAUNCH_CHECK(ctx);
-    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', m2, k, nbg, -1.0, VG, n, X2,
-                           nbg, 1.0, U + (p0 + off), n);
+    rc = itg_gemm_internal(ctx, ITG_F64, ITG_MODE_NATIVE, 'N', 'N', m2, kc, nbg, -1.0, VG, m, X2,
+                           nbg, 1.0, UG, m);
     if (rc) return rc;
   }
   return ITG_OK;
@@ -2145,8 +2080,7 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   const bool two = !cplx && n >= TWO_STAGE_MIN && two_env && two_env[0] == '1';
   const size_t Tw = (size_t)(n + 63) / 64;   // tile rows of the tiled symv
   size_t bytes = (3 * nn + (f32 ? 2 * nn : 0)) * sizeof(double) + 3 * (size_t)n * NB * 8 +
-                 (2 * (size_t)BTG * NB * n + (size_t)BTG * NB * BTG * NB) * 8 +
-                 (size_t)((n + NB - 1) / NB) * NB * NB * 8 +
+                 (2 * (size_t)BT_GROUP * n + (size_t)BT_GROUP * BT_GROUP) * 8 +
                  (size_t)n * 8 * 26 + 4 * (size_t)n * NB * 8 + 4 * NB * NB * 8 + 64 * 1024 +
                  (Tw * n + Tw * (Tw + 1) / 2 + 64) * 8 + 64 * 256 +
                  ((size_t)n / POST_ROWS + 1) * 8 +
@@ -2158,8 +2092,7 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   Carver cv{(char*)ws};
   double* Qa = cv.take<double>(nn);
   double* Qb = cv.take<double>(nn);
-  // D&C merge vectors; afterwards the back-transform's compact-WY factors
-  double* Vbuf = cv.take<double>(std::max(nn, (size_t)((n + NB - 1) / NB) * NB * NB));
+  double* Vbuf = cv.take<double>(nn);   // D&C merge vectors
   // complex: A stays the caller's (complex) matrix, U a real n x k staging
   // buffer for the tridiagonal's eigenvectors
   double* A = f32 ? cv.take<double>(nn) : cplx ? nullptr : (double*)Ain;
@@ -2188,9 +2121,9 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   int64_t* tab = cv.take<int64_t>(n);
   double* Gm = cv.take<double>(NB * NB);
   double* Tm = cv.take<double>(NB * NB);
-  double* Ygrp = cv.take<double>((size_t)BTG * NB * n);
-  double* X2grp = cv.take<double>((size_t)BTG * NB * n);
-  double* Ggrp = cv.take<double>((size_t)BTG * NB * BTG * NB);
+  double* Ygrp = cv.take<double>((size_t)BT_GROUP * n);
+  double* X2grp = cv.take<double>((size_t)BT_GROUP * n);
+  double* Ggrp = cv.take<double>((size_t)BT_GROUP * BT_GROUP);
   double* out3 = cv.take<double>(4);
   eig2::Bufs eb{};
   if (two) eig2::carve(n, cv.take<double>(eig2::doubles_needed(n)), &eb);
@@ -2268,10 +2201,15 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   } else if (two) {
     rc = eig2::apply_q2(ctx, n, (int)k, U, eb);
     if (rc) return rc;
-    rc = back_transform_trd(ctx, n, (int)k, A, nullptr, U, eb.Tall, Ygrp, X2grp, Ggrp, eig2::SB,
-                            true);
+    static_assert(eig2::SB == NB, "panels of one width");
+    bt_tau_kernel<<<(n + 255) / 256, 256, 0, ctx->stream>>>(eb.Tall, n - eig2::SB, tau);
+    ITG_LAUNCH_CHECK(ctx);
+    rc = back_transform_groups(ctx, n, n - eig2::SB, eig2::SB, (int)k, A, tau, U, false, Ygrp,
+                               X2grp, Ggrp);
   } else {
-    rc = back_transform_trd(ctx, n, (int)k, A, tau, U, Vbuf, Ygrp, X2grp, Ggrp);
+    bt_clear_upper_kernel<<<itg_blocks((int64_t)n * n, 256, 16384), 256, 0, ctx->stream>>>(A, n);
+    ITG_LAUNCH_CHECK(ctx);
+    rc = back_transform_groups(ctx, n, n - 1, 1, (int)k, A, tau, U, false, Ygrp, X2grp, Ggrp);
   }
   if (rc) return rc;
   if (f32) {
@@ -2287,7 +2225,8 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
 // ====================================================================== QR
 // Householder QR (culinearalgebra.jl:110-121): reflectors of W = A column by
 // column, then Q = H_0...H_{r-1} [I; 0] by the same compact-WY
-// back-transform, R = triu(W).
+// back-transform, R = triu(W). Q of 2000 x 1000 in groups of 128 reflectors
+// takes 0.45 ms; panel by panel (16 reflectors, two launches each), 1.45.
 namespace {
 
 __global__ __launch_bounds__(1024) void qr_reflect_kernel(double* __restrict__ W, int m, int j,
@@ -2539,12 +2478,11 @@ __global__ __launch_bounds__(512) void qr_panel_kernel(double* __restrict__ A, i
   }
 }
 
-// C <- H^T C (trans) or H C, H = H_0 ... H_{w-1} = I - V T V^T of the panel in
-// A (m2 rows), in two launches over 256 rows x 16 columns per workgroup:
-// partials of Y = V^T C, and of G = V^T V as one more column block; then
-// X = T^T Y or T Y and C -= V X. T is not formed: T^-1 = diag(1 / tau) + the
-// upper triangle of G, so X comes from substitution, x_i = tau_i (y_i -
-// sum_{k<i} G(k, i) x_k) upwards for T^T, from k > i downwards for T. A memory
+// C <- H^T C, H = H_0 ... H_{w-1} = I - V T V^T of the panel in A (m2 rows), in
+// two launches over 256 rows x 16 columns per workgroup: partials of Y = V^T C,
+// and of G = V^T V as one more column block; then X = T^T Y and C -= V X. T is
+// not formed: T^-1 = diag(1 / tau) + the upper triangle of G, so X comes from
+// substitution, x_i = tau_i (y_i - sum_{k<i} G(k, i) x_k). A memory
 // round trip bounds either launch (the matrix is in the Infinity Cache, not
 // in the writer's L2), so a wave's loads all go out together and the grid
 // spans rows as well as columns: one workgroup per 16 columns, walking the
@@ -2577,7 +2515,7 @@ __global__ __launch_bounds__(256) void qr_y_kernel(const double* __restrict__ A,
 
 __global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict__ A, int ld,
                                                         int m2, int w,
-                                                        const double* __restrict__ tau, int trans,
+                                                        const double* __restrict__ tau,
                                                         double* __restrict__ C, int ldc, int nc,
                                                         const double* __restrict__ Yp) {
   __shared__ double ys[QW * 16], gs[QW * QW], xs[QW * 16], ts[QW];
@@ -2622,20 +2560,11 @@ __global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict
     double x[QW];   // y, less the terms of the x found so far
 #pragma unroll
     for (int i = 0; i < QW; ++i) x[i] = ys[i + QW * t];
-    if (trans) {
 #pragma unroll
-      for (int i = 0; i < QW; ++i) {
-        x[i] *= ts[i];
+    for (int i = 0; i < QW; ++i) {
+      x[i] *= ts[i];
 #pragma unroll
-        for (int k = i + 1; k < QW; ++k) x[k] -= gs[i + QW * k] * x[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = QW - 1; i >= 0; --i) {
-        x[i] *= ts[i];
-#pragma unroll
-        for (int k = 0; k < i; ++k) x[k] -= gs[k + QW * i] * x[i];
-      }
+      for (int k = i + 1; k < QW; ++k) x[k] -= gs[i + QW * k] * x[i];
     }
 #pragma unroll
     for (int i = 0; i < QW; ++i) xs[i + QW * t] = -x[i];
@@ -2661,6 +2590,16 @@ __global__ void qr_init_q_kernel(int m, int r, double* __restrict__ Q) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot;
        e += (int64_t)gridDim.x * blockDim.x)
     Q[e] = ((e % m) == (e / m)) ? 1.0 : 0.0;
+}
+
+// columns j < r of W: the reflectors, v(j) = 1 stored and zeros above
+__global__ void qr_unit_lower_kernel(int m, int r, double* __restrict__ W) {
+  int64_t tot = (int64_t)m * r;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    int i = (int)(e % m), j = (int)(e / m);
+    if (i <= j) W[e] = i == j ? 1.0 : 0.0;
+  }
 }
 
 __global__ void qr_extract_r_kernel(int m, int n, int r, const double* __restrict__ W,
@@ -2869,18 +2808,18 @@ static size_t qr_yp_doubles(int m, int nc) {
 }
 
 static int qr_block_apply(itg_ctx* ctx, const double* A, int ld, int m2, int w, const double* tau,
-                          int trans, double* C, int ldc, int nc, double* Yp) {
+                          double* C, int ldc, int nc, double* Yp) {
   const unsigned nb = (nc + 15) / 16, ns = (m2 + QR_ROWS - 1) / QR_ROWS;
   qr_y_kernel<<<dim3(nb + 1, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, C, ldc, nc, Yp);
-  qr_update_kernel<<<dim3(nb, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, tau, trans, C, ldc, nc,
+  qr_update_kernel<<<dim3(nb, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, tau, C, ldc, nc,
                                                           Yp);
   ITG_LAUNCH_CHECK(ctx);
   return ITG_OK;
 }
 
-// W (m x n, m <= QR_MAX_ROWS) <- its QR in dgeqrf's layout and Q (m x r,
-// column-major) formed; Yp holds qr_yp_doubles(m, n)
-static int qr_blocked(itg_ctx* ctx, int m, int n, double* W, double* Q, double* tau, double* Yp) {
+// W (m x n, m <= QR_MAX_ROWS) <- its QR in dgeqrf's layout; Yp holds
+// qr_yp_doubles(m, n)
+static int qr_blocked(itg_ctx* ctx, int m, int n, double* W, double* tau, double* Yp) {
   const int r = std::min(m, n);
   for (int p = 0; p < r; p += QW) {
     const int w = std::min(QW, r - p), m2 = m - p, nt = n - p - w;
@@ -2893,15 +2832,7 @@ static int qr_blocked(itg_ctx* ctx, int m, int n, double* W, double* Q, double* 
     else qr_panel_kernel<16, 4><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
     ITG_LAUNCH_CHECK(ctx);
     if (nt <= 0) continue;
-    int rc = qr_block_apply(ctx, A, m, m2, w, tau + p, 1, A + (size_t)w * m, m, nt, Yp);
-    if (rc) return rc;
-  }
-  qr_init_q_kernel<<<itg_blocks((int64_t)m * r, 256, 8192), 256, 0, ctx->stream>>>(m, r, Q);
-  ITG_LAUNCH_CHECK(ctx);
-  for (int p = (r - 1) / QW * QW; p >= 0; p -= QW) {
-    // columns before p are still those of the identity
-    int rc = qr_block_apply(ctx, W + (size_t)p * m + p, m, m - p, std::min(QW, r - p), tau + p, 0,
-                            Q + (size_t)p * m + p, m, r - p, Yp);
+    int rc = qr_block_apply(ctx, A, m, m2, w, tau + p, A + (size_t)w * m, m, nt, Yp);
     if (rc) return rc;
   }
   return ITG_OK;
@@ -2917,8 +2848,10 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   if (dtype == ITG_C64) return itg_c64_qr(ctx, m64, n64, Ain, Qo, Ro);
   int m = (int)m64, n = (int)n64, r = std::min(m, n);
   bool f32 = dtype == ITG_F32;
-  size_t bytes = ((size_t)m * n + (size_t)m * r + (size_t)r * n + (size_t)m * NB + 2 * (size_t)NB * n +
-                  2 * NB * NB + (size_t)r + (m <= QR_MAX_ROWS ? qr_yp_doubles(m, n) : 0) + 64) * sizeof(double) + 16 * 256;
+  const size_t nx = std::max((size_t)NB * n, (size_t)BT_GROUP * r);
+  size_t bytes = ((size_t)m * n + (size_t)m * r + (size_t)r * n + (size_t)m * NB + 2 * nx +
+                  (size_t)BT_GROUP * BT_GROUP + NB * NB + (size_t)r +
+                  (m <= QR_MAX_ROWS ? qr_yp_doubles(m, n) : 0) + 64) * sizeof(double) + 16 * 256;
   void* ws;
   int rc = eig_workspace(ctx, bytes, &ws);
   if (rc) return rc;
@@ -2927,26 +2860,21 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   double* Q = cv.take<double>((size_t)m * r);
   double* R = cv.take<double>((size_t)r * n);
   double* Vb = cv.take<double>((size_t)m * NB);
-  double* X = cv.take<double>((size_t)NB * n);
-  double* X2 = cv.take<double>((size_t)NB * n);
-  double* Gm = cv.take<double>(NB * NB);
+  double* X = cv.take<double>(nx);
+  double* X2 = cv.take<double>(nx);
+  double* Gm = cv.take<double>((size_t)BT_GROUP * BT_GROUP);
   double* Tm = cv.take<double>(NB * NB);
   double* tau = cv.take<double>(r);
   rc = itg_convert(ctx, (int64_t)m * n, dtype, Ain, ITG_F64, W);
   if (rc) return rc;
   if (m <= QR_MAX_ROWS) {
-    rc = qr_blocked(ctx, m, n, W, Q, tau, cv.take<double>(qr_yp_doubles(m, n)));
+    rc = qr_blocked(ctx, m, n, W, tau, cv.take<double>(qr_yp_doubles(m, n)));
     if (rc) return rc;
-    qr_extract_r_kernel<<<itg_blocks((int64_t)r * n, 256, 8192), 256, 0, ctx->stream>>>(m, n, r, W, R);
-    ITG_LAUNCH_CHECK(ctx);
-    rc = itg_convert(ctx, (int64_t)m * r, ITG_F64, Q, dtype, Qo);
-    if (rc) return rc;
-    return itg_convert(ctx, (int64_t)r * n, ITG_F64, R, dtype, Ro);
   }
   // taller matrices: blocked Householder QR (dgeqrf): each panel of NB columns is factored
   // column by column within itself, then the trailing columns take the
   // panel's block reflector, W2 -= V T^T (V^T W2), as GEMMs
-  for (int p = 0; p < r; p += NB) {
+  for (int p = 0; p < r && m > QR_MAX_ROWS; p += NB) {
     const int nbp = std::min(NB, r - p), pe = p + nbp;
     for (int j = p; j < pe; ++j) {
       qr_reflect_kernel<<<1, 1024, 0, ctx->stream>>>(W, m, j, tau);
@@ -2976,12 +2904,12 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
                            nbp, 1.0, W2, m);
     if (rc) return rc;
   }
+  qr_extract_r_kernel<<<itg_blocks((int64_t)r * n, 256, 8192), 256, 0, ctx->stream>>>(m, n, r, W, R);
+  qr_unit_lower_kernel<<<itg_blocks((int64_t)m * r, 256, 8192), 256, 0, ctx->stream>>>(m, r, W);
   qr_init_q_kernel<<<itg_blocks((int64_t)m * r, 256, 8192), 256, 0, ctx->stream>>>(m, r, Q);
   ITG_LAUNCH_CHECK(ctx);
-  rc = back_transform(ctx, m, r, 0, r, W, tau, Q, Vb, Gm, Tm, X, X2);
+  rc = back_transform_groups(ctx, m, r, 0, r, W, tau, Q, true, X, X2, Gm);
   if (rc) return rc;
-  qr_extract_r_kernel<<<itg_blocks((int64_t)r * n, 256, 8192), 256, 0, ctx->stream>>>(m, n, r, W, R);
-  ITG_LAUNCH_CHECK(ctx);
   rc = itg_convert(ctx, (int64_t)m * r, ITG_F64, Q, dtype, Qo);
   if (rc) return rc;
   return itg_convert(ctx, (int64_t)r * n, ITG_F64, R, dtype, Ro);
