@@ -626,11 +626,12 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
   }
 }
 
-// -------------------------------------------- resident reduction (m <= 2560)
+// -------------------------------------------- resident reduction (m <= 3072)
 // The trailing block of m = n - p <= 512 K rows and columns (every earlier
 // update applied, its lower triangle current) reduced by `cols` columns by
-// workgroups that keep it in registers: workgroup g owns rows 16 g .. 16 g + 15
-// (whole rows, both triangles), thread t of 512 columns t + 512 k, k < K.
+// workgroups that keep it in registers: workgroup g owns rows R g .. R g + R - 1
+// (whole rows, both triangles; R = 16, for K = 6 12, which the registers still
+// hold), thread t of 512 columns t + 512 k, k < K.
 //
 // Bound: the latency of one exchange per column between the workgroups (write
 // to memory, poll, read); the rest is the chain of
@@ -638,7 +639,8 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
 // launches and three dependent passes over memory per column instead. A column
 // takes 3.1, 3.7, 4.5, 5.2 us for K = 1, 2, 3, 4 (8.2 to 13 before); whole
 // eigendecompositions: n = 512 3.68 -> 2.13 ms, 1000 8.3 -> 4.5, 2048 20.4 ->
-// 10.9, 2560 (K = 5) 18.9 -> 15.5 over K = 4 alone, 4096 61.6 -> 48.6.
+// 10.9, 4096 61.6 -> 48.6 with K up to 5, then 47.5 -> 43.1 with K = 6 (n = 3000
+// 23.5 -> 18.9).
 //
 // Column j, every workgroup alike: from a = A(:, j) (known to all) the norm,
 // the reflector v and tau; one pass over the workgroup's rows applies the
@@ -657,12 +659,12 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
 // store is waited for before the same thread publishes. A workgroup whose rows
 // are done leaves before it would gather (nothing waits for it any more).
 //
-// All workgroups have to be resident at once: at most 160 of one per CU. The
+// All workgroups have to be resident at once: at most 256, one per CU. The
 // host lets one such reduction run at a time on a device. Against other
 // processes on it every wait is bounded by `limit` ticks (100 MHz): then
 // *stop is set, every workgroup leaves, and the host starts over without this
 // kernel.
-constexpr int MID_ROWS = 16, MID_MAX = 2560;
+constexpr int MID_MAX = 3072;
 constexpr unsigned long long MID_EMPTY = 0x7FF8A5A5C3C35A5AULL;
 typedef unsigned long long mid_t;
 
@@ -679,14 +681,14 @@ __global__ void trd_mid_clear_kernel(mid_t* ring, int count, int* stop, bool fir
   if (e == 0 && first) *stop = 0;
 }
 
-template <int K>
+template <int K, int R>
 __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, int n, int p, int cols,
                                                       double* __restrict__ d,
                                                       double* __restrict__ e,
                                                       double* __restrict__ tau, mid_t* ring,
                                                       int* stop, long long limit) {
-  constexpr int R = MID_ROWS, MP = 512 * K;
-  __shared__ double red1[8], red2[8], part[8][R], ncol[R], rv[R], rw[R], sc[2];
+  constexpr int MP = 512 * K;
+  __shared__ double red1[8], red2[8], part[8][16], ncol[R], rv[R], rw[R], sc[2];
   __shared__ int bad;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int m = n - p, row0 = (int)blockIdx.x * R;
@@ -714,9 +716,9 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
   if (t == 0) bad = 0;
   for (int j = 0; j < cols; ++j) {
     mid_t* slot = ring + (size_t)(j % 3) * 2 * MP;
-    if (t < 2 * R && row0 + (t & (R - 1)) > j) {
+    if (t < 2 * R && row0 + t % R > j && row0 + t % R < m) {
       mid_t* old = ring + (size_t)((j + 1) % 3) * 2 * MP;
-      mid_put(old + (t / R) * MP + row0 + (t & (R - 1)), MID_EMPTY);
+      mid_put(old + (t / R) * MP + row0 + t % R, MID_EMPTY);
     }
     double s = 0.0;
 #pragma unroll
@@ -737,7 +739,7 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
       tv = (beta - alpha) / beta;
       scale = 1.0 / (alpha - beta);
     }
-    double vn[K], y[R];
+    double vn[K], y[16];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int c = t + 512 * k;
@@ -766,12 +768,14 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
           for (int i = 0; i < R; ++i) ncol[i] = x[k][i];
         }
     }
-    fold_halves<R, 32>(y, lane);
+#pragma unroll
+    for (int i = R; i < 16; ++i) y[i] = 0.0;
+    fold_halves<16, 32>(y, lane);
     const double z = fold_sum<2>(y[0]);
     if ((lane & 3) == 0) part[wv][lane >> 2] = z;
     __syncthreads();
     if (t < 2 * R) {
-      const int i = t & (R - 1), r = row0 + i;
+      const int i = t % R, r = row0 + i;
       double q = ncol[i];
       if (t < R)
         q = ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) +
@@ -1802,7 +1806,7 @@ static int eig_workspace(itg_ctx* ctx, size_t bytes, void** out) {
 // From this many trailing rows on: the copy, the loads and the read-back cost
 // 31 us, a column of the chip-wide kernels 5 us more than one of these (n = 220
 // whole: 1045 us without, 934 with; even at six columns). Up to MID_MAX rows:
-// K = 6 would not fit the registers.
+// the registers of 256 CUs hold no more.
 constexpr int MID_MIN = TRD_TAIL + 8;
 
 // Columns p .. n - TRD_TAIL - 1 by the resident kernels, the trailing block
@@ -1812,7 +1816,7 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
                         double* copy, mid_t* ring, bool* ok) {
   static std::mutex turn[64];   // one reduction at a time on a device
   const char* env = getenv("ITG_TRD_WAIT_MS");
-  const long long limit = (env ? atoll(env) : 2000) * 100000LL;
+  const long long limit = (env ? atoll(env) : 50) * 100000LL;
   int dev = 0;
   ITG_HIP(ctx, hipGetDevice(&dev));
   int* stop = (int*)(ring + 3 * 2 * MID_MAX);
@@ -1825,16 +1829,18 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
     for (int end; p < n - TRD_TAIL; p = end) {
       const int m = n - p, K = (m + 511) / 512;
       end = K == 1 ? n - TRD_TAIL : n - 512 * (K - 1);
-      const int count = 3 * 2 * 512 * K, G = (m + MID_ROWS - 1) / MID_ROWS;
+      const int count = 3 * 2 * 512 * K;
       trd_mid_clear_kernel<<<(count + 255) / 256, 256, 0, st>>>(ring, count, stop, p == p0);
-      auto go = [&](auto kernel) {
-        kernel<<<G, 512, 0, st>>>(A, n, p, end - p, d, e, tau, ring, stop, limit);
+      auto go = [&](auto kernel, int rows) {
+        kernel<<<(m + rows - 1) / rows, 512, 0, st>>>(A, n, p, end - p, d, e, tau, ring, stop,
+                                                      limit);
       };
-      if (K == 1) go(trd_mid_kernel<1>);
-      else if (K == 2) go(trd_mid_kernel<2>);
-      else if (K == 3) go(trd_mid_kernel<3>);
-      else if (K == 4) go(trd_mid_kernel<4>);
-      else go(trd_mid_kernel<5>);
+      if (K == 1) go(trd_mid_kernel<1, 16>, 16);
+      else if (K == 2) go(trd_mid_kernel<2, 16>, 16);
+      else if (K == 3) go(trd_mid_kernel<3, 16>, 16);
+      else if (K == 4) go(trd_mid_kernel<4, 16>, 16);
+      else if (K == 5) go(trd_mid_kernel<5, 16>, 16);
+      else go(trd_mid_kernel<6, 12>, 12);
       ITG_LAUNCH_CHECK(ctx);
     }
     ITG_HIP(ctx, hipMemcpyAsync(&stopped, stop, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -2140,7 +2146,7 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
     // with every CU its workgroups need
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     ITG_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
-    const bool resident = cap == hipStreamCaptureStatusNone && ctx->num_cu >= MID_MAX / MID_ROWS;
+    const bool resident = cap == hipStreamCaptureStatusNone && ctx->num_cu >= MID_MAX / 12;
     rc = tridiagonalize(ctx, n, A, d, e, tau, VW, Ypart, ab, pnorm, pyv, trd_sc,
                         resident ? Qa : nullptr, Qb);
   }
