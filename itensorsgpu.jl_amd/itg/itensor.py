@@ -431,7 +431,7 @@ def svd(A, Linds, maxdim=None, mindim=1, cutoff=0.0, absolute_cutoff=False,
     dt = _dtype_name(A.data)
     Ut = ITensor(Li + [u], U[: m * k])
     Vt = ITensor(Ri + [v], V[: n * k])
-    St = itensor(np.diag(s), u, v, dtype=dt).roc()
+    St = ITensor((u, v), ops.diag_dense(S, k, dt))
     return Ut, St, Vt, Spectrum(s ** 2, te)
 
 

@@ -657,7 +657,7 @@ def _replacebond_complex(phi, m, n, ortho, maxdim, mindim, cutoff, drho, noise, 
         U, S, V, k, terr, _ = ops.svd_trunc(ops.copy(phi), m, n, maxdim=maxdim, mindim=mindim,
                                             cutoff=cut)
         s = ops.to_host(S)[:k]
-        Sd = ops.to_device(np.ravel(np.diag(s).astype(np.complex128), order="F"), "complex128")
+        Sd = ops.diag_dense(S, k, "complex128")
         Vh, _ = ops.permute(_bra(V[: n * k]), (n, k), (1, 0))          # k x n
         if ortho == "left":
             A = U[: m * k].clone()
@@ -727,7 +727,7 @@ def replacebond(psi, b, phi, pdims, ortho, maxdim, mindim, cutoff, drho=None, no
         U, S, V, k, terr, _ = ops.svd_trunc(work, m, n, maxdim=maxdim, mindim=mindim,
                                             cutoff=0.0 if cutoff is None else cutoff)
         s = ops.to_host(S)[:k]
-        Sd = ops.to_device(np.ravel(np.diag(s), order="F"), dt)
+        Sd = ops.diag_dense(S, k, dt)
         if ortho == "left":
             A = U[: m * k].clone()
             B = ops.empty(k * n, dt)

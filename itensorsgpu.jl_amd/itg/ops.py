@@ -218,6 +218,16 @@ def diag_contract(D, dimsD, labelsD, B, dimsB, labelsB, labelsC, uniform=None, a
     return out, dimsC
 
 
+def diag_dense(s, k, dtype):
+    """The dense k x k matrix with s[:k] (device, FP64) on its diagonal, built
+    on the device: at k = 2048 the host's copy took 6 ms to fill and send."""
+    if k == 0:
+        return empty(0, dtype)
+    d = s[:k] if dtype == "float64" else convert(s[:k], dtype)
+    one = fill(empty(1, dtype), 1.0)
+    return diag_contract(d, (k, k), [1, 2], one, (), (), [1, 2], dtype=dtype)[0]
+
+
 def hadamard(x, y, out=None):
     """out = x .* y element-wise."""
     out = out if out is not None else empty(x.numel(), dtype_name(x))
