@@ -2453,9 +2453,10 @@ struct QrPanel {
   }
 };
 
-template <int RPT, int CW>
-__global__ __launch_bounds__(512) void qr_panel_kernel(double* __restrict__ A, int ld, int m2,
-                                                       int w, double* __restrict__ tau) {
+// load(x, c0): columns c0 .. c0 + CW - 1 of the panel
+template <int RPT, int CW, typename F>
+__device__ __forceinline__ void qr_panel(double* A, int ld, int m2, int w, double* tau,
+                                         F&& load) {
   __shared__ double red[2][8][16], rowv[2][16], ts[QW];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   QrPanel<RPT, CW> q;
@@ -2472,10 +2473,7 @@ __global__ __launch_bounds__(512) void qr_panel_kernel(double* __restrict__ A, i
   q.wave = wave;
   q.buf = 0;
   for (int c0 = 0; c0 < w; c0 += CW) {
-#pragma unroll
-    for (int c = 0; c < CW; ++c)
-#pragma unroll
-      for (int a = 0; a < RPT; ++a) q.x[a][c] = qr_c(A, ld, m2, w, t + 512 * a, c0 + c);
+    load(q.x, c0);
     constexpr int LOG = CW == 16 ? 4 : CW == 8 ? 3 : 2;
     for (int j = 0; j < c0; ++j) q.template apply<LOG>(j);
     // the columns in hand halve as they are finished
@@ -2491,6 +2489,18 @@ __global__ __launch_bounds__(512) void qr_panel_kernel(double* __restrict__ A, i
     if (j < w) q.template factor<2>(j, min(w, j + 4));
     __syncthreads();   // the next turn reads what was stored
   }
+}
+
+template <int RPT, int CW>
+__global__ __launch_bounds__(512) void qr_panel_kernel(double* __restrict__ A, int ld, int m2,
+                                                       int w, double* __restrict__ tau) {
+  qr_panel<RPT, CW>(A, ld, m2, w, tau, [&](double (&x)[RPT][CW], int c0) {
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int a = 0; a < RPT; ++a)
+        x[a][c] = qr_c(A, ld, m2, w, (int)threadIdx.x + 512 * a, c0 + c);
+  });
 }
 
 // C <- H^T C, H = H_0 ... H_{w-1} = I - V T V^T of the panel in A (m2 rows), in
@@ -2528,48 +2538,33 @@ __global__ __launch_bounds__(256) void qr_y_kernel(const double* __restrict__ A,
       (ys[0][t] + ys[1][t]) + (ys[2][t] + ys[3][t]);
 }
 
-__global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict__ A, int ld,
-                                                        int m2, int w,
-                                                        const double* __restrict__ tau,
-                                                        double* __restrict__ C, int ldc, int nc,
-                                                        const double* __restrict__ Yp) {
-  __shared__ double ys[QW * 16], gs[QW * QW], xs[QW * 16], ts[QW];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int lr = lane & 15, lg = lane >> 4;
-  const int cols = min(16, nc - (int)blockIdx.x * 16);
-  C += (size_t)blockIdx.x * 16 * ldc;
-  // this wave's four 16-row blocks: loads and stores run along the rows (the
-  // product is issued transposed)
-  const int b0 = (int)blockIdx.y * QR_ROWS + 64 * wave;
-  double vb[4][4];
-  d4v_t z[4];   // C(l, 4 r + lg)
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      vb[u][q] = qr_v(A, ld, m2, w, b0 + 16 * u + lr, 4 * q + lg);
-      z[u][q] = qr_c(C, ldc, m2, cols, b0 + 16 * u + lr, 4 * q + lg);
-    }
+// -X(i, c) of columns 16 cb .. into xs (i + QW c), from the ns partials of Y
+// and G; LDS ys, gs and ts, blocks of at least 256 threads
+__device__ __forceinline__ void qr_coefficients(const double* __restrict__ Yp, int cb, int nb,
+                                                int ns, int w, const double* __restrict__ tau,
+                                                double* ys, double* gs, double* ts, double* xs) {
+  const int t = threadIdx.x;
   if (t < QW) ts[t] = t < w ? tau[t] : 0.0;
-  double y = 0.0, g = 0.0;
-  const size_t nb = gridDim.x + 1;
-  for (int q0 = 0; q0 < (int)gridDim.y; q0 += 8) {
-    double yq[8], gq[8];
+  if (t < 256) {
+    double y = 0.0, g = 0.0;
+    for (int q0 = 0; q0 < ns; q0 += 8) {
+      double yq[8], gq[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const size_t s = min(q0 + q, (int)gridDim.y - 1);
-      yq[q] = Yp[(s * nb + blockIdx.x) * 256 + t];
-      gq[q] = Yp[(s * nb + gridDim.x) * 256 + t];
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q)
-      if (q0 + q < (int)gridDim.y) {
-        y += yq[q];
-        g += gq[q];
+      for (int q = 0; q < 8; ++q) {
+        const size_t s = min(q0 + q, ns - 1);
+        yq[q] = Yp[(s * (nb + 1) + cb) * 256 + t];
+        gq[q] = Yp[(s * (nb + 1) + nb) * 256 + t];
       }
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (q0 + q < ns) {
+          y += yq[q];
+          g += gq[q];
+        }
+    }
+    ys[t] = y;
+    gs[t] = g;
   }
-  ys[t] = y;
-  gs[t] = g;
   __syncthreads();
   if (t < 16) {
     double x[QW];   // y, less the terms of the x found so far
@@ -2585,19 +2580,133 @@ __global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict
     for (int i = 0; i < QW; ++i) xs[i + QW * t] = -x[i];
   }
   __syncthreads();
-  double xa[4];   // -X(4 q + lg, lr), the left operand X^T(column, k)
+}
+
+// rows b0 .. b0 + 63 of A's panel and of a 16-column block of C for one wave:
+// loads and stores run along the rows (the product is issued transposed)
+struct QrRows {
+  double vb[4][4];
+  d4v_t z[4];   // C(l, 4 r + lg)
+  __device__ __forceinline__ void load(const double* __restrict__ A, int ld, int m2, int w,
+                                       const double* C, int ldc, int cols, int b0, int lr, int lg) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) xa[q] = xs[(4 * q + lg) + QW * lr];
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int l = b0 + 16 * u + lr;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      z[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[q], vb[u][q], z[u], 0, 0, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (l < m2 && 4 * r + lg < cols) C[l + (size_t)(4 * r + lg) * ldc] = z[u][r];
+      for (int q = 0; q < 4; ++q) {
+        vb[u][q] = qr_v(A, ld, m2, w, b0 + 16 * u + lr, 4 * q + lg);
+        z[u][q] = qr_c(C, ldc, m2, cols, b0 + 16 * u + lr, 4 * q + lg);
+      }
   }
+  __device__ __forceinline__ void update(const double* xs, double* C, int ldc, int m2, int cols,
+                                         int b0, int lr, int lg) {
+    double xa[4];   // -X(4 q + lg, lr), the left operand X^T(column, k)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) xa[q] = xs[(4 * q + lg) + QW * lr];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int l = b0 + 16 * u + lr;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        z[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[q], vb[u][q], z[u], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (l < m2 && 4 * r + lg < cols) C[l + (size_t)(4 * r + lg) * ldc] = z[u][r];
+    }
+  }
+};
+
+__global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict__ A, int ld,
+                                                        int m2, int w,
+                                                        const double* __restrict__ tau,
+                                                        double* C, int ldc, int nc,
+                                                        const double* __restrict__ Yp) {
+  __shared__ double ys[QW * 16], gs[QW * QW], xs[QW * 16], ts[QW];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int cols = min(16, nc - (int)blockIdx.x * 16);
+  const int b0 = (int)blockIdx.y * QR_ROWS + 64 * wave;
+  C += (size_t)blockIdx.x * 16 * ldc;
+  QrRows q;
+  q.load(A, ld, m2, w, C, ldc, cols, b0, lr, lg);
+  qr_coefficients(Yp, blockIdx.x, gridDim.x, gridDim.y, w, tau, ys, gs, ts, xs);
+  q.update(xs, C, ldc, m2, cols, b0, lr, lg);
+}
+
+// The update, and the next panel (C's first block of columns, from row QW on)
+// factored in the same launch: workgroup 0 updates that block in the registers
+// it factors it in, while the others (512 rows x 16 columns each) update the
+// rest. A panel takes longer than the update beside it (33 against 14 us),
+// which is hidden: 34 us a panel, 2000 x 1000 3.92 -> 3.14 ms.
+template <int RPT, int CW>
+__global__ __launch_bounds__(512) void qr_step_kernel(const double* A, int ld, int m2,
+                                                      const double* __restrict__ tau, double* C,
+                                                      int nc, const double* __restrict__ Yp, int ns,
+                                                      int wn, double* tau_next) {
+  __shared__ double ys[QW * 16], gs[QW * QW], xs[QW * 16], ts[QW];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lr = lane & 15, lg = lane >> 4, nb = (nc + 15) / 16;
+  if (blockIdx.x > 0) {
+    const int nr = (m2 + 511) / 512;
+    const bool top = blockIdx.x + 1 == gridDim.x;   // the panel's block: R's rows only
+    const int cb = top ? 0 : 1 + ((int)blockIdx.x - 1) / nr;
+    const int cols = min(16, nc - cb * 16);
+    const int b0 = top ? 64 * wave : ((int)blockIdx.x - 1) % nr * 512 + 64 * wave;
+    C += (size_t)cb * 16 * ld;
+    QrRows q;
+    q.load(A, ld, m2, QW, C, ld, cols, b0, lr, lg);
+    qr_coefficients(Yp, cb, nb, ns, QW, tau, ys, gs, ts, xs);
+    q.update(xs, C, ld, top ? min(QW, m2) : m2, cols, b0, lr, lg);
+    return;
+  }
+  const int cols = min(16, nc);
+  constexpr int VC = 8 / RPT;   // reflectors a turn
+  qr_panel<RPT, CW>(C + QW, ld, m2 - QW, wn, tau_next, [&](double (&x)[RPT][CW], int c0) {
+    // row QW + t + 512 a of the panel and of C; every load is clamped
+    int l[RPT];
+#pragma unroll
+    for (int a = 0; a < RPT; ++a) l[a] = min(QW + t + 512 * a, m2 - 1);
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+      const double* cc = C + (size_t)min(c0 + c, cols - 1) * ld;
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) x[a][c] = cc[l[a]];
+    }
+    if (c0 == 0) qr_coefficients(Yp, 0, nb, ns, QW, tau, ys, gs, ts, xs);
+    double v[RPT][VC];
+#pragma unroll
+    for (int i = 0; i < VC; ++i)
+#pragma unroll
+      for (int a = 0; a < RPT; ++a) v[a][i] = A[l[a] + (size_t)i * ld];
+    // VC reflectors a turn, the next turn's loads in flight
+#pragma unroll 1
+    for (int i0 = 0; i0 < QW; i0 += VC) {
+      double vn[RPT][VC];
+      const double* an = A + (size_t)min(i0 + VC, QW - VC) * ld;
+#pragma unroll
+      for (int i = 0; i < VC; ++i)
+#pragma unroll
+        for (int a = 0; a < RPT; ++a) vn[a][i] = an[l[a] + (size_t)i * ld];
+#pragma unroll
+      for (int c = 0; c < CW; ++c) {
+#pragma unroll
+        for (int i = 0; i < VC; ++i) {
+          const double f = xs[i0 + i + QW * ((c0 + c) & 15)];
+#pragma unroll
+          for (int a = 0; a < RPT; ++a) x[a][c] += v[a][i] * f;
+        }
+        if (c % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // or every f is read up front
+      }
+#pragma unroll
+      for (int a = 0; a < RPT; ++a)
+#pragma unroll
+        for (int i = 0; i < VC; ++i) v[a][i] = vn[a][i];
+    }
+#pragma unroll
+    for (int a = 0; a < RPT; ++a)
+#pragma unroll
+      for (int c = 0; c < CW; ++c)
+        if (QW + t + 512 * a >= m2 || c0 + c >= wn) x[a][c] = 0.0;
+  });
 }
 
 __global__ void qr_init_q_kernel(int m, int r, double* __restrict__ Q) {
@@ -2822,33 +2931,44 @@ static size_t qr_yp_doubles(int m, int nc) {
   return (size_t)((m + QR_ROWS - 1) / QR_ROWS) * ((nc + 15) / 16 + 1) * 256;
 }
 
-static int qr_block_apply(itg_ctx* ctx, const double* A, int ld, int m2, int w, const double* tau,
-                          double* C, int ldc, int nc, double* Yp) {
-  const unsigned nb = (nc + 15) / 16, ns = (m2 + QR_ROWS - 1) / QR_ROWS;
-  qr_y_kernel<<<dim3(nb + 1, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, C, ldc, nc, Yp);
-  qr_update_kernel<<<dim3(nb, ns), 256, 0, ctx->stream>>>(A, ld, m2, w, tau, C, ldc, nc,
-                                                          Yp);
-  ITG_LAUNCH_CHECK(ctx);
-  return ITG_OK;
-}
-
 // W (m x n, m <= QR_MAX_ROWS) <- its QR in dgeqrf's layout; Yp holds
 // qr_yp_doubles(m, n)
 static int qr_blocked(itg_ctx* ctx, int m, int n, double* W, double* tau, double* Yp) {
   const int r = std::min(m, n);
+  hipStream_t st = ctx->stream;
+  // rows a thread x columns a turn: at most 64 doubles of the panel
+  auto panel = [&](double* A, int rows, int w, double* tp) {
+    if (rows <= 1024) qr_panel_kernel<2, 16><<<1, 512, 0, st>>>(A, m, rows, w, tp);
+    else if (rows <= 2048) qr_panel_kernel<4, 16><<<1, 512, 0, st>>>(A, m, rows, w, tp);
+    else if (rows <= 4096) qr_panel_kernel<8, 8><<<1, 512, 0, st>>>(A, m, rows, w, tp);
+    else qr_panel_kernel<16, 4><<<1, 512, 0, st>>>(A, m, rows, w, tp);
+  };
+  panel(W, m, std::min(QW, r), tau);
+  ITG_LAUNCH_CHECK(ctx);
   for (int p = 0; p < r; p += QW) {
     const int w = std::min(QW, r - p), m2 = m - p, nt = n - p - w;
+    if (nt <= 0) break;
     double* A = W + (size_t)p * m + p;
-    hipStream_t st = ctx->stream;
-    // rows a thread x columns a turn: at most 64 doubles of the panel
-    if (m2 <= 1024) qr_panel_kernel<2, 16><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
-    else if (m2 <= 2048) qr_panel_kernel<4, 16><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
-    else if (m2 <= 4096) qr_panel_kernel<8, 8><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
-    else qr_panel_kernel<16, 4><<<1, 512, 0, st>>>(A, m, m2, w, tau + p);
+    double* C = A + (size_t)w * m;
+    const int nb = (nt + 15) / 16, ns = (m2 + QR_ROWS - 1) / QR_ROWS;
+    qr_y_kernel<<<dim3(nb + 1, ns), 256, 0, st>>>(A, m, m2, w, C, m, nt, Yp);
+    const int pn = p + QW, rows = m - pn, wn = std::min(QW, r - pn);
+    auto step = [&](auto kernel) {
+      kernel<<<2 + (nb - 1) * ((m2 + 511) / 512), 512, 0, st>>>(A, m, m2, tau + p, C, nt, Yp, ns, wn,
+                                                                tau + pn);
+    };
+    // past 4096 rows the panel's registers leave no room for the update
+    if (wn <= 0 || rows > 4096) {
+      qr_update_kernel<<<dim3(nb, ns), 256, 0, st>>>(A, m, m2, w, tau + p, C, m, nt, Yp);
+      if (wn > 0) panel(C + QW, rows, wn, tau + pn);
+    } else if (rows <= 1024) {
+      step(qr_step_kernel<2, 16>);
+    } else if (rows <= 2048) {
+      step(qr_step_kernel<4, 16>);
+    } else {
+      step(qr_step_kernel<8, 8>);
+    }
     ITG_LAUNCH_CHECK(ctx);
-    if (nt <= 0) continue;
-    int rc = qr_block_apply(ctx, A, m, m2, w, tau + p, A + (size_t)w * m, m, nt, Yp);
-    if (rc) return rc;
   }
   return ITG_OK;
 }
