@@ -645,10 +645,11 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
 // to memory, poll, read); the rest is the chain of
 // three barriers and two sums over the block. The chip-wide kernels pay two
 // launches and three dependent passes over memory per column instead. A column
-// takes 3.1, 3.7, 4.5, 5.2 us for K = 1, 2, 3, 4 (8.2 to 13 before); whole
-// eigendecompositions: n = 512 3.68 -> 2.13 ms, 1000 8.3 -> 4.5, 2048 20.4 ->
-// 10.9, 4096 61.6 -> 48.6 with K up to 5, then 47.5 -> 43.1 with K = 6 (n = 3000
-// 23.5 -> 18.9).
+// takes 2.8, 3.4, 4.2, 4.9 us for K = 1, 2, 3, 4 (8.2 to 13 before; 0.3 more
+// where the slot is emptied before the column and not while its exchange is
+// under way); whole eigendecompositions: n = 512 3.7 -> 1.9 ms, 1000 8.3 -> 4.1,
+// 2048 20.4 -> 10.1, 3000 23.5 -> 18.4 by K = 6. A workgroup's 16 values go out
+// as one store: sixteen by the lane that holds them took 15% longer.
 //
 // Column j, every workgroup alike: from a = A(:, j) (known to all) the norm,
 // the reflector v and tau; one pass over the workgroup's rows applies the
@@ -660,11 +661,12 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
 //
 // The exchange is data that validates itself: a slot holds MID_EMPTY until its
 // value is there (a result with these very bits is published with the last bit
-// flipped; both are NaNs). Three slots take turns: at column j a workgroup
-// empties its part of slot (j + 1) mod 3, last used at column j - 2; all that
-// read that have published column j - 1 since, which has just been gathered.
+// flipped; both are NaNs). Four slots take turns: at column j a workgroup
+// empties its part of slot (j + 2) mod 4, last used at column j - 2; all that
+// read that have published column j - 1 since, which was gathered before.
 // Values go through agent-scope atomics (past the L2 of the XCD); the emptying
-// store is waited for before the same thread publishes. A workgroup whose rows
+// stores are waited for before the barrier that comes before the next column
+// is published, so whoever has seen that one sees them. A workgroup whose rows
 // are done leaves before it would gather (nothing waits for it any more).
 //
 // All workgroups have to be resident at once: at most 256, one per CU. The
@@ -723,11 +725,7 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
   if (t < R) rv[t] = rw[t] = 0.0;
   if (t == 0) bad = 0;
   for (int j = 0; j < cols; ++j) {
-    mid_t* slot = ring + (size_t)(j % 3) * 2 * MP;
-    if (t < 2 * R && row0 + t % R > j && row0 + t % R < m) {
-      mid_t* old = ring + (size_t)((j + 1) % 3) * 2 * MP;
-      mid_put(old + (t / R) * MP + row0 + t % R, MID_EMPTY);
-    }
+    mid_t* slot = ring + (j & 3) * 2 * MP;
     double s = 0.0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -788,14 +786,16 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
       if (t < R)
         q = ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) +
             ((part[4][i] + part[5][i]) + (part[6][i] + part[7][i]));
-      // the emptying store above is done before this one starts
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if (r > j && r < m) {
         mid_t b = (mid_t)__double_as_longlong(q);
         if (b == MID_EMPTY) b ^= 1;
         mid_put(slot + (t / R) * MP + r, b);
       }
     }
+    // two columns ahead: done, and past a barrier, before the next column is
+    // published
+    if (wv == 7 && lane < 2 * R && row0 + lane % R > j && row0 + lane % R < m)
+      mid_put(ring + ((j + 2) & 3) * 2 * MP + (lane / R) * MP + row0 + lane % R, MID_EMPTY);
     // whole workgroup: no row after j + 1 and none to hand back
     if (row0 + R - 1 <= j + 1 && row0 + R - 1 < cols) return;
     mid_t yb[K], ab[K];
@@ -825,6 +825,7 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
         }
       }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the emptying stores
     double g = 0.0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -1827,7 +1828,7 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
   const long long limit = (env ? atoll(env) : 50) * 100000LL;
   int dev = 0;
   ITG_HIP(ctx, hipGetDevice(&dev));
-  int* stop = (int*)(ring + 3 * 2 * MID_MAX);
+  int* stop = (int*)(ring + 4 * 2 * MID_MAX);
   hipStream_t st = ctx->stream;
   const int m0 = n - p, p0 = p;
   trd_copy_kernel<<<itg_blocks((int64_t)m0 * m0, 256, 8192), 256, 0, st>>>(A, n, p, copy, false);
@@ -1837,7 +1838,7 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
     for (int end; p < n - TRD_TAIL; p = end) {
       const int m = n - p, K = (m + 511) / 512;
       end = K == 1 ? n - TRD_TAIL : n - 512 * (K - 1);
-      const int count = 3 * 2 * 512 * K;
+      const int count = 4 * 2 * 512 * K;
       trd_mid_clear_kernel<<<(count + 255) / 256, 256, 0, st>>>(ring, count, stop, p == p0);
       auto go = [&](auto kernel, int rows) {
         kernel<<<(m + rows - 1) / rows, 512, 0, st>>>(A, n, p, end - p, d, e, tau, ring, stop,
