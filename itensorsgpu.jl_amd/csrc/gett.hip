@@ -72,6 +72,21 @@ __device__ __forceinline__ void tile_coords(int64_t tilesM, int64_t tilesN, int6
   tn = in / gsize;
 }
 
+// Band products (square C, tiles tm <= tn + 1 only): the live tiles alone are
+// numbered, column by column, and each XCD takes an equal run of them. With
+// the full grid's numbering the dead tiles left some XCDs idle, and half the
+// work took as long as all of it (4096^3 FP64: 2240 us, 1240 now).
+__host__ __device__ inline int64_t band_tiles(int64_t T) { return T * (T + 1) / 2 + T - 1; }
+__device__ __forceinline__ bool band_coords(int64_t T, int64_t& tm, int64_t& tn) {
+  const int64_t lid = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  if (lid >= band_tiles(T)) return false;
+  tn = (int64_t)((sqrt(9.0 + 8.0 * (double)lid) - 3.0) * 0.5);
+  while (tn * (tn + 3) / 2 > lid) --tn;
+  while ((tn + 1) * (tn + 4) / 2 <= lid) ++tn;
+  tm = lid - tn * (tn + 3) / 2;
+  return true;
+}
+
 // Epilogue of gett_kernel's 128 x 128 tile (2 x 2 waves of 4 x 4 blocks):
 // lane holds D[4*lg + r][lr] of each 16x16 block
 template <typename T>
@@ -488,8 +503,11 @@ __global__ __launch_bounds__(256, TS == 128 ? 2 : 4) void gett_native_kernel(Get
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   int64_t tm, tn;
-  tile_coords(g.tilesM, g.tilesN, tm, tn);
-  if (g.band && tm > tn + 1) return;   // whole workgroup, before any barrier
+  if (g.band) {
+    if (!band_coords(g.tilesM, tm, tn)) return;   // whole workgroup, before any barrier
+  } else {
+    tile_coords(g.tilesM, g.tilesN, tm, tn);
+  }
   const int64_t m0 = tm * TS, n0 = tn * TS;
   const int64_t kbeg = (int64_t)blockIdx.z * g.kchunk;
   const int klen = (int)(kbeg + g.kchunk < g.K ? g.kchunk : g.K - kbeg);
@@ -1207,7 +1225,7 @@ static int launch_native(itg_ctx* ctx, GettArgs& g, bool ak, bool bk) {
   NativeChoice c = choose_native(ctx, g, F64);
   g.tilesM = (g.M + c.ts - 1) / c.ts;
   g.tilesN = (g.N + c.ts - 1) / c.ts;
-  const int64_t tiles = g.tilesM * g.tilesN;
+  const int64_t tiles = g.band ? (band_tiles(g.tilesM) + 7) / 8 * 8 : g.tilesM * g.tilesN;
   if (tiles > 0x7fffffff) return itg_fail(ctx, ITG_EUNSUPPORTED, "contraction too large");
   // a workgroup counts its k in 32 bits
   constexpr int64_t kMaxChunk = (int64_t)1 << 30;
@@ -1261,6 +1279,44 @@ static int launch_gett(itg_ctx* ctx, int dtype, int mode, GettArgs& g, bool ak, 
   }
   if (mode == ITG_MODE_BF16X3) return launch_gett_t<float, ITG_MODE_BF16X3>(ctx, g, ak, bk);
   return launch_native<float>(ctx, g, ak, bk);
+}
+
+// C(r, c) = C(c, r) for r < c from the lower triangle, through 32 x 32 LDS
+// tiles (block (bi, bj) writes the upper tile at rows bi, columns bj >= bi)
+template <typename T>
+__global__ __launch_bounds__(256) void mirror_lower_kernel(int64_t n, T* __restrict__ C,
+                                                           int64_t ldc) {
+  __shared__ T t[32][33];
+  const int64_t bi = blockIdx.x, bj = blockIdx.y;
+  if (bj < bi) return;
+  for (int yy = threadIdx.y; yy < 32; yy += 8) {
+    int64_t r = bj * 32 + threadIdx.x, c = bi * 32 + yy;
+    if (r < n && c < n) t[yy][threadIdx.x] = C[r + c * ldc];
+  }
+  __syncthreads();
+  for (int yy = threadIdx.y; yy < 32; yy += 8) {
+    int64_t r = bi * 32 + threadIdx.x, c = bj * 32 + yy;
+    if (r < n && c < n && r < c) C[r + c * ldc] = t[threadIdx.x][yy];
+  }
+}
+
+static int mirror_lower(itg_ctx* ctx, int dtype, int64_t n, void* C, int64_t ldc) {
+  dim3 grid((unsigned)((n + 31) / 32), (unsigned)((n + 31) / 32));
+  if (dtype == ITG_F64)
+    mirror_lower_kernel<double><<<grid, dim3(32, 8), 0, ctx->stream>>>(n, (double*)C, ldc);
+  else
+    mirror_lower_kernel<float><<<grid, dim3(32, 8), 0, ctx->stream>>>(n, (float*)C, ldc);
+  ITG_LAUNCH_CHECK(ctx);
+  return ITG_OK;
+}
+
+// Whether C = alpha A A^T (n x n) is computed as its lower triangle (and one
+// tile band), mirrored: a band with fewer 64 x 64 tiles than CUs is no faster
+// than the whole product, which can split K. FP64, us, band against whole:
+// 1024 x 1024: 58 / 59, 512 x 2048: 103 / 39, 256 x 256: 20 / 12; on the other
+// side 1500 x 1500: 121 / 150, 2048 x 2048: 220 / 255, 4096 x 4096: 1240 / 1820.
+static bool band_wins(const itg_ctx* ctx, int mode, int64_t n) {
+  return mode != ITG_MODE_NATIVE || band_tiles((n + 63) / 64) >= std::max(ctx->num_cu, 1);
 }
 
 // The library does not split K: a product with fewer 64 x 64 tiles than half
@@ -1395,8 +1451,19 @@ extern "C" int itg_contract(itg_ctx* ctx, int dtype, int mode, int rA, const int
   g.tBn = tp(p->oBn); g.tCm = tp(p->oCm); g.tCn = tp(p->oCn);
   g.alpha = alpha;
   g.beta = beta;
-  if (!g.tAm && !g.tAk && !g.tBk && !g.tBn && !g.tCm && !g.tCn &&
-      itg_libgemm_ok(ctx, dtype, mode, g.M, g.N, g.K) && !split_k_wins(ctx, g.M, g.N, g.K)) {
+  const bool plain = !g.tAm && !g.tAk && !g.tBk && !g.tBn && !g.tCm && !g.tCn;
+  // a tensor with itself over the same modes (a density matrix): half of it
+  // is computed
+  if (plain && g.A == g.B && g.M == g.N && g.sAm == g.sBn && g.sAk == g.sBk &&
+      std::min(g.sCm, g.sCn) == 1 && std::max(g.sCm, g.sCn) >= g.M && mode == ITG_MODE_NATIVE &&
+      alpha != 0.0 && beta == 0.0 && g.M >= 256 && band_wins(ctx, mode, g.M)) {
+    g.sCm = std::max(g.sCm, g.sCn);
+    g.sCn = 1;
+    g.band = 1;
+    const int rc = launch_gett(ctx, dtype, mode, g, p->akfast, p->bkfast);
+    return rc ? rc : mirror_lower(ctx, dtype, g.M, C, g.sCm);
+  }
+  if (plain && itg_libgemm_ok(ctx, dtype, mode, g.M, g.N, g.K) && !split_k_wins(ctx, g.M, g.N, g.K)) {
     int rc = contract_on_lib(ctx, g);
     if (rc != 1) return rc;
   }
@@ -1440,25 +1507,6 @@ int itg_gemm_internal(itg_ctx* ctx, int dtype, int mode, char ta, char tb, int64
   return launch_gett(ctx, dtype, mode, g, ak, bk);
 }
 
-// C(r, c) = C(c, r) for r < c from the lower triangle, through 32 x 32 LDS
-// tiles (block (bi, bj) writes the upper tile at rows bi, columns bj >= bi)
-template <typename T>
-__global__ __launch_bounds__(256) void mirror_lower_kernel(int64_t n, T* __restrict__ C,
-                                                           int64_t ldc) {
-  __shared__ T t[32][33];
-  const int64_t bi = blockIdx.x, bj = blockIdx.y;
-  if (bj < bi) return;
-  for (int yy = threadIdx.y; yy < 32; yy += 8) {
-    int64_t r = bj * 32 + threadIdx.x, c = bi * 32 + yy;
-    if (r < n && c < n) t[yy][threadIdx.x] = C[r + c * ldc];
-  }
-  __syncthreads();
-  for (int yy = threadIdx.y; yy < 32; yy += 8) {
-    int64_t r = bi * 32 + threadIdx.x, c = bj * 32 + yy;
-    if (r < n && c < n && r < c) C[r + c * ldc] = t[threadIdx.x][yy];
-  }
-}
-
 extern "C" int itg_gemm(itg_ctx* ctx, int dtype, int mode, char ta, char tb, int64_t m, int64_t n,
                         int64_t k, double alpha, const void* A, int64_t lda, const void* B,
                         int64_t ldb, double beta, void* C, int64_t ldc) {
@@ -1471,24 +1519,10 @@ extern "C" int itg_gemm(itg_ctx* ctx, int dtype, int mode, char ta, char tb, int
   const bool tn = (ta == 'T' || ta == 't') && (tb == 'N' || tb == 'n');
   if (A == B && lda == ldb && m == n && m >= 256 && k > 0 && beta == 0.0 && alpha != 0.0 &&
       (nt || tn)) {
-    // C = alpha A A^T (or A^T A), the density matrix of a bond: the lower
-    // triangle (and one tile band) on MFMA, the rest mirrored, so C is
-    // exactly symmetric
-    int rc;
-    if (lda >= (nt ? m : k) && itg_libgemm_ok(ctx, dtype, mode, m, n, k))
-      rc = itg_libsyrk_lower(ctx, nt ? 'N' : 'T', m, k, alpha, (const double*)A, lda, (double*)C,
-                             ldc);
-    else
-      rc = itg_gemm_internal(ctx, dtype, mode, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C,
-                             ldc, true);
-    if (rc) return rc;
-    dim3 grid((unsigned)((m + 31) / 32), (unsigned)((m + 31) / 32));
-    if (dtype == ITG_F64)
-      mirror_lower_kernel<double><<<grid, dim3(32, 8), 0, ctx->stream>>>(m, (double*)C, ldc);
-    else
-      mirror_lower_kernel<float><<<grid, dim3(32, 8), 0, ctx->stream>>>(m, (float*)C, ldc);
-    ITG_LAUNCH_CHECK(ctx);
-    return ITG_OK;
+    // C = alpha A A^T (or A^T A), the density matrix of a bond, exactly symmetric
+    const int rc = itg_gemm_internal(ctx, dtype, mode, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta,
+                                     C, ldc, band_wins(ctx, mode, m));
+    return rc ? rc : mirror_lower(ctx, dtype, m, C, ldc);
   }
   return itg_gemm_internal(ctx, dtype, mode, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }

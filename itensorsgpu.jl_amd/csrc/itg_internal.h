@@ -131,14 +131,11 @@ void itg_plan_cache_clear(itg_ctx* ctx);
 // Plain FP64 GEMMs on the vendor library (libgemm.hip). itg_libgemm_ok says
 // whether a native FP64 product of this size may go there (not while the
 // stream is being captured, not inside a no-alloc call, dimensions in 32
-// bits); itg_libgemm is column-major C = alpha op(A) op(B) + beta C and
-// itg_libsyrk the lower triangle of C = alpha op(A) op(A)^T.
+// bits); itg_libgemm is column-major C = alpha op(A) op(B) + beta C.
 bool itg_libgemm_ok(itg_ctx* ctx, int dtype, int mode, int64_t m, int64_t n, int64_t k);
 int itg_libgemm(itg_ctx* ctx, char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha,
                 const double* A, int64_t lda, const double* B, int64_t ldb, double beta,
                 double* C, int64_t ldc);
-int itg_libsyrk_lower(itg_ctx* ctx, char trans, int64_t n, int64_t k, double alpha,
-                      const double* A, int64_t lda, double* C, int64_t ldc);
 void itg_libgemm_free(itg_ctx* ctx);
 // Event bracket of one launch for itg_timing: t = itg_tstart(ctx, kind)
 // before the launch, itg_tstop(ctx, t, kind, flops, bytes) after it (no-ops

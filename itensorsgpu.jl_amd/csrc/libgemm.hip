@@ -1,10 +1,10 @@
-// Plain FP64 GEMMs on the vendor library (rocBLAS). On the products of this
-// path the library's FP64 MFMA kernels run at 61-76 TFLOP/s (4096^3,
-// 8192x2048x10240, 10240x8192x2048) against 34 TFLOP/s for the GETT kernel,
-// whose point is the permutation fused into its loads: contractions whose
-// modes group into plain column-major matrices, and itg_gemm itself, come
-// here; the rest stay on GETT. Products inside a stream capture or a
-// no-alloc call stay on GETT too (the library may allocate its workspace).
+// Plain FP64 GEMMs on the vendor library (rocBLAS). On large products its FP64
+// MFMA kernels run at 61-76 TFLOP/s (4096^3, 8192x2048x10240,
+// 10240x8192x2048) against 66 for the contraction kernel, whose point is the
+// permutation fused into its loads: large contractions whose modes group into
+// plain column-major matrices come here; the rest stay on the contraction
+// kernel. Products inside a stream capture or a no-alloc call stay there too
+// (the library may allocate its workspace).
 #include <rocblas/rocblas.h>
 
 #include <climits>
@@ -19,6 +19,13 @@ namespace {
 // library was slower (73.1 against 69.4 ms per n = 4096 eigendecomposition
 // with them on it), and small products launch faster there
 constexpr int64_t kLibMinDim = 256;
+// and products with fewer multiply-adds than this, where the contraction
+// kernel's choice of tile and K split is the faster (us, library against it,
+// NN / NT / TN): 256^3 18 18 18 / 8 8 9, 512 x 512 x 1000 35 34 35 / 22 20 24,
+// 800^3 31 50 48 / 32 29 34, 2000 x 300 x 600 25 72 39 / 24 23 26; on the other
+// side 2048 x 512 x 512 22 20 32 / 31 29 31, 1024^3 38 59 60 / 56 53 56,
+// 1024 x 4096 x 512 66 65 64 / 74 75 74
+constexpr double kLibMinWork = (double)(1 << 29);
 
 rocblas_handle handle_of(itg_ctx* ctx) {
   if (!ctx->blas) {
@@ -45,6 +52,7 @@ bool itg_libgemm_ok(itg_ctx* ctx, int dtype, int mode, int64_t m, int64_t n, int
   if (ctx->fixed_ws) return false;
   if (!fits32(m) || !fits32(n) || !fits32(k)) return false;
   if (m < kLibMinDim || n < kLibMinDim || k < kLibMinDim) return false;
+  if ((double)m * (double)n * (double)k < kLibMinWork) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) return false;
   return st == hipStreamCaptureStatusNone;
@@ -66,24 +74,6 @@ int itg_libgemm(itg_ctx* ctx, char ta, char tb, int64_t m, int64_t n, int64_t k,
             8.0 * (m * k + k * n + m * n * (beta != 0.0 ? 2 : 1)));
   if (s != rocblas_status_success)
     return itg_fail(ctx, ITG_EHIP, "rocblas_dgemm: %s", rocblas_status_to_string(s));
-  return ITG_OK;
-}
-
-int itg_libsyrk_lower(itg_ctx* ctx, char trans, int64_t n, int64_t k, double alpha,
-                      const double* A, int64_t lda, double* C, int64_t ldc) {
-  if (!fits32(lda) || !fits32(ldc))
-    return itg_fail(ctx, ITG_EUNSUPPORTED, "leading dimension beyond 32 bits");
-  rocblas_handle h = handle_of(ctx);
-  if (!h) return itg_fail(ctx, ITG_EHIP, "rocblas_create_handle failed");
-  rocblas_set_stream(h, ctx->stream);
-  const double beta = 0.0;
-  const int t = itg_tstart(ctx, ITG_K_GETT);
-  rocblas_status s = rocblas_dsyrk(h, rocblas_fill_lower, op_of(trans), (rocblas_int)n,
-                                   (rocblas_int)k, &alpha, A, (rocblas_int)lda, &beta, C,
-                                   (rocblas_int)ldc);
-  itg_tstop(ctx, t, ITG_K_GETT, 1.0 * n * (n + 1) * k, 8.0 * (n * k + 0.5 * n * (n + 1)));
-  if (s != rocblas_status_success)
-    return itg_fail(ctx, ITG_EHIP, "rocblas_dsyrk: %s", rocblas_status_to_string(s));
   return ITG_OK;
 }
 
