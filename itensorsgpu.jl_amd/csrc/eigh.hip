@@ -634,12 +634,13 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
   }
 }
 
-// -------------------------------------------- resident reduction (m <= 3072)
+// -------------------------------------------- resident reduction (m <= 3584)
 // The trailing block of m = n - p <= 512 K rows and columns (every earlier
 // update applied, its lower triangle current) reduced by `cols` columns by
 // workgroups that keep it in registers: workgroup g owns rows R g .. R g + R - 1
-// (whole rows, both triangles; R = 16, for K = 6 12, which the registers still
-// hold), thread t of 512 columns t + 512 k, k < K.
+// (whole rows, both triangles; R = 16; K = 6 has 12, which the registers still
+// hold, K = 7 has 14, RL = 4 of them in LDS), thread t of 512 columns t + 512 k,
+// k < K.
 //
 // Bound: the latency of one exchange per column between the workgroups (write
 // to memory, poll, read); the rest is the chain of
@@ -648,8 +649,9 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
 // takes 2.8, 3.4, 4.2, 4.9 us for K = 1, 2, 3, 4 (8.2 to 13 before; 0.3 more
 // where the slot is emptied before the column and not while its exchange is
 // under way); whole eigendecompositions: n = 512 3.7 -> 1.9 ms, 1000 8.3 -> 4.1,
-// 2048 20.4 -> 10.1, 3000 23.5 -> 18.4 by K = 6. A workgroup's 16 values go out
-// as one store: sixteen by the lane that holds them took 15% longer.
+// 2048 20.4 -> 10.1, 3000 23.5 -> 18.4 by K = 6, 4096 40.0 -> 36.2 by K = 7. A
+// workgroup's values go out as one store: one by one, by the lane that holds
+// them, took 15% longer.
 //
 // Column j, every workgroup alike: from a = A(:, j) (known to all) the norm,
 // the reflector v and tau; one pass over the workgroup's rows applies the
@@ -674,7 +676,8 @@ __global__ __launch_bounds__(512) void trd_tail_kernel(double* __restrict__ A, i
 // processes on it every wait is bounded by `limit` ticks (100 MHz): then
 // *stop is set, every workgroup leaves, and the host starts over without this
 // kernel.
-constexpr int MID_MAX = 3072;
+constexpr int MID_MAX = 3584;
+constexpr size_t MID_LDS = 4 * 3584 * sizeof(double);
 constexpr unsigned long long MID_EMPTY = 0x7FF8A5A5C3C35A5AULL;
 typedef unsigned long long mid_t;
 
@@ -691,27 +694,31 @@ __global__ void trd_mid_clear_kernel(mid_t* ring, int count, int* stop, bool fir
   if (e == 0 && first) *stop = 0;
 }
 
-template <int K, int R>
+template <int K, int RV, int RL>
 __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, int n, int p, int cols,
                                                       double* __restrict__ d,
                                                       double* __restrict__ e,
                                                       double* __restrict__ tau, mid_t* ring,
                                                       int* stop, long long limit) {
-  constexpr int MP = 512 * K;
+  constexpr int MP = 512 * K, R = RV + RL;
+  extern __shared__ double trd_mid_lds[];   // rows RV .. R - 1, MP each
   __shared__ double red1[8], red2[8], part[8][16], ncol[R], rv[R], rw[R], sc[2];
   __shared__ int bad;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int m = n - p, row0 = (int)blockIdx.x * R;
   const bool writer = blockIdx.x + 1 == gridDim.x;   // its rows are the last ones done
   double* Ap = A + (size_t)p * n + p;
-  double x[K][R];
+  double x[K][RV];
+  double* xl = trd_mid_lds + t;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int c = t + 512 * k;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int r = row0 + i, hi = r > c ? r : c, lo = r > c ? c : r;
-      x[k][i] = hi < m ? Ap[(size_t)lo * n + hi] : 0.0;
+      const double q = hi < m ? Ap[(size_t)lo * n + hi] : 0.0;
+      if (i < RV) x[k][i < RV ? i : 0] = q;
+      else xl[(i - RV) * MP + 512 * k] = q;
     }
   }
   // a: column j; v, w: column j - 1's until the pass, then j's
@@ -757,7 +764,7 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
       tau[p + j] = tv;
     }
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
+    for (int i = 0; i < RV; ++i) {
       const double pr = rv[i], qr = rw[i];
       y[i] = 0.0;
 #pragma unroll
@@ -766,12 +773,26 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
         y[i] += x[k][i] * vn[k];
       }
     }
+#pragma unroll
+    for (int i = RV; i < R; ++i) {
+      const double pr = rv[i], qr = rw[i];
+      y[i] = 0.0;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        double q = xl[(i - RV) * MP + 512 * k];
+        q -= pr * w[k] + qr * v[k];
+        xl[(i - RV) * MP + 512 * k] = q;
+        y[i] += q * vn[k];
+      }
+    }
     if (t == ((j + 1) & 511)) {
 #pragma unroll
       for (int k = 0; k < K; ++k)
         if (k == (j + 1) / 512) {
 #pragma unroll
-          for (int i = 0; i < R; ++i) ncol[i] = x[k][i];
+          for (int i = 0; i < RV; ++i) ncol[i] = x[k][i];
+#pragma unroll
+          for (int i = RV; i < R; ++i) ncol[i] = xl[(i - RV) * MP + 512 * k];
         }
     }
 #pragma unroll
@@ -874,7 +895,8 @@ __global__ __launch_bounds__(512) void trd_mid_kernel(double* __restrict__ A, in
     for (int k = 0; k < K; ++k) {
       const int c = t + 512 * k;
       if (r >= cols && c >= r && c < m)
-        Ap[(size_t)r * n + c] = x[k][i] - (pr * w[k] + qr * v[k]);
+        Ap[(size_t)r * n + c] = (i < RV ? x[k][i < RV ? i : 0] : xl[(i - RV) * MP + 512 * k]) -
+                                (pr * w[k] + qr * v[k]);
     }
   }
 }
@@ -1784,6 +1806,8 @@ int set_lds_limit(itg_ctx* ctx) {
   if (done) return ITG_OK;
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_prepare_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 8192 * 12));
+  ITG_HIP(ctx, hipFuncSetAttribute((const void*)trd_mid_kernel<7, 10, 4>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, MID_LDS));
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_leaf_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(DcLeaf)));
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_final_sort_kernel,
@@ -1815,7 +1839,7 @@ static int eig_workspace(itg_ctx* ctx, size_t bytes, void** out) {
 // From this many trailing rows on: the copy, the loads and the read-back cost
 // 31 us, a column of the chip-wide kernels 5 us more than one of these (n = 220
 // whole: 1045 us without, 934 with; even at six columns). Up to MID_MAX rows:
-// the registers of 256 CUs hold no more.
+// the registers and LDS of 256 CUs hold no more.
 constexpr int MID_MIN = TRD_TAIL + 8;
 
 // Columns p .. n - TRD_TAIL - 1 by the resident kernels, the trailing block
@@ -1840,16 +1864,17 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
       end = K == 1 ? n - TRD_TAIL : n - 512 * (K - 1);
       const int count = 4 * 2 * 512 * K;
       trd_mid_clear_kernel<<<(count + 255) / 256, 256, 0, st>>>(ring, count, stop, p == p0);
-      auto go = [&](auto kernel, int rows) {
-        kernel<<<(m + rows - 1) / rows, 512, 0, st>>>(A, n, p, end - p, d, e, tau, ring, stop,
-                                                      limit);
+      auto go = [&](auto kernel, int rows, size_t lds) {
+        kernel<<<(m + rows - 1) / rows, 512, lds, st>>>(A, n, p, end - p, d, e, tau, ring, stop,
+                                                        limit);
       };
-      if (K == 1) go(trd_mid_kernel<1, 16>, 16);
-      else if (K == 2) go(trd_mid_kernel<2, 16>, 16);
-      else if (K == 3) go(trd_mid_kernel<3, 16>, 16);
-      else if (K == 4) go(trd_mid_kernel<4, 16>, 16);
-      else if (K == 5) go(trd_mid_kernel<5, 16>, 16);
-      else go(trd_mid_kernel<6, 12>, 12);
+      if (K == 1) go(trd_mid_kernel<1, 16, 0>, 16, 0);
+      else if (K == 2) go(trd_mid_kernel<2, 16, 0>, 16, 0);
+      else if (K == 3) go(trd_mid_kernel<3, 16, 0>, 16, 0);
+      else if (K == 4) go(trd_mid_kernel<4, 16, 0>, 16, 0);
+      else if (K == 5) go(trd_mid_kernel<5, 16, 0>, 16, 0);
+      else if (K == 6) go(trd_mid_kernel<6, 12, 0>, 12, 0);
+      else go(trd_mid_kernel<7, 10, 4>, 14, MID_LDS);
       ITG_LAUNCH_CHECK(ctx);
     }
     ITG_HIP(ctx, hipMemcpyAsync(&stopped, stop, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -2156,7 +2181,7 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
     // with every CU its workgroups need
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     ITG_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cap));
-    const bool resident = cap == hipStreamCaptureStatusNone && ctx->num_cu >= MID_MAX / 12;
+    const bool resident = cap == hipStreamCaptureStatusNone && ctx->num_cu >= MID_MAX / 14;
     rc = tridiagonalize(ctx, n, A, d, e, tau, VW, Ypart, ab, pnorm, pyv, trd_sc,
                         resident ? Qa : nullptr, Qb);
   }

@@ -1,6 +1,6 @@
 """Eigendecompositions whose tridiagonalisation runs in workgroups that keep
 the matrix in registers: sizes around its first one, around a workgroup's 16
-(12) rows and around each 512 columns at which one kernel hands over to the next;
+(12, 14) rows and around each 512 columns at which one kernel hands over to the next;
 the start over without it when a wait runs out; several threads at once.
 Bounds: eigenvalues, U^T U - I and A U - U w within 8 n eps ||A||_2 of a
 backward stable reduction (eps = 2^-52)."""
@@ -54,7 +54,8 @@ def test_sizes(n, kind):
     _check(A, *_solve(A))
 
 
-@pytest.mark.parametrize("n", [1537, 2049, 2560, 2561, 2569, 2580, 3072, 3073])
+@pytest.mark.parametrize("n", [1537, 2049, 2560, 2561, 2569, 2580, 3072, 3073, 3300,
+                               3584, 3585, 3650])
 def test_large(n):
     A = _matrix(n, "graded" if n == 2560 else "full")
     _check(A, *_solve(A))
