@@ -3,16 +3,18 @@
 // syevd, eigenvalues reversed to descending, truncate!, columns reversed and
 // sliced) used by replacebond! on the density matrix rho = phi phi^T.
 //
-// 1. Householder tridiagonalisation, blocked as in LAPACK dsytrd/dlatrd
-//    (panels of NB columns): per column two kernels spanning the GPU (the
-//    reflector fused into the symmetric matrix-vector product over the
-//    trailing block, then w and the next column's update; see below); per
-//    panel the rank-2*NB trailing update A -= V W^T + W V^T on FP64 MFMA.
+// 1. Householder tridiagonalisation. More than 3584 trailing rows: blocked as
+//    in LAPACK dsytrd/dlatrd (panels of NB columns), per column two kernels
+//    spanning the GPU (the reflector fused into the symmetric matrix-vector
+//    product over the trailing block, then w and the next column's update; see
+//    below), per panel the rank-2*NB trailing update A -= V W^T + W V^T on FP64
+//    MFMA. Then in the registers of many workgroups that exchange one vector
+//    pair per column, and the last 192 rows in one workgroup.
 // 2. Divide and conquer on the tridiagonal (Cuppen tearing at every split,
-//    bottom-up merges of blocks 1,2,4,...): per merge a sort + deflation
-//    workgroup, rotation, secular-root, Gu-Eisenstat and eigenvector kernels,
-//    and Q_new = Q_old[:, nondeflated] V on MFMA (gathered columns through
-//    a device offset table) for large merges.
+//    bottom-up merges): blocks up to 64 in one launch; per larger merge a sort
+//    + deflation workgroup, rotation, secular-root, Gu-Eisenstat and
+//    eigenvector kernels, and Q_new = Q_old[:, nondeflated] V on MFMA (gathered
+//    columns through a device offset table) for large merges.
 // 3. Eigenvalues sorted descending, truncate! decided on the device, and only
 //    the k kept eigenvectors back-transformed by the compact-WY block
 //    reflectors (Schreiber & Van Loan 1989) on MFMA.
