@@ -2744,7 +2744,8 @@ __global__ __launch_bounds__(256) void qr_update_kernel(const double* __restrict
 // factored in the same launch: workgroup 0 updates that block in the registers
 // it factors it in, while the others (512 rows x 16 columns each) update the
 // rest. A panel takes longer than the update beside it (33 against 14 us),
-// which is hidden: 34 us a panel, 2000 x 1000 3.92 -> 3.14 ms.
+// which is hidden: 34 us a panel, 2000 x 1000 3.92 -> 3.14 ms. The block's
+// columns have to be the panel's: wn = min(QW, nc).
 template <int RPT, int CW>
 __global__ __launch_bounds__(512) void qr_step_kernel(const double* A, int ld, int m2,
                                                       const double* __restrict__ tau, double* C,
@@ -3065,8 +3066,10 @@ static int qr_blocked(itg_ctx* ctx, int m, int n, double* W, double* tau, double
       kernel<<<2 + (nb - 1) * ((m2 + 511) / 512), 512, 0, st>>>(A, m, m2, tau + p, C, nt, Yp, ns, wn,
                                                                 tau + pn);
     };
-    // past 4096 rows the panel's registers leave no room for the update
-    if (wn <= 0 || rows > 4096) {
+    // past 4096 rows the panel's registers leave no room for the update; and a
+    // last panel narrower than its block of columns (a wide matrix) leaves
+    // columns of the block that the panel's workgroup does not hold
+    if (wn < std::min(QW, nt) || rows > 4096) {
       qr_update_kernel<<<dim3(nb, ns), 256, 0, st>>>(A, m, m2, w, tau + p, C, m, nt, Yp);
       if (wn > 0) panel(C + QW, rows, wn, tau + pn);
     } else if (rows <= 1024) {
