@@ -1616,12 +1616,13 @@ __global__ __launch_bounds__(256) void dc_leaf_kernel(int n, const double* __res
     const int i = g - r0;
     double* Q = L.Q[cur];
     double* D = L.D[cur];
-    // z and the position in the merge's ascending order
+    // z and the position in the merge's ascending order (NaN after all
+    // others, so that the positions are a permutation whatever D holds)
     if (act && g < nl) {
       int before = 0;
-      const double dg = D[g];
+      const double dv = D[g], dg = fmin(dv, INFINITY);
       for (int c = q4; c < sm; c += 4) {
-        const double dc = D[r0 + c];
+        const double dc = fmin(D[r0 + c], INFINITY);
         before += (dc < dg || (dc == dg && c < i)) ? 1 : 0;
       }
       before += __builtin_amdgcn_mov_dpp(before, 0xB1, 0xF, 0xF, false);
@@ -1630,7 +1631,7 @@ __global__ __launch_bounds__(256) void dc_leaf_kernel(int n, const double* __res
         const double beta = e[r00 + r0 + half - 1];
         const double sg = beta >= 0.0 ? 1.0 : -1.0;
         const double z = i < half ? Q[g * LD + r0 + half - 1] : sg * Q[g * LD + r0 + half];
-        L.ds[r0 + before] = dg;
+        L.ds[r0 + before] = dv;
         L.zs[r0 + before] = z * 0.7071067811865476;
         L.col[r0 + before] = g;
         if (i == 0) L.rho[r0] = 2.0 * fabs(beta);
