@@ -1197,11 +1197,14 @@ __global__ __launch_bounds__(1024) void dc_prepare_kernel(int n, int s_lvl, int 
       zm = fmax(zm, amax[1][q]);
     }
     const double tol = 8.0 * ITG_DC_EPS * fmax(dm, zm);
+    // one test for the counts and the lists (NaN is kept): a list shorter
+    // than its count would leave indices unset
+    auto drops = [&](int i) { return rho * fabs(z[i]) <= tol; };
     // thread t owns the contiguous entries [t cs, t cs + cs)
     const int cs = (s + (int)blockDim.x - 1) / (int)blockDim.x;
     const int i0 = min(s, t * cs), i1 = min(s, i0 + cs);
     int cnt = 0;
-    for (int i = i0; i < i1; ++i) cnt += (rho * fabs(z[i]) <= tol) ? 0 : 1;
+    for (int i = i0; i < i1; ++i) cnt += drops(i) ? 0 : 1;
     // exclusive scan of the kept counts over the block
     int inc = cnt;
     for (int o = 1; o < 64; o <<= 1) {
@@ -1217,7 +1220,7 @@ __global__ __launch_bounds__(1024) void dc_prepare_kernel(int n, int s_lvl, int 
     }
     const int pos0 = base + inc - cnt;
     for (int i = i0, pos = pos0; i < i1; ++i)
-      if (rho * fabs(z[i]) > tol) kidx[pos++] = i;
+      if (!drops(i)) kidx[pos++] = i;
     __syncthreads();
     for (int p = t + 1; p < total; p += blockDim.x) {
       const int pj = kidx[p - 1], j = kidx[p];
@@ -1288,7 +1291,7 @@ __global__ __launch_bounds__(1024) void dc_prepare_kernel(int n, int s_lvl, int 
     }
     // dropped entries, among them in order the entries rotated away
     for (int i = i0, pos = pos0; i < i1; ++i) {
-      if (rho * fabs(z[i]) > tol) {
+      if (!drops(i)) {
         ++pos;
         continue;
       }

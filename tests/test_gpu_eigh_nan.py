@@ -31,3 +31,8 @@ def _check(n):
 @pytest.mark.parametrize("n", [2, 3, 5, 16, 17, 33, 63, 64])
 def test_one_leaf(n):
     _check(n)
+
+
+@pytest.mark.parametrize("n", [65, 100, 128, 130, 193, 257, 300, 520, 1030])
+def test_merges(n):
+    _check(n)
