@@ -20,6 +20,7 @@
 
 #include "bf16x3.h"
 #include "itg_internal.h"
+#include "wpass_core.h"
 
 // X[q][o], q = wl + WL*(s1 + d*s2), o = s1' + d*(s2' + d*wr)
 template <typename T>
@@ -89,10 +90,6 @@ __global__ __launch_bounds__(256) void heff_wpass_fixed_kernel(int64_t chiL, int
 //   Q = O = 45, 300 x 300 FP64: 56 -> 25; Q = O = 20, 20 x 20 FP64: 20 -> 8
 typedef double d4w_t __attribute__((ext_vector_type(4)));
 
-__host__ __device__ constexpr int wpass_ldo(int O) {
-  return ((O + 15) / 16 * 16) % 32 == 0 ? (O + 15) / 16 * 16 + 16 : (O + 15) / 16 * 16;
-}
-
 template <typename T, int NT, int AT>
 __global__ __launch_bounds__(256) void heff_wpass_mfma_kernel(int chiL, int chiR, int Q,
                                                               int64_t Oall, int O,
@@ -102,7 +99,7 @@ __global__ __launch_bounds__(256) void heff_wpass_mfma_kernel(int chiL, int chiR
   extern __shared__ double xs[];
   const int t = threadIdx.x, lane = t & 63, lr = lane & 15, lg = lane >> 4;
   const int kt = (Q + 3) / 4, ldo = wpass_ldo(O), ot = (O + 15) / 16;
-  for (int e = t; e < 4 * kt * ldo; e += 256) {
+  for (int e = t; e < wpass_doubles(Q, O, NT); e += 256) {
     const int q = e / ldo, o = e % ldo;
     xs[e] = q < Q && o < O ? X[q + Q * o] : 0.0;
   }
@@ -136,10 +133,9 @@ __global__ __launch_bounds__(256) void heff_wpass_mfma_kernel(int chiL, int chiR
 #pragma unroll
         for (int i = 0; i < KC; ++i) {
           if (k0 + i >= kt) break;
-          const double* x = xs + (4 * (k0 + i) + lg) * ldo + 16 * o0 + lr;
 #pragma unroll
           for (int j = 0; j < NT; ++j) {
-            const double xj = x[16 * j];
+            const double xj = xs[wpass_at(4 * (k0 + i) + lg, ldo, o0, j, lr)];
 #pragma unroll
             for (int s = 0; s < AT; ++s)
               acc[s][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(xj, (double)v[i][s], acc[s][j], 0, 0, 0);
@@ -173,11 +169,10 @@ static void wpass(itg_ctx* ctx, int64_t chiL, int64_t chiR, int64_t Q, int64_t O
   }
   // outputs per launch: as many as X has room for in 64 KB of LDS (all of
   // them but for an MPO of thousands of channels and d = 1)
-  const int64_t rows = (Q + 3) / 4 * 4;
+  const int nt = wpass_nt(O);
   int64_t os = O;
-  while (rows * wpass_ldo((int)os) * 8 > 65536) os = (os / 2 + 15) / 16 * 16;
-  const size_t lds = (size_t)rows * wpass_ldo((int)os) * sizeof(double);
-  const int nt = (O + 15) / 16 <= 1 ? 1 : (O + 15) / 16 == 2 ? 2 : 4;
+  while (wpass_doubles((int)Q, (int)os, nt) * 8 > 65536) os = (os / 2 + 15) / 16 * 16;
+  const size_t lds = (size_t)wpass_doubles((int)Q, (int)os, nt) * sizeof(double);
   // two row tiles a wave once there are enough of them
   const int at = chiL >= 200 ? 2 : 1;
   const int64_t units = (chiL + 16 * at - 1) / (16 * at) * chiR;
