@@ -128,11 +128,16 @@ __global__ __launch_bounds__(256) void heff_wpass_mfma_kernel(int chiL, int chiR
           const int q = 4 * (k0 + i) + lg;
 #pragma unroll
           for (int s = 0; s < AT; ++s)
-            v[i][s] = src[s][(int64_t)chiL * (q < Q ? q : Q - 1)];   // X is zero past Q
+            v[i][s] = src[s][(int64_t)chiL * (q < Q ? q : Q - 1)];
         }
 #pragma unroll
         for (int i = 0; i < KC; ++i) {
           if (k0 + i >= kt) break;
+          // zero past Q, as X is: an infinity times zero would be a NaN
+          if (4 * (k0 + i) + lg >= Q) {
+#pragma unroll
+            for (int s = 0; s < AT; ++s) v[i][s] = (T)0;
+          }
 #pragma unroll
           for (int j = 0; j < NT; ++j) {
             const double xj = xs[wpass_at(4 * (k0 + i) + lg, ldo, o0, j, lr)];
