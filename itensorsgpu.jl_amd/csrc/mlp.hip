@@ -93,8 +93,8 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(int f, int64_t rows, con
 // GELU' passes instead of being products of their own; only the hidden x
 // hidden products stay on MFMA. Thread = hidden unit (blockIdx.y: groups of
 // 256), block = a range of rows; layer 3's sums over the hidden units take a
-// wave per row instead. Weight and bias gradients leave one partial per block,
-// summed in one last launch. Forward and backward of 4096 rows at 12 -> 256 ->
+// wave per row instead. Weight and bias gradients (these in FP64) leave one
+// partial per block, summed in one last launch. Forward and backward of 4096 rows at 12 -> 256 ->
 // 256 -> 4 take 10 launches and 97 us; as products and elementwise passes,
 // 142. At the limit: in = 32, out = 16 122 us, past it 154 to 158 (200 rows:
 // 87 against 130; 65536 rows: 722 against 960 to 999).
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void mlp_back3_kernel(int64_t rows, int h, int
                                                         const float* __restrict__ A2,
                                                         float* __restrict__ dZ2,
                                                         float* __restrict__ pw,
-                                                        float* __restrict__ pb) {
+                                                        double* __restrict__ pb) {
   __shared__ float ds[MLP_TILE][OUT];
   const int t = threadIdx.x, f = blockIdx.y * 256 + t;
   float w[OUT], gw[OUT];
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(256) void mlp_back3_kernel(int64_t rows, int h, int
 #pragma unroll
   for (int o = 0; o < OUT; ++o)
     if (o < out) pw[((int64_t)blockIdx.x * out + o) * h + f] = gw[o];
-  pb[(int64_t)blockIdx.x * h + f] = (float)gb;
+  pb[(int64_t)blockIdx.x * h + f] = gb;
 }
 
 // with dZ1 = dA1 gelu'(Z1): this block's partials of dW1 (in x h here) and db1
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) void mlp_back1_kernel(int64_t rows, int in, in
                                                         const float* __restrict__ Z1,
                                                         const float* __restrict__ dA1,
                                                         float* __restrict__ pw,
-                                                        float* __restrict__ pb) {
+                                                        double* __restrict__ pb) {
   __shared__ float xs[MLP_TILE][IN];
   const int t = threadIdx.x, f = blockIdx.y * 256 + t;
   float gw[IN];
@@ -308,12 +308,13 @@ __global__ __launch_bounds__(256) void mlp_back1_kernel(int64_t rows, int in, in
 #pragma unroll
   for (int k = 0; k < IN; ++k)
     if (k < in) pw[((int64_t)blockIdx.x * in + k) * h + f] = gw[k];
-  pb[(int64_t)blockIdx.x * h + f] = (float)gb;
+  pb[(int64_t)blockIdx.x * h + f] = gb;
 }
 
 struct GradSums {
-  const float *w1, *b1, *w3, *b2;   // nb partials each of in x h, h, out x h, h
-  const double* y;                  // ny partials of out + 1
+  const float *w1, *w3;        // nb partials each of in x h, out x h
+  const double *b1, *b2;       // nb partials each of h
+  const double* y;             // ny partials of out + 1
   int nb, ny, in, h, out;
   float *gw1, *gb1, *gw3, *gb2, *gb3;
   double* loss;
@@ -332,20 +333,22 @@ __global__ __launch_bounds__(1024) void mlp_grad_sum_kernel(GradSums g) {
   if ((int64_t)blockIdx.x * 64 >= cnt) return;   // whole block
   double s = 0.0;
   if (e < cnt) {
-    if (job == 4) {
-      for (int z = zi; z < g.ny; z += 16) s += g.y[(int64_t)z * cnt + e];
-    } else {
-      const float* p = (job == 0 ? g.w1 : job == 1 ? g.b1 : job == 2 ? g.w3 : g.b2) + e;
+    auto add = [&](auto* p, int nb) {
       int z = zi;
-      for (; z + 112 < g.nb; z += 128) {
-        float v[8];
+      for (; z + 112 < nb; z += 128) {
+        double v[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = p[(int64_t)(z + 16 * q) * cnt];
+        for (int q = 0; q < 8; ++q) v[q] = (double)p[(int64_t)(z + 16 * q) * cnt];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) s += (double)v[q];
+        for (int q = 0; q < 8; ++q) s += v[q];
       }
-      for (; z < g.nb; z += 16) s += (double)p[(int64_t)z * cnt];
-    }
+      for (; z < nb; z += 16) s += (double)p[(int64_t)z * cnt];
+    };
+    if (job == 0) add(g.w1 + e, g.nb);
+    else if (job == 1) add(g.b1 + e, g.nb);
+    else if (job == 2) add(g.w3 + e, g.nb);
+    else if (job == 3) add(g.b2 + e, g.nb);
+    else add(g.y + e, g.ny);
   }
   sh[zi][ei] = s;
   __syncthreads();
@@ -670,18 +673,18 @@ extern "C" int itg_mlp_backward(itg_ctx* ctx, int rows, int in, int h, int out, 
   if (mlp_outer_fused(in, out)) {
     const int64_t rpb = mlp_rpb(ctx, rows, h), nbr = (rows + rpb - 1) / rpb;
     const int64_t rpy = std::max<int64_t>(16, (rows + 511) / 512), ny = (rows + rpy - 1) / rpy;
-    const size_t floats = (size_t)ro + 2 * rh + (size_t)nbr * h * (in + out + 2);
-    rc = mlp_workspace(ctx, floats * sizeof(float) + (size_t)ny * (out + 1) * sizeof(double) + 256,
-                       &ws);
+    const size_t floats = (size_t)ro + 2 * rh + (size_t)nbr * h * (in + out);
+    const size_t doubles = (size_t)nbr * h * 2 + (size_t)ny * (out + 1);
+    rc = mlp_workspace(ctx, floats * sizeof(float) + doubles * sizeof(double) + 256, &ws);
     if (rc) return rc;
     float* dY = (float*)ws;
     float* dZ2 = dY + ro;
     float* dA1 = dZ2 + rh;
     float* pw1 = dA1 + rh;
-    float* pb1 = pw1 + nbr * h * in;
-    float* pw3 = pb1 + nbr * h;
-    float* pb2 = pw3 + nbr * h * out;
-    double* py = (double*)(((uintptr_t)(pb2 + nbr * h) + 255) & ~(uintptr_t)255);
+    float* pw3 = pw1 + nbr * h * in;
+    double* pb1 = (double*)(((uintptr_t)(pw3 + nbr * h * out) + 255) & ~(uintptr_t)255);
+    double* pb2 = pb1 + nbr * h;
+    double* py = pb2 + nbr * h;
     hipStream_t st = ctx->stream;
     const dim3 grid((unsigned)nbr, (h + 255) / 256);
     mlp_mse_kernel<<<(unsigned)ny, 256, 0, st>>>(rows, out, rpy, Y, T, 1.0f / (float)ro, dY, py);
@@ -696,7 +699,7 @@ extern "C" int itg_mlp_backward(itg_ctx* ctx, int rows, int in, int h, int out, 
     if (rc) return rc;
     if (in <= 16) mlp_back1_kernel<16><<<grid, 256, 0, st>>>(rows, in, h, rpb, X, Z1, dA1, pw1, pb1);
     else mlp_back1_kernel<32><<<grid, 256, 0, st>>>(rows, in, h, rpb, X, Z1, dA1, pw1, pb1);
-    const GradSums gs = {pw1, pb1, pw3, pb2, py, (int)nbr, (int)ny, in, h, out, G + L.W1,
+    const GradSums gs = {pw1, pw3, pb1, pb2, py, (int)nbr, (int)ny, in, h, out, G + L.W1,
                          G + L.b1, G + L.W3, G + L.b2, G + L.b3,
                          loss ? ctx->red_host : nullptr};
     const int64_t most = (int64_t)h * std::max(in, out);
