@@ -2356,20 +2356,37 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
 // takes 0.45 ms; panel by panel (16 reflectors, two launches each), 1.45.
 namespace {
 
+// A reflector whose tail x below the pivot alpha has |x|^2 < QR_TINY2: near
+// underflow, in its squares and in its products with other columns as small.
+// Beside a pivot of QR_TINY_PIVOT or more the tail is less than 2^-60 of the
+// column and counts as zero; else the reflector is formed from QR_UP times the
+// tail (or QR_UP^2 times, if that is still as small), so that a matrix of any
+// scale satisfies A = QR relative to itself.
+constexpr double QR_TINY2 = 0x1p-600, QR_TINY_PIVOT = 0x1p-240, QR_UP = 0x1p500;
+
 __global__ __launch_bounds__(1024) void qr_reflect_kernel(double* __restrict__ W, int m, int j,
                                                           double* __restrict__ tau) {
   __shared__ double red[16];
   __shared__ double sc;
   double* a = W + (size_t)j * m;
-  double part = 0.0;
-  for (int r = j + 1 + threadIdx.x; r < m; r += blockDim.x) part += a[r] * a[r];
-  double xn2 = block_sum(part, red);
+  double xn2, up = 1.0;
+  while (true) {
+    double part = 0.0;
+    for (int r = j + 1 + threadIdx.x; r < m; r += blockDim.x) part += (a[r] * up) * (a[r] * up);
+    xn2 = block_sum(part, red);
+    // the same in the whole workgroup
+    if (!(xn2 < QR_TINY2) || !(fabs(a[j]) * up < QR_TINY_PIVOT) || up > QR_UP) break;
+    up *= QR_UP;
+  }
+  __syncthreads();   // a[j] is read above
   if (threadIdx.x == 0) {
-    double alpha = a[j], beta = alpha, tv = 0.0, scale = 1.0;
-    if (xn2 != 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-      tv = (beta - alpha) / beta;
-      scale = 1.0 / (alpha - beta);
+    const double alpha = a[j], au = alpha * up;
+    double beta = alpha, tv = 0.0, scale = 0.0;
+    if (!(xn2 < QR_TINY2) || (up > 1.0 && xn2 > 0.0)) {
+      const double bu = -copysign(sqrt(au * au + xn2), au);
+      beta = bu / up;
+      tv = (bu - au) / bu;
+      scale = 1.0 / (au - bu);
     }
     a[j] = beta;
     tau[j] = tv;
@@ -2377,7 +2394,7 @@ __global__ __launch_bounds__(1024) void qr_reflect_kernel(double* __restrict__ W
   }
   __syncthreads();
   double scale = sc;
-  for (int r = j + 1 + threadIdx.x; r < m; r += blockDim.x) a[r] *= scale;
+  for (int r = j + 1 + threadIdx.x; r < m; r += blockDim.x) a[r] = a[r] * up * scale;
 }
 
 // W[j:m, c] -= tau_j v (v^T W[j:m, c]) for j < c < nend (the rest of the
@@ -2494,29 +2511,40 @@ struct QrPanel {
   __device__ __forceinline__ void factor(int j0, int j1) {
     constexpr int NC = 1 << LOG;
     for (int j = j0; j < j1; ++j) {
-      double d[NC];
+      double g, rv, alpha, xn2, up = 1.0, down = 1.0;
+      while (true) {
+        double d[NC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) d[c] = 0.0;
+        for (int c = 0; c < NC; ++c) d[c] = 0.0;
 #pragma unroll
-      for (int a = 0; a < RPT; ++a) {
-        const double xj = (a > 0 || t > j) ? x[a][0] : 0.0;
+        for (int a = 0; a < RPT; ++a) {
+          const double xj = (a > 0 || t > j) ? x[a][0] : 0.0;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) d[c] += xj * x[a][c];
+          for (int c = 0; c < NC; ++c) d[c] += xj * x[a][c];
+        }
+        if (t == j) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) rowv[buf][c] = x[0][c];
+        }
+        g = reduce<LOG>(d);
+        rv = rowv[buf][lane & (NC - 1)];
+        buf ^= 1;
+        alpha = read_lane(rv, 0);
+        xn2 = read_lane(g, 0);
+        // the same in the whole workgroup
+        if (!(xn2 < QR_TINY2) || !(fabs(alpha) * up < QR_TINY_PIVOT) || up > QR_UP) break;
+#pragma unroll
+        for (int a = 0; a < RPT; ++a)
+          if (a > 0 || t > j) x[a][0] *= QR_UP;
+        up *= QR_UP;
+        down /= QR_UP;
       }
-      if (t == j) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) rowv[buf][c] = x[0][c];
-      }
-      const double g = reduce<LOG>(d);
-      const double rv = rowv[buf][lane & (NC - 1)];
-      buf ^= 1;
-      const double alpha = read_lane(rv, 0), xn2 = read_lane(g, 0);
-      // a column whose squares underflow has no direction left: it is dropped
       double beta = alpha, tj = 0.0, scale = 0.0;
-      if (xn2 >= 0x1p-1010) {
-        beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-        tj = (beta - alpha) / beta;
-        scale = 1.0 / (alpha - beta);
+      if (!(xn2 < QR_TINY2) || (up > 1.0 && xn2 > 0.0)) {
+        const double au = alpha * up, bu = -copysign(sqrt(au * au + xn2), au);
+        beta = bu * down;
+        tj = (bu - au) / bu;
+        scale = 1.0 / (au - bu);
       }
       if (t == 0) {
         tau[j] = tj;
