@@ -1927,6 +1927,7 @@ static int eig_workspace(itg_ctx* ctx, size_t bytes, void** out) {
 // whole: 1045 us without, 934 with; even at six columns). Up to MID_MAX rows:
 // the registers and LDS of 256 CUs hold no more.
 constexpr int MID_MIN = TRD_TAIL + 8;
+constexpr int MID_SKIP = 32;
 
 // Columns p .. n - TRD_TAIL - 1 by the resident kernels, the trailing block
 // handed from one to the next as it shrinks; *ok = false if a wait ran out
@@ -1967,6 +1968,11 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
     ITG_HIP(ctx, hipStreamSynchronize(st));
   }
   *ok = stopped == 0;
+  // a device that is shared for long: from the second run-out in a row on,
+  // 2, 4, .. MID_SKIP calls of this context do without before the next try,
+  // so that the waits cost them at most limit / MID_SKIP each
+  ctx->trd_outs = stopped ? std::min(ctx->trd_outs + 1, 31) : 0;
+  ctx->trd_skip = ctx->trd_outs > 1 ? std::min(1 << (ctx->trd_outs - 1), MID_SKIP) : 0;
   if (stopped) {
     trd_copy_kernel<<<itg_blocks((int64_t)m0 * m0, 256, 8192), 256, 0, st>>>(A, n, p0, copy, true);
     ITG_LAUNCH_CHECK(ctx);
@@ -1986,6 +1992,10 @@ static int tridiagonalize(itg_ctx* ctx, int n, double* A, double* d, double* e, 
   double* V2 = VW + 2 * (size_t)n * NB;
   bool resident = copy != nullptr;
   for (int p = 0, nbp; p < n; p += nbp) {
+    if (resident && n - p <= MID_MAX && n - p >= MID_MIN && ctx->trd_skip > 0) {
+      --ctx->trd_skip;
+      resident = false;
+    }
     if (resident && n - p <= MID_MAX && n - p >= MID_MIN) {
       int rc = trd_resident(ctx, n, p, A, d, e, tau, copy, (mid_t*)ring, &resident);
       if (rc) return rc;

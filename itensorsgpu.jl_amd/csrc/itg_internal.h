@@ -46,6 +46,9 @@ struct itg_ctx {
   std::vector<TimedLaunch> launches;
   std::vector<hipEvent_t> event_pool;
   size_t event_next = 0;
+  // resident tridiagonalisations in a row whose wait ran out, and calls that
+  // do without one before the next try (eigh.hip)
+  int trd_outs = 0, trd_skip = 0;
   // captured Heff-apply graphs of itg_davidson2 (null: seen once, eager)
   std::unordered_map<std::string, hipGraphExec_t> graphs;
   // this device's copy of the no-alloc scratch array (heff.hip), resolved
