@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -28,6 +29,10 @@ extern "C" const char* itg_last_error(itg_ctx* ctx) {
 }
 
 // =============================================================== context
+static std::atomic<int> live_contexts[64];   // by device mod 64
+
+int itg_live_contexts(int device) { return live_contexts[device & 63].load(); }
+
 extern "C" int itg_init(int device, itg_ctx** out) {
   if (!out) return ITG_EARG;
   *out = nullptr;
@@ -63,6 +68,7 @@ extern "C" int itg_init(int device, itg_ctx** out) {
     delete ctx;
     return ITG_EHIP;
   }
+  ++live_contexts[device & 63];
   *out = ctx;
   return ITG_OK;
 }
@@ -84,6 +90,7 @@ extern "C" int itg_destroy(itg_ctx* ctx) {
   if (ctx->red) hipFree(ctx->red);
   if (ctx->red_host) hipHostFree(ctx->red_host);
   hipStreamDestroy(ctx->own_stream);
+  --live_contexts[ctx->device & 63];
   delete ctx;
   return ITG_OK;
 }

@@ -1944,6 +1944,8 @@ static int trd_resident(itg_ctx* ctx, int n, int p, double* A, double* d, double
   const int m0 = n - p, p0 = p;
   trd_copy_kernel<<<itg_blocks((int64_t)m0 * m0, 256, 8192), 256, 0, st>>>(A, n, p, copy, false);
   int stopped = 0;
+  // no other context waits for what this stream still has queued
+  if (itg_live_contexts(dev) > 1) ITG_HIP(ctx, hipStreamSynchronize(st));
   {
     std::lock_guard<std::mutex> lock(turn[dev & 63]);
     for (int end; p < n - TRD_TAIL; p = end) {

@@ -76,6 +76,9 @@ struct itg_ctx {
 
 constexpr int kRedSlots = 16384;
 
+// contexts that exist on a device (core.hip)
+int itg_live_contexts(int device);
+
 // ---------------------------------------------------------------- errors
 int itg_fail(itg_ctx* ctx, int code, const char* fmt, ...);
 
