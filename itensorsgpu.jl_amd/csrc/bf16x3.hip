@@ -361,9 +361,6 @@ __global__ __launch_bounds__(512) void gemm_split_wide_kernel(
   }
 }
 
-bool lds_ready = false;
-bool wide_ok = false;
-
 // One round of the wide kernel (one 256 x 256 tile per CU) takes as long as
 // ~1.66 rounds of the 128 x 128 kernel (two tiles per CU) at the same K
 // (MI355X, K = 2048 and 10240), so the wide tile is chosen when its rounds,
@@ -406,26 +403,27 @@ int itg_gemm_split(itg_ctx* ctx, int dtype, int64_t M, int64_t N, int64_t K, int
     return itg_fail(ctx, ITG_EARG, "split gemm: K %lld, lda %lld, ldb %lld", (long long)Kp,
                     (long long)lda, (long long)ldb);
   const size_t lds = (size_t)(2 * SB_M + 2 * SB_N) * SB_LD * sizeof(uint16_t);
-  if (!lds_ready) {
+  if (!(ctx->lds_set & ITG_LDS_SPLIT)) {
     ITG_HIP(ctx, hipFuncSetAttribute((const void*)gemm_split_kernel<double>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     ITG_HIP(ctx, hipFuncSetAttribute((const void*)gemm_split_kernel<float>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // the wide tile needs 128 KB of a CU's 160 KB of LDS; without it the
     // 128 x 128 kernel serves every shape
-    wide_ok = getenv("ITG_SPLIT_WIDE") == nullptr || strcmp(getenv("ITG_SPLIT_WIDE"), "0") != 0;
-    if (wide_ok &&
+    ctx->split_wide =
+        getenv("ITG_SPLIT_WIDE") == nullptr || strcmp(getenv("ITG_SPLIT_WIDE"), "0") != 0;
+    if (ctx->split_wide &&
         (hipFuncSetAttribute((const void*)gemm_split_wide_kernel<double>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)SW_LDS) != hipSuccess ||
          hipFuncSetAttribute((const void*)gemm_split_wide_kernel<float>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)SW_LDS) != hipSuccess)) {
       (void)hipGetLastError();
-      wide_ok = false;
+      ctx->split_wide = false;
     }
-    lds_ready = true;
+    ctx->lds_set |= ITG_LDS_SPLIT;
   }
   const int64_t wM = (M + SW_M - 1) / SW_M, wN = (N + SW_N - 1) / SW_N;
-  if (wide_ok && use_wide(wM * wN, ((M + SB_M - 1) / SB_M) * ((N + SB_N - 1) / SB_N),
+  if (ctx->split_wide && use_wide(wM * wN, ((M + SB_M - 1) / SB_M) * ((N + SB_N - 1) / SB_N),
                           ctx->num_cu)) {
     if (wM * wN > 0x7fffffff) return itg_fail(ctx, ITG_EUNSUPPORTED, "split gemm: too large");
     itg_tev tk = itg_tevents(ctx, ITG_K_GEMM_SPLIT);

@@ -472,12 +472,11 @@ int itg_zunmtr(itg_ctx* ctx, int n, int k, const void* Av, const void* tauv, con
   to_complex_kernel<<<itg_blocks((int64_t)n * k, 256, 16384), 256, 0, ctx->stream>>>(
       (int64_t)n * k, Z, U);
   ITG_LAUNCH_CHECK(ctx);
-  static bool attr = false;
-  if (!attr) {
+  if (!(ctx->lds_set & ITG_LDS_ZUNM)) {
     ITG_HIP(ctx, hipFuncSetAttribute((const void*)zunm_group_kernel,
                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                      8192 * (int)sizeof(double2)));
-    attr = true;
+    ctx->lds_set |= ITG_LDS_ZUNM;
   }
   constexpr int G = 32;
   const int nrefl = n - 1;
@@ -735,12 +734,11 @@ int itg_c64_qr(itg_ctx* ctx, int64_t m64, int64_t n64, const void* A, void* Qo, 
     if (j + 1 < n) zqr_apply_kernel<<<n - j - 1, 256, 0, ctx->stream>>>(W, m, n, j, tau);
     ITG_LAUNCH_CHECK(ctx);
   }
-  static bool attr = false;
-  if (!attr) {
+  if (!(ctx->lds_set & ITG_LDS_ZQR)) {
     ITG_HIP(ctx, hipFuncSetAttribute((const void*)zqr_form_q_kernel,
                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                      8192 * (int)sizeof(double2)));
-    attr = true;
+    ctx->lds_set |= ITG_LDS_ZQR;
   }
   zqr_form_q_kernel<<<r, 256, (size_t)m * sizeof(double2), ctx->stream>>>(W, m, r, tau,
                                                                           (double2*)Qo);

@@ -894,12 +894,11 @@ __global__ void truncate_kernel(const double* P, int64_t n, int64_t maxdim, int6
 int itg_truncate_device_async(itg_ctx* ctx, const double* P, int64_t n, int64_t maxdim,
                               int64_t mindim, double cutoff, int abs_cut, int rel_cut,
                               int semantics, double* out3) {
-  static bool lds_set = false;
-  if (!lds_set) {
+  if (!(ctx->lds_set & ITG_LDS_TRUNC)) {
     ITG_HIP(ctx, hipFuncSetAttribute((const void*)truncate_kernel,
                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)(kTruncLds * sizeof(double))));
-    lds_set = true;
+    ctx->lds_set |= ITG_LDS_TRUNC;
   }
   size_t lds = n <= kTruncLds ? (size_t)std::max<int64_t>(n, 1) * sizeof(double) : 0;
   truncate_kernel<<<1, 256, lds, ctx->stream>>>(P, n, maxdim, mindim, cutoff, abs_cut, rel_cut,

@@ -1888,8 +1888,7 @@ struct Carver {
 };
 
 int set_lds_limit(itg_ctx* ctx) {
-  static bool done = false;
-  if (done) return ITG_OK;
+  if (ctx->lds_set & ITG_LDS_EIGH) return ITG_OK;
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_prepare_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, DC_ZLDS * 28));
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)trd_mid_kernel<7, 10, 4>,
@@ -1898,7 +1897,7 @@ int set_lds_limit(itg_ctx* ctx) {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(DcLeaf)));
   ITG_HIP(ctx, hipFuncSetAttribute((const void*)dc_final_sort_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, 8192 * 12));
-  done = true;
+  ctx->lds_set |= ITG_LDS_EIGH;
   return ITG_OK;
 }
 

@@ -49,6 +49,10 @@ struct itg_ctx {
   // resident tridiagonalisations in a row whose wait ran out, and calls that
   // do without one before the next try (eigh.hip)
   int trd_outs = 0, trd_skip = 0;
+  // kernels whose dynamic LDS limit is set (ITG_LDS_* bits): the attribute is a
+  // device's, and contexts of several threads set it side by side
+  unsigned lds_set = 0;
+  bool split_wide = false;      // the split-BF16 GEMM's wide tile may run
   // captured Heff-apply graphs of itg_davidson2 (null: seen once, eager)
   std::unordered_map<std::string, hipGraphExec_t> graphs;
   // this device's copy of the no-alloc scratch array (heff.hip), resolved
@@ -75,6 +79,9 @@ struct itg_ctx {
 };
 
 constexpr int kRedSlots = 16384;
+enum : unsigned {
+  ITG_LDS_EIGH = 1, ITG_LDS_ZUNM = 2, ITG_LDS_ZQR = 4, ITG_LDS_TRUNC = 8, ITG_LDS_SPLIT = 16
+};
 
 // contexts that exist on a device (core.hip)
 int itg_live_contexts(int device);
