@@ -3295,7 +3295,8 @@ int ortho_columns(itg_ctx* ctx, int rows, int n, double tol, double small2, Orth
       if (fresh > 6 * (int64_t)n) return ITG_OK;
       const size_t wo = (size_t)first * rows, vo = (size_t)first * n;
       rc = itg_gemm(ctx, ITG_F64, ITG_MODE_NATIVE, 'T', 'N', t, t, rows,
-                    std::ldexp(1.0, -std::ilogb(gf)), b.W + wo, rows, b.W + wo, rows, 0.0, b.G, t);
+                    std::ldexp(1.0, std::min(1023, -std::ilogb(gf))), b.W + wo, rows, b.W + wo, rows,
+                    0.0, b.G, t);
       if (rc) return rc;
       int64_t kg = 0;
       double teg = 0.0, dcg = 0.0;
