@@ -172,11 +172,8 @@ static void wpass(itg_ctx* ctx, int64_t chiL, int64_t chiR, int64_t Q, int64_t O
                                                                               T3);
     return;
   }
-  // outputs per launch: as many as X has room for in 64 KB of LDS (all of
-  // them but for an MPO of thousands of channels and d = 1)
   const int nt = wpass_nt(O);
-  int64_t os = O;
-  while (wpass_doubles((int)Q, (int)os, nt) * 8 > 65536) os = (os / 2 + 15) / 16 * 16;
+  const int64_t os = wpass_outputs((int)Q, (int)O, nt);
   const size_t lds = (size_t)wpass_doubles((int)Q, (int)os, nt) * sizeof(double);
   // two row tiles a wave once there are enough of them
   const int at = chiL >= 200 ? 2 : 1;
@@ -304,7 +301,7 @@ int check_heff(itg_ctx* ctx, int dtype, int mode, const HeffDims& h) {
   if (mode < 0 || mode > 2) return itg_fail(ctx, ITG_EARG, "unknown mode %d", mode);
   if (h.chiL <= 0 || h.chiR <= 0 || h.wl <= 0 || h.wm <= 0 || h.wr <= 0 || h.d <= 0)
     return itg_fail(ctx, ITG_EDIM, "heff2: non-positive dimension");
-  if (h.Q * 64 + h.Q * h.O > 8192)   // LDS budget of the W pass (64 KB)
+  if (!wpass_takes(h.Q, h.O))
     return itg_fail(ctx, ITG_EUNSUPPORTED, "heff2: MPO bond dimension too large for the W pass");
   return ITG_OK;
 }

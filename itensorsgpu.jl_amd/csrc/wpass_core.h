@@ -35,3 +35,18 @@ ITG_HD static inline int wpass_doubles(int Q, int O, int nt) {
 ITG_HD static inline int wpass_nt(int64_t O) {
   return O <= 16 ? 1 : O <= 32 ? 2 : 4;
 }
+
+constexpr int64_t WPASS_LDS = 65536;   // bytes of X per launch
+
+// operators the apply takes (w = 14, d = 2: 56 (64 + 56) = 6720); Q <= 126, so
+// that X has room for at least 16 outputs
+ITG_HD static inline bool wpass_takes(int64_t Q, int64_t O) { return Q * (64 + O) <= 8192; }
+
+// outputs per launch: as many as X has room for (all of them but for an MPO of
+// thousands of channels and d = 1)
+ITG_HD static inline int wpass_outputs(int Q, int O, int nt) {
+  int os = O;
+  while (os > 16 && wpass_doubles(Q, os, nt) * (int64_t)sizeof(double) > WPASS_LDS)
+    os = (os / 2 + 15) / 16 * 16;
+  return os;
+}

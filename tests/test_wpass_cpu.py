@@ -19,6 +19,7 @@ def wp(tmp_path_factory):
     L = C.CDLL(out)
     L.wpass_last_read.restype = L.wpass_size.restype = C.c_int64
     L.wpass_tiles.argtypes = [C.c_int64]
+    L.wpass_taken.argtypes = [C.c_int64, C.c_int64]
     return L
 
 
@@ -29,3 +30,18 @@ def test_reads_stay_inside(wp):
             if O <= top and wp.wpass_size(Q, O, 4) * 8 <= 65536:
                 nt = wp.wpass_tiles(O)
                 assert wp.wpass_last_read(Q, O, nt) < wp.wpass_size(Q, O, nt), (Q, O)
+
+
+def test_slices(wp):
+    """the operators taken are those with Q (64 + O) <= 8192, and each is cut
+    into launches whose X fits in 64 KB"""
+    for Q in list(range(1, 140)) + [512, 600, 8192]:
+        for O in sorted({1, 15, 16, 17, 33, 45, 80, 137, 340, 2000, 8128, 8192 // Q - 64, 8192 // Q - 63}):
+            if O < 1:
+                continue
+            assert wp.wpass_taken(Q, O) == (Q * 64 + Q * O <= 8192)
+            nt = wp.wpass_tiles(O)
+            os_ = wp.wpass_slice(Q, O, nt)          # returns for any Q
+            assert 1 <= os_ <= O
+            if wp.wpass_taken(Q, O):
+                assert wp.wpass_size(Q, os_, nt) * 8 <= 65536

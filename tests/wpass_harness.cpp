@@ -18,3 +18,5 @@ extern "C" int64_t wpass_last_read(int Q, int O, int nt) {
 
 extern "C" int64_t wpass_size(int Q, int O, int nt) { return wpass_doubles(Q, O, nt); }
 extern "C" int wpass_tiles(int64_t O) { return wpass_nt(O); }
+extern "C" int wpass_slice(int Q, int O, int nt) { return wpass_outputs(Q, O, nt); }
+extern "C" int wpass_taken(int64_t Q, int64_t O) { return wpass_takes(Q, O) ? 1 : 0; }
