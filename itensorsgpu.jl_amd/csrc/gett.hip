@@ -1319,16 +1319,6 @@ static bool band_wins(const itg_ctx* ctx, int mode, int64_t n) {
   return mode != ITG_MODE_NATIVE || band_tiles((n + 63) / 64) >= std::max(ctx->num_cu, 1);
 }
 
-// The library does not split K: a product with fewer 64 x 64 tiles than half
-// the CUs and a long K leaves most of the chip idle there, and the native
-// kernel's K split is faster. FP64, us, library against native: 1200 x 277 x
-// 3878: 123 / 70, 600 x 600 x 6000: 182 / 105, 300 x 300 x 10000: 274 to 1074 /
-// 72, 700 x 277 x 1500: 34 to 86 / 27; on the other side 512^3: 12 / 18,
-// 256 x 1280 x 512: 19 / 21, 2000 x 400 x 5000 (224 tiles): 157 / 179.
-static bool split_k_wins(const itg_ctx* ctx, int64_t m, int64_t n, int64_t k) {
-  return ((m + 63) / 64) * ((n + 63) / 64) * 2 < std::max(ctx->num_cu, 1) && k >= 1024;
-}
-
 // A contraction whose M, N and K modes each merge into one stride is a plain
 // product C(m, n) = alpha sum_k A(m, k) B(k, n) + beta C(m, n), elements at
 // m sAm + k sAk, k sBk + n sBn, m sCm + n sCn. It runs as a column-major
@@ -1355,12 +1345,14 @@ static int contract_on_lib(itg_ctx* ctx, const GettArgs& g) {
   int64_t la, lb, lc;
   if (!as_col(g.M, g.N, g.sCm, g.sCn, oc, lc)) return 1;
   if (oc == 'N') {
-    if (as_col(g.M, g.K, g.sAm, g.sAk, oa, la) && as_col(g.K, g.N, g.sBk, g.sBn, ob, lb))
+    if (as_col(g.M, g.K, g.sAm, g.sAk, oa, la) && as_col(g.K, g.N, g.sBk, g.sBn, ob, lb) &&
+        itg_libgemm_ok(ctx, ITG_F64, ITG_MODE_NATIVE, oa, ob, g.M, g.N, g.K))
       return itg_libgemm(ctx, oa, ob, g.M, g.N, g.K, g.alpha, (const double*)g.A, la,
                          (const double*)g.B, lb, g.beta, (double*)g.C, lc);
   } else {
     // C^T (n x m, column-major with ld lc) = B^T A^T
-    if (as_col(g.N, g.K, g.sBn, g.sBk, ob, lb) && as_col(g.K, g.M, g.sAk, g.sAm, oa, la))
+    if (as_col(g.N, g.K, g.sBn, g.sBk, ob, lb) && as_col(g.K, g.M, g.sAk, g.sAm, oa, la) &&
+        itg_libgemm_ok(ctx, ITG_F64, ITG_MODE_NATIVE, ob, oa, g.N, g.M, g.K))
       return itg_libgemm(ctx, ob, oa, g.N, g.M, g.K, g.alpha, (const double*)g.B, lb,
                          (const double*)g.A, la, g.beta, (double*)g.C, lc);
   }
@@ -1463,7 +1455,7 @@ extern "C" int itg_contract(itg_ctx* ctx, int dtype, int mode, int rA, const int
     const int rc = launch_gett(ctx, dtype, mode, g, p->akfast, p->bkfast);
     return rc ? rc : mirror_lower(ctx, dtype, g.M, C, g.sCm);
   }
-  if (plain && itg_libgemm_ok(ctx, dtype, mode, g.M, g.N, g.K) && !split_k_wins(ctx, g.M, g.N, g.K)) {
+  if (plain && dtype == ITG_F64 && mode == ITG_MODE_NATIVE) {
     int rc = contract_on_lib(ctx, g);
     if (rc != 1) return rc;
   }
@@ -1484,7 +1476,7 @@ int itg_gemm_internal(itg_ctx* ctx, int dtype, int mode, char ta, char tb, int64
   }
   bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
   if (!lower_band && lda >= (tA ? k : m) && ldb >= (tB ? n : k) && ldc >= m &&
-      itg_libgemm_ok(ctx, dtype, mode, m, n, k) && !split_k_wins(ctx, m, n, k))
+      itg_libgemm_ok(ctx, dtype, mode, ta, tb, m, n, k))
     return itg_libgemm(ctx, ta, tb, m, n, k, alpha, (const double*)A, lda, (const double*)B, ldb,
                        beta, (double*)C, ldc);
   GettArgs g;

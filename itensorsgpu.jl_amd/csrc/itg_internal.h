@@ -145,7 +145,8 @@ void itg_plan_cache_clear(itg_ctx* ctx);
 // whether a native FP64 product of this size may go there (not while the
 // stream is being captured, not inside a no-alloc call, dimensions in 32
 // bits); itg_libgemm is column-major C = alpha op(A) op(B) + beta C.
-bool itg_libgemm_ok(itg_ctx* ctx, int dtype, int mode, int64_t m, int64_t n, int64_t k);
+bool itg_libgemm_ok(itg_ctx* ctx, int dtype, int mode, char ta, char tb, int64_t m, int64_t n,
+                    int64_t k);
 int itg_libgemm(itg_ctx* ctx, char ta, char tb, int64_t m, int64_t n, int64_t k, double alpha,
                 const double* A, int64_t lda, const double* B, int64_t ldb, double beta,
                 double* C, int64_t ldc);
