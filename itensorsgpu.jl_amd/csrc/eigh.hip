@@ -1118,8 +1118,8 @@ __device__ void bitonic_sort(double* key, int* val, int np2) {
 }
 
 struct DcBufs {
-  double *ds, *zs, *dl, *wv, *dval, *rcs, *tau, *zh, *mrho;
-  int *cs, *gcol, *dcol, *rcol, *org, *meta;
+  double *zs, *dl, *wv, *dval, *rcs, *tau, *zh, *mrho;
+  int *gcol, *dcol, *rcol, *org, *meta;
 };
 
 constexpr int DC_ZLDS = 4096;   // largest merge whose z is staged in LDS
@@ -2219,7 +2219,7 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   const size_t Tw = (size_t)(n + 63) / 64;   // tile rows of the tiled symv
   size_t bytes = (3 * nn + (f32 ? 2 * nn : 0)) * sizeof(double) + 3 * (size_t)n * NB * 8 +
                  (2 * (size_t)BT_GROUP * n + (size_t)BT_GROUP * BT_GROUP) * 8 +
-                 (size_t)n * 8 * 26 + 4 * (size_t)n * NB * 8 + 4 * NB * NB * 8 + 64 * 1024 +
+                 (size_t)n * 8 * 25 + 4 * (size_t)n * NB * 8 + 64 * 1024 +
                  (Tw * n + Tw * (Tw + 1) / 2 + 64) * 8 + 64 * 256 +
                  ((size_t)n / POST_ROWS + 1) * 8 +
                  (two ? eig2::doubles_needed(n) * 8 + 256 : 0) +
@@ -2250,15 +2250,13 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   double* Da = cv.take<double>(n);
   double* Db = cv.take<double>(n);
   DcBufs b;
-  b.ds = cv.take<double>(n); b.zs = cv.take<double>(n); b.dl = cv.take<double>(n);
+  b.zs = cv.take<double>(n); b.dl = cv.take<double>(n);
   b.wv = cv.take<double>(n); b.dval = cv.take<double>(n); b.rcs = cv.take<double>(2 * (size_t)n);
   b.tau = cv.take<double>(n); b.zh = cv.take<double>(n); b.mrho = cv.take<double>(2 * (size_t)n);
-  b.cs = cv.take<int>(n); b.gcol = cv.take<int>(n); b.dcol = cv.take<int>(n);
+  b.gcol = cv.take<int>(n); b.dcol = cv.take<int>(n);
   b.rcol = cv.take<int>(2 * (size_t)n); b.org = cv.take<int>(n); b.meta = cv.take<int>(3 * (size_t)n);
   int* perm = cv.take<int>(n);
   int64_t* tab = cv.take<int64_t>(n);
-  double* Gm = cv.take<double>(NB * NB);
-  double* Tm = cv.take<double>(NB * NB);
   double* Ygrp = cv.take<double>((size_t)BT_GROUP * n);
   double* X2grp = cv.take<double>((size_t)BT_GROUP * n);
   double* Ggrp = cv.take<double>((size_t)BT_GROUP * BT_GROUP);
@@ -3136,7 +3134,6 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   if (m64 == 0 || n64 == 0) return ITG_OK;
   if (dtype == ITG_C64) return itg_c64_qr(ctx, m64, n64, Ain, Qo, Ro);
   int m = (int)m64, n = (int)n64, r = std::min(m, n);
-  bool f32 = dtype == ITG_F32;
   const size_t nx = std::max((size_t)NB * n, (size_t)BT_GROUP * r);
   size_t bytes = ((size_t)m * n + (size_t)m * r + (size_t)r * n + (size_t)m * NB + 2 * nx +
                   (size_t)BT_GROUP * BT_GROUP + NB * NB + (size_t)r +
@@ -3202,7 +3199,6 @@ extern "C" int itg_qr(itg_ctx* ctx, int dtype, int64_t m64, int64_t n64, const v
   rc = itg_convert(ctx, (int64_t)m * r, ITG_F64, Q, dtype, Qo);
   if (rc) return rc;
   return itg_convert(ctx, (int64_t)r * n, ITG_F64, R, dtype, Ro);
-  (void)f32;
 }
 
 // Buffers of ortho_columns: W and V with a second buffer each (swapped as

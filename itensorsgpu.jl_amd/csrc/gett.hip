@@ -1177,8 +1177,8 @@ static void native_kernel(itg_ctx* ctx, const GettArgs& g, dim3 grid, bool ak, b
 // FP64 at 128 x 128 gains nothing over 64 x 64 (59 against 61 TFLOP/s at
 // 4096^3: 64 cycles per product hide the smaller tile's reads) and rounds
 // worse, so it is not built. The estimates are within 15% of the measured
-// times over 18 shapes, 80 x 20 x 100 to 4096^3, and pick the fastest tile
-// and split or one within 10% of it.
+// times over 26 shapes, 80 x 20 x 100 to 4096 x 4096 x 1024, and on nearly all of
+// them pick the fastest tile and split or one within 10% of it.
 struct NativeChoice {
   int ts, nsplit;
 };
@@ -1315,6 +1315,9 @@ static int mirror_lower(itg_ctx* ctx, int dtype, int64_t n, void* C, int64_t ldc
 // than the whole product, which can split K. FP64, us, band against whole:
 // 1024 x 1024: 58 / 59, 512 x 2048: 103 / 39, 256 x 256: 20 / 12; on the other
 // side 1500 x 1500: 121 / 150, 2048 x 2048: 220 / 255, 4096 x 4096: 1240 / 1820.
+// FP32: 640 x 2048: 66 / 38, 1024 x 512: 24 / 24, 1024 x 2048: 67 / 60; on the other
+// side 1400 x 512: 32 / 32, 1500 x 2048: 92 / 120, 4096 x 4096: 769 / 1161 (1200 x
+// 512, just below the line, 25 / 31).
 static bool band_wins(const itg_ctx* ctx, int mode, int64_t n) {
   return mode != ITG_MODE_NATIVE || band_tiles((n + 63) / 64) >= std::max(ctx->num_cu, 1);
 }

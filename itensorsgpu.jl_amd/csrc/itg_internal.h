@@ -133,8 +133,8 @@ static inline unsigned itg_blocks(int64_t n, int threads, int64_t cap = 65535 * 
 }
 
 // Internal (non-exported) entry points used across translation units.
-// lower_band: compute only the 128 x 128 output tiles on or below the
-// diagonal and the first tile band above it (square C whose upper part far
+// lower_band: compute only the output tiles (64 or 128 rows and columns) on or
+// below the diagonal and the first tile band above it (square C whose upper part far
 // from the diagonal is never read)
 int itg_gemm_internal(itg_ctx* ctx, int dtype, int mode, char ta, char tb,
                       int64_t m, int64_t n, int64_t k, double alpha,
