@@ -2212,7 +2212,7 @@ extern "C" int itg_eigh_trunc(itg_ctx* ctx, int dtype, int64_t n64, void* Ain, d
   bool f32 = dtype == ITG_F32;
   // the two-stage reduction (dense -> band -> tridiagonal) on request
   // (ITG_EIGH_TWOSTAGE=1, read per call): correct, but at n = 4096 it takes
-  // 113 ms against the one-stage reduction's 77 ms, its bulge chasing and
+  // 113 ms against 36 with the one-stage reduction, its bulge chasing and
   // tall-panel QRs being latency-bound
   const char* two_env = getenv("ITG_EIGH_TWOSTAGE");
   const bool two = !cplx && n >= TWO_STAGE_MIN && two_env && two_env[0] == '1';
