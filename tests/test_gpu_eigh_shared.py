@@ -157,5 +157,6 @@ def test_other_contexts_queue():
 
     if not _in_thread(both):
         pytest.skip("no two streams on hardware queues of their own")
-    # the other one took milliseconds of the two seconds
-    assert times["other"] < times["busy"] - 1.0
+    # the other one took milliseconds of the queued two seconds (less if the
+    # clock rose since they were counted out)
+    assert times["other"] < times["busy"] - 0.25
