@@ -2370,7 +2370,10 @@ namespace {
 // Beside a pivot of QR_TINY_PIVOT or more the tail is less than 2^-60 of the
 // column and counts as zero; else the reflector is formed from QR_UP times the
 // tail (or QR_UP^2 times, if that is still as small), so that a matrix of any
-// scale satisfies A = QR relative to itself.
+// scale satisfies A = QR relative to itself. In the panel kernels that is the
+// column's step taken again, which costs other matrices nothing to 1.5% (us,
+// without and with: 2000 x 1000 3148 / 3150, 600 x 500 1205 / 1218, 3600 x 1500
+// 8670 / 8795, 5000 x 600 6025 / 5848); as code of its own it cost 4.5%.
 constexpr double QR_TINY2 = 0x1p-600, QR_TINY_PIVOT = 0x1p-240, QR_UP = 0x1p500;
 
 __global__ __launch_bounds__(1024) void qr_reflect_kernel(double* __restrict__ W, int m, int j,
